@@ -219,7 +219,8 @@ __global__ __launch_bounds__(256) void uvw_antisym_kernel(N3Source p, unsigned c
   if (threadIdx.x == 0) out[s] = bad ? 0 : 1;
 }
 
-// min / max of u over the points of item k (a sample, or a listed range of slots).
+// min / max of u over the points of item k (a sample, or a listed range of slots), the item's
+// slots split over gridDim.y workgroups; workgroup (k, y) writes out[6 (k gridDim.y + y)].
 __global__ __launch_bounds__(256) void slot_range_kernel(N3Source p,
                                                          const unsigned long long* list,
                                                          const unsigned* begin,
@@ -229,7 +230,8 @@ __global__ __launch_bounds__(256) void slot_range_kernel(N3Source p,
   const long long sps = p.slots_per_sample();
   const long long n = list ? static_cast<long long>(count[k]) : sps;
   double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
-  for (long long i = threadIdx.x; i < n; i += blockDim.x) {
+  const long long step = (long long)blockDim.x * gridDim.y;
+  for (long long i = blockIdx.y * (long long)blockDim.x + threadIdx.x; i < n; i += step) {
     const unsigned long long slot =
         list ? list[static_cast<long long>(begin[k]) + i] : (unsigned long long)k * sps + i;
     const int s = static_cast<int>(slot / sps);
@@ -257,41 +259,107 @@ __global__ __launch_bounds__(256) void slot_range_kernel(N3Source p,
     __syncthreads();
   }
   if (threadIdx.x < 3) {
-    out[6 * (size_t)k + threadIdx.x] = red[0][threadIdx.x][0];
-    out[6 * (size_t)k + 3 + threadIdx.x] = red[1][threadIdx.x][0];
+    double* o = out + 6 * ((size_t)k * gridDim.y + blockIdx.y);
+    o[threadIdx.x] = red[0][threadIdx.x][0];
+    o[3 + threadIdx.x] = red[1][threadIdx.x][0];
   }
 }
 
+// The partial ranges of an item (`parts` of them, parts <= 64) into one; a wavefront per item.
+__global__ __launch_bounds__(64) void slot_range_reduce_kernel(const double* part, int parts,
+                                                               double* out) {
+  const int k = blockIdx.x;
+  const double* q = part + 6 * ((size_t)k * parts + threadIdx.x);
+#pragma unroll
+  for (int d = 0; d < 6; ++d) {
+    double v = static_cast<int>(threadIdx.x) < parts ? q[d] : (d < 3 ? 1e300 : -1e300);
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) {
+      const double o = __shfl_xor(v, m, 64);
+      v = d < 3 ? fmin(v, o) : fmax(v, o);
+    }
+    if (threadIdx.x == 0) out[6 * (size_t)k + d] = v;
+  }
+}
+
+// Slots per workgroup of the box assignment and of the counting sort by box, and the number
+// of boxes up to which a workgroup counts in LDS and adds its totals with one atomic per box.
+// A few boxes hold all points, so one atomic per point serialises on their counters: 11.0 ms
+// for 1.6 million slots in two boxes, each of the two kernels, against 0.03 ms.  Above the bound
+// the points spread over so many counters that the totals would save nothing (at least 8
+// slots per box and workgroup below it).
+constexpr int PART_PER = 16;
+constexpr int PART_LDS_GROUPS = 512;
+
 // Box of every slot's point (-1 without a point) and the point count of every box.
-__global__ void n3_partition_kernel(N3PartParams p) {
+__global__ __launch_bounds__(256) void n3_partition_kernel(N3PartParams p, int n_groups) {
+  __shared__ unsigned cnt[PART_LDS_GROUPS];
+  const bool lds = n_groups <= PART_LDS_GROUPS;
+  if (lds) {
+    for (int g = threadIdx.x; g < n_groups; g += 256) cnt[g] = 0;
+    __syncthreads();
+  }
   const long long sps = p.src.slots_per_sample();
-  const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (i >= sps * p.n_samples) return;
-  const int s = static_cast<int>(i / sps);
-  SlotPoint sp;
-  if (!slot_point(p.src, s, i - (long long)s * sps, sp)) {
-    p.group_of[i] = -1;
-    return;
+  const long long n_slots = sps * p.n_samples;
+  const long long i0 = blockIdx.x * (256LL * PART_PER) + threadIdx.x;
+  for (int r = 0; r < PART_PER; ++r) {
+    const long long i = i0 + 256LL * r;
+    if (i >= n_slots) break;
+    const int s = static_cast<int>(i / sps);
+    SlotPoint sp;
+    if (!slot_point(p.src, s, i - (long long)s * sps, sp)) {
+      p.group_of[i] = -1;
+      continue;
+    }
+    int g = 0;
+    for (int d = 2; d >= 0; --d) {
+      const double x = p.inv[d] * (sp.u[d] - p.lo[d]);
+      const int k = x > 0.0 ? static_cast<int>(fmin(x, static_cast<double>(p.dims[d] - 1))) : 0;
+      g = g * p.dims[d] + k;
+    }
+    p.group_of[i] = g;
+    atomicAdd(lds ? &cnt[g] : &p.group_count[g], 1u);
   }
-  int g = 0;
-  for (int d = 2; d >= 0; --d) {
-    const double x = p.inv[d] * (sp.u[d] - p.lo[d]);
-    const int k = x > 0.0 ? static_cast<int>(fmin(x, static_cast<double>(p.dims[d] - 1))) : 0;
-    g = g * p.dims[d] + k;
-  }
-  p.group_of[i] = g;
-  atomicAdd(&p.group_count[g], 1u);
+  if (!lds) return;
+  __syncthreads();
+  for (int g = threadIdx.x; g < n_groups; g += 256)
+    if (cnt[g]) atomicAdd(&p.group_count[g], cnt[g]);
 }
 
 // slot ids in box order (counting sort)
-__global__ void n3_group_scatter_kernel(long long n_slots, const int* group_of,
-                                        const unsigned* group_start, unsigned* group_fill,
-                                        unsigned long long* list) {
-  const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (i >= n_slots) return;
-  const int g = group_of[i];
-  if (g < 0) return;
-  list[group_start[g] + atomicAdd(&group_fill[g], 1u)] = static_cast<unsigned long long>(i);
+__global__ __launch_bounds__(256) void n3_group_scatter_kernel(long long n_slots, int n_groups,
+                                                               const int* group_of,
+                                                               const unsigned* group_start,
+                                                               unsigned* group_fill,
+                                                               unsigned long long* list) {
+  __shared__ unsigned cnt[PART_LDS_GROUPS], base[PART_LDS_GROUPS];
+  const long long i0 = blockIdx.x * (256LL * PART_PER) + threadIdx.x;
+  if (n_groups > PART_LDS_GROUPS) {
+    for (int r = 0; r < PART_PER; ++r) {
+      const long long i = i0 + 256LL * r;
+      if (i >= n_slots) break;
+      const int g = group_of[i];
+      if (g >= 0) list[group_start[g] + atomicAdd(&group_fill[g], 1u)] = static_cast<unsigned long long>(i);
+    }
+    return;
+  }
+  for (int g = threadIdx.x; g < n_groups; g += 256) cnt[g] = 0;
+  __syncthreads();
+  int gr[PART_PER];
+  unsigned rank[PART_PER];
+#pragma unroll
+  for (int r = 0; r < PART_PER; ++r) {
+    const long long i = i0 + 256LL * r;
+    gr[r] = i < n_slots ? group_of[i] : -1;
+    rank[r] = gr[r] >= 0 ? atomicAdd(&cnt[gr[r]], 1u) : 0u;
+  }
+  __syncthreads();
+  for (int g = threadIdx.x; g < n_groups; g += 256)
+    base[g] = cnt[g] ? group_start[g] + atomicAdd(&group_fill[g], cnt[g]) : 0u;
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < PART_PER; ++r)
+    if (gr[r] >= 0) list[base[gr[r]] + rank[r]] = static_cast<unsigned long long>(i0 + 256LL * r);
 }
 
 // exclusive scan helpers (counts -> starts)
@@ -1463,25 +1531,43 @@ void launch_uvw_antisym(const N3Source& src, int n_samples, unsigned char* out, 
   check_launch("uvw_antisym_kernel");
 }
 
+// Workgroups per item: about 2048 workgroups over all items (8 per CU), at least 1024 slots
+// each, at most the 64 partial ranges that one wavefront reduces.
+int slot_range_parts(int n_items, long long n_slots) {
+  if (n_items <= 0) return 1;
+  const long long by_grid = (2048 + n_items - 1) / n_items, by_work = n_slots / n_items / 1024;
+  return static_cast<int>(std::max<long long>(1, std::min<long long>(64, std::min(by_grid, by_work))));
+}
+
 void launch_slot_range(const N3Source& src, int n_items, const unsigned long long* list,
-                       const unsigned* begin, const unsigned* count, double* out, hipStream_t st) {
+                       const unsigned* begin, const unsigned* count, int parts, double* part,
+                       double* out, hipStream_t st) {
   if (n_items <= 0) return;
-  slot_range_kernel<<<n_items, 256, 0, st>>>(src, list, begin, count, out);
+  if (parts < 1 || parts > 64) fail(BIPP_INTERNAL_ERROR, "slot range parts");
+  slot_range_kernel<<<dim3(n_items, parts), 256, 0, st>>>(src, list, begin, count,
+                                                          parts > 1 ? part : out);
   check_launch("slot_range_kernel");
+  if (parts == 1) return;
+  slot_range_reduce_kernel<<<n_items, 64, 0, st>>>(part, parts, out);
+  check_launch("slot_range_reduce_kernel");
 }
 
 void launch_n3_partition(const N3PartParams& p, hipStream_t st) {
   const long long n = p.src.slots_per_sample() * p.n_samples;
   if (n <= 0) return;
-  n3_partition_kernel<<<static_cast<unsigned>((n + 255) / 256), 256, 0, st>>>(p);
+  const long long per = 256LL * PART_PER;
+  n3_partition_kernel<<<static_cast<unsigned>((n + per - 1) / per), 256, 0, st>>>(
+      p, p.dims[0] * p.dims[1] * p.dims[2]);
   check_launch("n3_partition_kernel");
 }
 
-void launch_n3_group_scatter(long long n_slots, const int* group_of, const unsigned* group_start,
-                             unsigned* group_fill, unsigned long long* list, hipStream_t st) {
+void launch_n3_group_scatter(long long n_slots, int n_groups, const int* group_of,
+                             const unsigned* group_start, unsigned* group_fill,
+                             unsigned long long* list, hipStream_t st) {
   if (n_slots <= 0) return;
-  n3_group_scatter_kernel<<<static_cast<unsigned>((n_slots + 255) / 256), 256, 0, st>>>(
-      n_slots, group_of, group_start, group_fill, list);
+  const long long per = 256LL * PART_PER;
+  n3_group_scatter_kernel<<<static_cast<unsigned>((n_slots + per - 1) / per), 256, 0, st>>>(
+      n_slots, n_groups, group_of, group_start, group_fill, list);
   check_launch("n3_group_scatter_kernel");
 }
 

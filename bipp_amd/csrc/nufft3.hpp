@@ -219,12 +219,17 @@ void launch_pos_range(int n_samples, const double* pos, long long pos_stride, in
 // 1 per sample whose nAnt^2 x 3 uvw is antisymmetric with a zero diagonal, else 0
 void launch_uvw_antisym(const N3Source& src, int n_samples, unsigned char* out, hipStream_t st);
 // min and max of u over the points of each item: item k covers the slots
-// list[begin[k] .. begin[k] + count[k]) (list == nullptr: slots of sample k); out [k][6]
+// list[begin[k] .. begin[k] + count[k]) (list == nullptr: slots of sample k); out [k][6].  Each
+// item is split over `parts` workgroups (slot_range_parts of the n_slots slots of all items);
+// part: scratch of 6 * parts doubles per item
+int slot_range_parts(int n_items, long long n_slots);
 void launch_slot_range(const N3Source& src, int n_items, const unsigned long long* list,
-                       const unsigned* begin, const unsigned* count, double* out, hipStream_t st);
+                       const unsigned* begin, const unsigned* count, int parts, double* part,
+                       double* out, hipStream_t st);
 void launch_n3_partition(const N3PartParams& p, hipStream_t st);
-void launch_n3_group_scatter(long long n_slots, const int* group_of, const unsigned* group_start,
-                             unsigned* group_fill, unsigned long long* list, hipStream_t st);
+void launch_n3_group_scatter(long long n_slots, int n_groups, const int* group_of,
+                             const unsigned* group_start, unsigned* group_fill,
+                             unsigned long long* list, hipStream_t st);
 template <typename R>
 void launch_zero(R* p, long long n, hipStream_t st);
 void launch_n3_points(const N3PointsParams& p, int n_samples, hipStream_t st);

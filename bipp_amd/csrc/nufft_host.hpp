@@ -635,8 +635,9 @@ struct N3Runner {
     if (n_slots > 0x7fffffffLL)
       fail(BIPP_INVALID_PARAMETER_ERROR, "too many NUFFT points in one batch (reduce the sample batch size)");
     // extent of every sample's points
-    double* rg = ranges.as<double>(6 * (size_t)nS);
-    launch_slot_range(src, nS, nullptr, nullptr, nullptr, rg, st);
+    const int rparts = slot_range_parts(nS, n_slots);
+    double* rg = ranges.as<double>(6 * (size_t)nS * (1 + rparts));
+    launch_slot_range(src, nS, nullptr, nullptr, nullptr, rparts, rg + 6 * (size_t)nS, rg, st);
     double* h = host_buf(6 * (size_t)nS);
     BIPP_HIP(hipMemcpyAsync(h, rg, sizeof(double) * 6 * nS, hipMemcpyDeviceToHost, st));
     c.sync();
@@ -705,10 +706,12 @@ struct N3Runner {
     unsigned* gfill = group_fill.as<unsigned>(n_groups);
     launch_zero<unsigned>(gfill, n_groups, st);
     unsigned long long* list = slot_list.as<unsigned long long>(n_slots);
-    launch_n3_group_scatter(n_slots, pp.group_of, gstart, gfill, list, st);
+    launch_n3_group_scatter(n_slots, (int)n_groups, pp.group_of, gstart, gfill, list, st);
     // extent of every box's points
-    double* grg = ranges.as<double>(6 * (size_t)n_groups);
-    launch_slot_range(src, (int)n_groups, list, gstart, pp.group_count, grg, st);
+    const int gparts = slot_range_parts((int)n_groups, n_slots);
+    double* grg = ranges.as<double>(6 * (size_t)n_groups * (1 + gparts));
+    launch_slot_range(src, (int)n_groups, list, gstart, pp.group_count, gparts,
+                      grg + 6 * (size_t)n_groups, grg, st);
     double* hb = host_buf(8 * (size_t)n_groups);
     BIPP_HIP(hipMemcpyAsync(hb, grg, sizeof(double) * 6 * n_groups, hipMemcpyDeviceToHost, st));
     // counts and starts as unsigned pairs after the ranges
