@@ -20,11 +20,11 @@
 //   FP32:   everything float32 (phase included) on v_mfma_f32_16x16x4_f32.
 //   FP64:   everything float64 on v_mfma_f64_16x16x4_f64 (the GPU oracle form).
 //
-// Workgroup = 8 waves (4 for FP64) over a tile of 128 (64) pixels; each wave owns 4 row
+// Workgroup = 8 waves (4 for FP64) over a tile of 128 (64) pixels; each wave owns up to 4 row
 // tiles (64 rows) and all pixel columns; the workgroup loops over every sample of the
 // batch, so each pixel tile is written once per launch (no atomics in HBM).  The E tile of
 // a 16-antenna chunk is generated once per workgroup into LDS (double-buffered) in the
-// exact MFMA B-operand layout.
+// exact MFMA B-operand layout.  BF16X3 has a kernel of its own (steer_bf16x3_kernel).
 #include "common.hpp"
 
 #include <algorithm>
@@ -251,12 +251,6 @@ __global__ void level_weights_kernel(int n_levels, int filter, const double* int
 template <int MODE>
 struct SteerCfg;
 template <>
-struct SteerCfg<STEER_BF16X3> {
-  static constexpr int NT = 512, TP = 128;
-  using Acc = f32x4;
-  using Img = float;
-};
-template <>
 struct SteerCfg<STEER_FP32> {
   static constexpr int NT = 512, TP = 128;
   using Acc = f32x4;
@@ -271,10 +265,6 @@ struct SteerCfg<STEER_FP64> {
 
 template <int MODE>
 struct SteerSmem;
-template <>
-struct SteerSmem<STEER_BF16X3> {
-  uint4 eb[2][SteerCfg<STEER_BF16X3>::TP / 16][2][64];
-};
 template <>
 struct SteerSmem<STEER_FP32> {
   float eb[2][32][SteerCfg<STEER_FP32>::TP + 16];
@@ -324,38 +314,13 @@ __global__ __launch_bounds__(SteerCfg<MODE>::NT) void steer_kernel(SteerParams p
         const double t = fma(px, lx, fma(py, ly, pz * lz));
         const double f = t - rint(t);
         sincospi(2.0 * f, &sn64[j], &cs64[j]);
-      } else if (p.phase_fp32) {
+      } else {
         const float t = fmaf(static_cast<float>(px), lxf,
                              fmaf(static_cast<float>(py), lyf, static_cast<float>(pz) * lzf));
         sincospif(2.0f * t, &sn[j], &cs[j]);
-      } else {
-        const double t = fma(px, lx, fma(py, ly, pz * lz));
-        const float f = static_cast<float>(t - rint(t));
-        sincospif(2.0f * f, &sn[j], &cs[j]);
       }
     }
-    if constexpr (MODE == STEER_BF16X3) {
-      unsigned short hi[8], lo[8];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        hi[2 * j] = bf16_bits(cs[j]);
-        hi[2 * j + 1] = bf16_bits(sn[j]);
-        lo[2 * j] = bf16_bits(cs[j] - bf16_to_f32(hi[2 * j]));
-        lo[2 * j + 1] = bf16_bits(sn[j] - bf16_to_f32(hi[2 * j + 1]));
-      }
-      uint4 h, l;
-      h.x = hi[0] | ((unsigned)hi[1] << 16);
-      h.y = hi[2] | ((unsigned)hi[3] << 16);
-      h.z = hi[4] | ((unsigned)hi[5] << 16);
-      h.w = hi[6] | ((unsigned)hi[7] << 16);
-      l.x = lo[0] | ((unsigned)lo[1] << 16);
-      l.y = lo[2] | ((unsigned)lo[3] << 16);
-      l.z = lo[4] | ((unsigned)lo[5] << 16);
-      l.w = lo[6] | ((unsigned)lo[7] << 16);
-      const int ct = gpx >> 4, fl = (gpx & 15) + 16 * gquad;
-      sm.eb[buf][ct][0][fl] = h;
-      sm.eb[buf][ct][1][fl] = l;
-    } else if constexpr (MODE == STEER_FP32) {
+    if constexpr (MODE == STEER_FP32) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         sm.eb[buf][2 * (gquad * 4 + j)][gpx] = cs[j];
@@ -395,57 +360,29 @@ __global__ __launch_bounds__(SteerCfg<MODE>::NT) void steer_kernel(SteerParams p
         const int buf = kc & 1;
         if (kc + 1 < nkc) gen(pos, p.apad, kc + 1, buf ^ 1);
         if (nmy > 0) {
-          if constexpr (MODE == STEER_BF16X3) {
-            const unsigned short* fr = static_cast<const unsigned short*>(p.afrag) + fbase;
-            bf16x8 ahi[RTW], alo[RTW];
+          using T = typename std::conditional<MODE == STEER_FP64, double, float>::type;
+          const T* fr = static_cast<const T*>(p.afrag) + fbase;
+          T af[RTW][8];
 #pragma unroll
-            for (int r = 0; r < RTW; ++r) {
-              if (r < nmy) {
-                const long long off = ((long long)(my_rt0 + r) * p.kchunks + kc) * 1024;
-                ahi[r] = *reinterpret_cast<const bf16x8*>(fr + off + lane * 8);
-                alo[r] = *reinterpret_cast<const bf16x8*>(fr + off + 512 + lane * 8);
-              }
+          for (int r = 0; r < RTW; ++r) {
+            if (r < nmy) {
+              const long long off = ((long long)(my_rt0 + r) * p.kchunks + kc) * 512 + lane * 8;
+#pragma unroll
+              for (int j = 0; j < 8; ++j) af[r][j] = fr[off + j];
             }
+          }
 #pragma unroll
-            for (int c = 0; c < CT; ++c) {
-              const uint4 bh = sm.eb[buf][c][0][lane];
-              const uint4 bl = sm.eb[buf][c][1][lane];
-              const bf16x8 bhi = __builtin_bit_cast(bf16x8, bh);
-              const bf16x8 blo = __builtin_bit_cast(bf16x8, bl);
+          for (int c = 0; c < CT; ++c) {
+#pragma unroll
+            for (int kk = 0; kk < 8; ++kk) {
+              const T b = sm.eb[buf][4 * kk + (lane >> 4)][c * 16 + (lane & 15)];
 #pragma unroll
               for (int r = 0; r < RTW; ++r) {
                 if (r < nmy) {
-                  acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(alo[r], bhi, acc[r][c], 0, 0, 0);
-                  acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ahi[r], blo, acc[r][c], 0, 0, 0);
-                  acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ahi[r], bhi, acc[r][c], 0, 0, 0);
-                }
-              }
-            }
-          } else {
-            using T = typename std::conditional<MODE == STEER_FP64, double, float>::type;
-            const T* fr = static_cast<const T*>(p.afrag) + fbase;
-            T af[RTW][8];
-#pragma unroll
-            for (int r = 0; r < RTW; ++r) {
-              if (r < nmy) {
-                const long long off = ((long long)(my_rt0 + r) * p.kchunks + kc) * 512 + lane * 8;
-#pragma unroll
-                for (int j = 0; j < 8; ++j) af[r][j] = fr[off + j];
-              }
-            }
-#pragma unroll
-            for (int c = 0; c < CT; ++c) {
-#pragma unroll
-              for (int kk = 0; kk < 8; ++kk) {
-                const T b = sm.eb[buf][4 * kk + (lane >> 4)][c * 16 + (lane & 15)];
-#pragma unroll
-                for (int r = 0; r < RTW; ++r) {
-                  if (r < nmy) {
-                    if constexpr (MODE == STEER_FP64)
-                      acc[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[r][kk], b, acc[r][c], 0, 0, 0);
-                    else
-                      acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[r][kk], b, acc[r][c], 0, 0, 0);
-                  }
+                  if constexpr (MODE == STEER_FP64)
+                    acc[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[r][kk], b, acc[r][c], 0, 0, 0);
+                  else
+                    acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[r][kk], b, acc[r][c], 0, 0, 0);
                 }
               }
             }
@@ -501,6 +438,298 @@ __global__ __launch_bounds__(SteerCfg<MODE>::NT) void steer_kernel(SteerParams p
   }
 }
 
+// --------------------------------------------------------------------------------------
+// BF16X3 contraction
+// --------------------------------------------------------------------------------------
+// cos and sin of f turns, f in [-1/2, 1/2]: reduced to a quarter turn (exactly: 4 f and its
+// distance g to the nearest integer are representable), then minimax polynomials in g^2 of
+// sin(pi/2 g) / g (error 4.8e-9) and cos(pi/2 g) (error 4.7e-11), both below float rounding,
+// fitted by exchange on [0, 1/4].
+__device__ __forceinline__ void cossin_turn(float f, float& c, float& s) {
+  const float u = 4.0f * f;
+  const float q = rintf(u);
+  const float g = u - q;
+  const float y = g * g;
+  float ps = fmaf(y, -0.00460217700f, 0.0796802281f);
+  ps = fmaf(y, ps, -0.645963479f);
+  ps = fmaf(y, ps, 1.57079632f);
+  float pc = fmaf(y, 0.000903631703f, -0.0208600713f);
+  pc = fmaf(y, pc, 0.253669204f);
+  pc = fmaf(y, pc, -1.23370054f);
+  pc = fmaf(y, pc, 1.0f);
+  ps *= g;
+  const unsigned qi = static_cast<unsigned>(static_cast<int>(q));
+  const bool odd = qi & 1u;
+  const float a = odd ? ps : pc, b = odd ? pc : ps;
+  c = __uint_as_float(__float_as_uint(a) ^ (((qi + 1u) & 2u) << 30));
+  s = __uint_as_float(__float_as_uint(b) ^ ((qi & 2u) << 30));
+}
+
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ unsigned pack_bf16(float a, float b) {
+  return __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{a, b}), bf16x2));
+}
+
+// Sums over the four 16-lane rows of a wavefront, four columns at once: lane row j gets the
+// total of v[0], v[2], v[1], v[3] (j = 0..3) at its lane of the row.  permlane32_swap leaves
+// the lower halves of both operands in the first result and the upper halves in the second,
+// permlane16_swap does the same with each pair of rows.
+__device__ __forceinline__ float sum_columns(const float* v) {
+  const auto add32 = [](float a, float b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  };
+  const float x = add32(v[0], v[1]), y = add32(v[2], v[3]);
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// Kernel and pixel tile as steer_kernel's, for the split-bf16 operands.
+//
+// Bound: the matrix cores (three products of 8 N K flops per pixel and sample) and, beside
+// them, the generation of E on the vector ALU (one cos/sin pair per antenna and pixel, about
+// 40 instructions with its phase and split).  The two run on separate pipes, so the two
+// wavefronts of a SIMD (w and w + 4) take the halves of a step in opposite order: one
+// generates the next chunk while the other multiplies the current one, with one barrier per
+// step.  Steps run through all (sample, row pass, chunk) triples without a break, so the
+// first chunk of a sample is generated during the last one of the sample before it.  Row
+// tiles are dealt evenly (a wavefront's count differs by at most one, the larger counts on
+// different SIMDs); RTW, the largest count, is a template argument, so up to 128 eigenvectors
+// (RTW <= 2) two workgroups fit a CU.  The fragments of a step are loaded one step ahead.  Every
+// wavefront adds its sums into an image of its own in LDS: LDS float atomics took 2.4 cycles
+// per lane (2.5 ms of 31 ms at 96 samples, 512^2 pixels).
+// Measured, 512^2 pixels, 4 levels: 96 samples of 180..256 antennas 41.4 to 28.2 ms (a
+// full-rate loop of these MFMAs alone runs at 1.5 PFLOP/s here, about 19 ms); 256^2 pixels,
+// 32 samples of 96 antennas 1.47 to 0.56 ms.
+// (the accumulators live in registers only if every lambda is inlined)
+#define SB_INLINE __attribute__((always_inline))
+constexpr int SB_NT = 512, SB_TP = 128, SB_CT = SB_TP / 16, SB_NW = SB_NT / 64;
+
+template <int RTW>
+__global__ __launch_bounds__(SB_NT, RTW <= 2 ? 4 : 2) void steer_bf16x3_kernel(SteerParams p) {
+  constexpr int TP = SB_TP, CT = SB_CT, NWV = SB_NW, RT_PASS = NWV * RTW;
+  __shared__ uint4 eb[2][CT][2][64];  // [buffer][column tile][hi, lo][lane]
+  __shared__ float img_acc[NWV][LMAX][TP];  // every wavefront's sums (sum_columns order)
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int q0 = blockIdx.x * TP;
+  const int L = p.n_levels;
+
+  // generator role: one pixel and one quad of antennas of each 16-antenna chunk
+  const int gpx = tid % TP, gquad = wave >> 1;
+  const int gq = q0 + gpx;
+  double lx = 0, ly = 0, lz = 0;
+  if (gq < p.n_pix) {
+    lx = p.lmn[gq];
+    ly = p.lmn[p.n_pix + gq];
+    lz = p.lmn[2 * (size_t)p.n_pix + gq];
+  }
+  for (int i = lane; i < LMAX * TP; i += 64) (&img_acc[wave][0][0])[i] = 0;
+
+  typedef const double __attribute__((address_space(4))) cdouble;  // read by scalar loads
+  auto gen = [&](int s, int kc, int buf) SB_INLINE {
+    cdouble* pos = (cdouble*)(p.pos + (size_t)s * p.pos_stride + kc * 16 + gquad * 4);
+    uint4 h, l;
+    unsigned* hp = &h.x;
+    unsigned* lp = &l.x;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const double t = fma(pos[j], lx, fma(pos[p.apad + j], ly, pos[2 * p.apad + j] * lz));
+      float c, sn;
+      cossin_turn(static_cast<float>(t - rint(t)), c, sn);
+      const unsigned hi = pack_bf16(c, sn);
+      hp[j] = hi;
+      lp[j] = pack_bf16(c - __uint_as_float(hi << 16), sn - __uint_as_float(hi & 0xffff0000u));
+    }
+    const int ct = gpx >> 4, fl = (gpx & 15) + 16 * gquad;
+    eb[buf][ct][0][fl] = h;
+    eb[buf][ct][1][fl] = l;
+  };
+
+  f32x4 acc[RTW][CT];
+  auto clear = [&]() SB_INLINE {
+#pragma unroll
+    for (int r = 0; r < RTW; ++r)
+#pragma unroll
+      for (int c = 0; c < CT; ++c) acc[r][c] = f32x4{0, 0, 0, 0};
+  };
+  bf16x8 ahi[RTW], alo[RTW], nhi[RTW], nlo[RTW];
+#pragma unroll
+  for (int r = 0; r < RTW; ++r) nhi[r] = nlo[r] = bf16x8{};
+  // operand fragments of this wavefront's row tiles for chunk kc, into nhi and nlo
+  auto load_a = [&](int s, int rt0, int nmy, int kc) SB_INLINE {
+    const unsigned short* fr = static_cast<const unsigned short*>(p.afrag) +
+                               (long long)s * p.afrag_stride +
+                               ((long long)rt0 * p.kchunks + kc) * 1024;
+#pragma unroll
+    for (int r = 0; r < RTW; ++r)
+      if (r < nmy) {
+        const unsigned short* f = fr + (long long)r * p.kchunks * 1024;
+        nhi[r] = *reinterpret_cast<const bf16x8*>(f + lane * 8);
+        nlo[r] = *reinterpret_cast<const bf16x8*>(f + 512 + lane * 8);
+      }
+  };
+  auto take_a = [&]() SB_INLINE {
+#pragma unroll
+    for (int r = 0; r < RTW; ++r) {
+      ahi[r] = nhi[r];
+      alo[r] = nlo[r];
+    }
+  };
+  // rows beyond nmy (at most one per wavefront in a full pass) hold old fragments; their
+  // sums are never read
+  auto mul = [&](int nmy, int buf) SB_INLINE {
+    const bool last = nmy == RTW;
+    const auto mma = [](bf16x8 a, bf16x8 b, f32x4 c) SB_INLINE {
+      return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+    };
+#pragma unroll
+    for (int c = 0; c < CT; c += 2) {
+      bf16x8 b[2][2];  // [column][hi, lo]
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) b[q][h] = __builtin_bit_cast(bf16x8, eb[buf][c + q][h][lane]);
+#pragma unroll
+      for (int k = 0; k < 3; ++k)  // lo hi, hi lo, hi hi
+#pragma unroll
+        for (int r = 0; r + 1 < RTW; ++r)
+#pragma unroll
+          for (int q = 0; q < 2; ++q)
+            acc[r][c + q] = mma(k == 0 ? alo[r] : ahi[r], b[q][k == 1], acc[r][c + q]);
+      if (last) {
+        constexpr int r = RTW - 1;
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+#pragma unroll
+          for (int q = 0; q < 2; ++q)
+            acc[r][c + q] = mma(k == 0 ? alo[r] : ahi[r], b[q][k == 1], acc[r][c + q]);
+      }
+    }
+  };
+
+  // the sequence of (sample, first row tile of the pass, chunk); uniform over the workgroup
+  struct Step {
+    int s, rb, kc, nkc, nrt;
+  };
+  auto open = [&](int s) SB_INLINE {  // the first step at or after sample s; s = n_samples: none
+    Step t{s, 0, 0, 0, 0};
+    for (; t.s < p.n_samples; ++t.s) {
+      const int ne = p.n_eig[t.s], na = p.n_ant[t.s];
+      if (ne <= 0 || na <= 0) continue;
+      t.nkc = (na + 15) >> 4;
+      t.nrt = (2 * ne + 15) >> 4;
+      break;
+    }
+    return t;
+  };
+  auto next = [&](Step t) SB_INLINE {
+    if (t.kc + 1 < t.nkc) {
+      ++t.kc;
+      return t;
+    }
+    if (t.rb + RT_PASS < t.nrt) {
+      t.rb += RT_PASS;
+      t.kc = 0;
+      return t;
+    }
+    return open(t.s + 1);
+  };
+  // row tiles of this wavefront in the pass: the pass's tiles dealt evenly
+  auto rows = [&](const Step& t, int& rt0, int& nmy) SB_INLINE {
+    const int m = min(t.nrt - t.rb, RT_PASS), base = m / NWV, rem = m % NWV;
+    nmy = base + (wave < rem ? 1 : 0);
+    rt0 = t.rb + wave * base + min(wave, rem);
+  };
+
+  Step cur = open(0);
+  clear();
+  int rt0 = 0, nmy = 0, buf = 0;
+  const bool gen_first = wave < NWV / 2;
+  if (cur.s < p.n_samples) {
+    rows(cur, rt0, nmy);
+    load_a(cur.s, rt0, nmy, 0);
+    gen(cur.s, 0, 0);
+    take_a();
+  }
+  __syncthreads();
+  while (cur.s < p.n_samples) {
+    const Step nxt = next(cur);
+    const bool more = nxt.s < p.n_samples;
+    int nrt0 = 0, nnmy = 0;
+    if (more) {
+      rows(nxt, nrt0, nnmy);
+      load_a(nxt.s, nrt0, nnmy, nxt.kc);  // in flight for the whole step
+    }
+#pragma unroll 1
+    for (int half = 0; half < 2; ++half) {
+      if ((half == 0) == gen_first) {
+        if (more) gen(nxt.s, nxt.kc, buf ^ 1);
+      } else {
+        __builtin_amdgcn_s_setprio(1);
+        if (nmy > 0) mul(nmy, buf);
+        __builtin_amdgcn_s_setprio(0);
+      }
+    }
+    if (cur.kc + 1 == cur.nkc) {
+      // epilogue of the pass: I_l(x) += sum_e w_l[e] (Re^2 + Im^2)
+      if (nmy > 0) {
+        const float* wts = static_cast<const float*>(p.wts) + (size_t)cur.s * p.w_stride;
+        float pw0[RTW][CT], pw1[RTW][CT];
+#pragma unroll
+        for (int r = 0; r < RTW; ++r)
+#pragma unroll
+          for (int c = 0; c < CT; ++c) {
+            pw0[r][c] = acc[r][c][0] * acc[r][c][0] + acc[r][c][1] * acc[r][c][1];
+            pw1[r][c] = acc[r][c][2] * acc[r][c][2] + acc[r][c][3] * acc[r][c][3];
+          }
+        for (int lv = 0; lv < L; ++lv) {
+          float w0[RTW], w1[RTW];
+#pragma unroll
+          for (int r = 0; r < RTW; ++r) {
+            // accumulator registers (0,1) and (2,3) of this lane hold eigenvectors e0, e0 + 1
+            const int e0 = (rt0 + r) * 8 + 2 * (lane >> 4);
+            w0[r] = r < nmy ? wts[(size_t)lv * p.epad + e0] : 0.0f;
+            w1[r] = r < nmy ? wts[(size_t)lv * p.epad + e0 + 1] : 0.0f;
+          }
+          float v[CT];
+#pragma unroll
+          for (int c = 0; c < CT; ++c) {
+            v[c] = 0;
+#pragma unroll
+            for (int r = 0; r < RTW; ++r) v[c] += w0[r] * pw0[r][c] + w1[r] * pw1[r][c];
+          }
+#pragma unroll
+          for (int h = 0; h < CT / 4; ++h) img_acc[wave][lv][h * 64 + lane] += sum_columns(v + 4 * h);
+        }
+      }
+      clear();
+    }
+    take_a();
+    __syncthreads();
+    cur = nxt;
+    rt0 = nrt0;
+    nmy = nnmy;
+    buf ^= 1;
+  }
+  __syncthreads();
+  float* img = static_cast<float*>(p.img);
+  for (int i = tid; i < L * TP; i += SB_NT) {
+    const int lv = i / TP, px = i % TP;
+    const int q = q0 + px;
+    if (q >= p.n_pix) continue;
+    // column tile c = px / 16 sits in lane row (c % 4 with its two bits swapped) of group c / 4
+    const int c = px >> 4, row = ((c & 1) << 1) | ((c >> 1) & 1);
+    const int k = (c >> 2) * 64 + row * 16 + (px & 15);
+    float v = img_acc[0][lv][k];
+#pragma unroll
+    for (int w = 1; w < NWV; ++w) v += img_acc[w][lv][k];
+    img[(size_t)lv * p.img_ld + q] += v;
+  }
+}
+
 }  // namespace
 
 size_t steer_frag_elems_per_sample(int mode, int rtiles, int kchunks) {
@@ -520,8 +749,14 @@ void launch_steer(const SteerParams& p, int mode, hipStream_t stream) {
   if (p.n_samples <= 0 || p.n_pix <= 0) return;
   if (p.n_levels > LMAX) fail(BIPP_INVALID_PARAMETER_ERROR, "at most 8 energy levels per image batch");
   if (mode == STEER_BF16X3) {
-    constexpr int TP = SteerCfg<STEER_BF16X3>::TP;
-    steer_kernel<STEER_BF16X3><<<ceil_div(p.n_pix, TP), SteerCfg<STEER_BF16X3>::NT, 0, stream>>>(p);
+    // row tiles per wavefront for the largest sample of the batch, at most four
+    const dim3 grid(ceil_div(p.n_pix, SB_TP));
+    switch (std::min(4, ceil_div(p.rtiles, SB_NW))) {
+      case 1: steer_bf16x3_kernel<1><<<grid, SB_NT, 0, stream>>>(p); break;
+      case 2: steer_bf16x3_kernel<2><<<grid, SB_NT, 0, stream>>>(p); break;
+      case 3: steer_bf16x3_kernel<3><<<grid, SB_NT, 0, stream>>>(p); break;
+      default: steer_bf16x3_kernel<4><<<grid, SB_NT, 0, stream>>>(p); break;
+    }
   } else if (mode == STEER_FP32) {
     constexpr int TP = SteerCfg<STEER_FP32>::TP;
     steer_kernel<STEER_FP32><<<ceil_div(p.n_pix, TP), SteerCfg<STEER_FP32>::NT, 0, stream>>>(p);
