@@ -16,6 +16,7 @@ template <typename R>
 struct EigRunner {
   DevBuf n_red, idx, n_vis, info, counter, order, d, z, ws_a, ws_l, ws_z, prof_buf;
   DevBuf sig, w_i, tmp, g, v_full;
+  DevBuf split_c, split_r, split_i;
   int n_samples = 0, n_ant = 0, nmax = 0;
   bool general_w = false;
   std::vector<int> h_info;
@@ -153,10 +154,17 @@ struct EigRunner {
     ep.ldz = nmax;
     ep.ws_ld = nmax;
     ep.ws_stride = nn;
+    ep.info = info.as<int>(nS);
+    if constexpr (sizeof(R) == 8) {
+      if (nmax > SPLIT_ABOVE && !standard) {
+        run_split(ctx, ep, h_nred, h_order, s_double);
+        unbeam_general(nS, nAnt, st);
+        return;
+      }
+    }
     ep.ws_a = ws_a.as<cplx<R>>((size_t)n_slots * nn);
     ep.ws_l = ws_l.as<cplx<R>>((size_t)n_slots * nn);
     ep.ws_z = ws_z.as<R>((size_t)n_slots * nn);
-    ep.info = info.as<int>(nS);
     // BIPP_EIG_PROFILE=1: per-phase wall-clock averages of this launch on stderr
     const bool prof = std::getenv("BIPP_EIG_PROFILE") != nullptr;
     if (prof) {
@@ -203,30 +211,60 @@ struct EigRunner {
       std::fprintf(stderr, "\n");
     }
 
-    if (general_w) {
-      // V = W_I Z (src/eigensolver.cpp:214-216)
-      cplx<R>* vf = v_full.as<cplx<R>>((size_t)nS * nAnt * nmax);
-      BIPP_HIP(hipMemsetAsync(vf, 0, sizeof(cplx<R>) * (size_t)nS * nAnt * nmax, st));
-      GemmBatch<R> g3{};
-      g3.n_batch = nS;
-      g3.m = nullptr;
-      g3.m0 = nAnt;
-      g3.n = fp.n_red;
-      g3.k = fp.n_red;
-      g3.op_a = 0;
-      g3.op_b = 0;
-      g3.alpha = mk<R>(1, 0);
-      g3.beta = mk<R>(0, 0);
-      g3.a = static_cast<const cplx<R>*>(w_i.p);
-      g3.lda = nAnt;
-      g3.stride_a = (long long)nAnt * nmax;
-      g3.b = ep.z_out;
-      g3.ldb = nmax;
-      g3.stride_b = nn;
-      g3.c = vf;
-      g3.ldc = nAnt;
-      g3.stride_c = (long long)nAnt * nmax;
-      launch_gemm_batch<R>(g3, nAnt, nmax, st);
+    unbeam_general(nS, nAnt, st);
+  }
+
+  // V = W_I Z for a general W (src/eigensolver.cpp:214-216)
+  void unbeam_general(int nS, int nAnt, hipStream_t st) {
+    if (!general_w) return;
+    cplx<R>* vf = v_full.as<cplx<R>>((size_t)nS * nAnt * nmax);
+    BIPP_HIP(hipMemsetAsync(vf, 0, sizeof(cplx<R>) * (size_t)nS * nAnt * nmax, st));
+    GemmBatch<R> g3{};
+    g3.n_batch = nS;
+    g3.m = nullptr;
+    g3.m0 = nAnt;
+    g3.n = d_n_red();
+    g3.k = d_n_red();
+    g3.op_a = 0;
+    g3.op_b = 0;
+    g3.alpha = mk<R>(1, 0);
+    g3.beta = mk<R>(0, 0);
+    g3.a = static_cast<const cplx<R>*>(w_i.p);
+    g3.lda = nAnt;
+    g3.stride_a = (long long)nAnt * nmax;
+    g3.b = d_z();
+    g3.ldb = nmax;
+    g3.stride_b = (long long)nmax * nmax;
+    g3.c = vf;
+    g3.ldc = nAnt;
+    g3.stride_c = (long long)nAnt * nmax;
+    launch_gemm_batch<R>(g3, nAnt, nmax, st);
+  }
+
+  // Above this many beams the batch is solved phase by phase over all samples, at most
+  // SPLIT_JOBS of them at a time (10 MB of scratch per sample at 512 beams, as many as the
+  // persistent form's slots): a sample's single-CU time there is 55 ms (400..512 beams), the
+  // phase-split batch takes PLACEHOLDER.  Up to 256 beams the persistent form keeps one workgroup
+  // per sample.
+  static constexpr int SPLIT_ABOVE = 256;
+  static constexpr int SPLIT_JOBS = 256;
+
+  void run_split(ContextImpl& ctx, EigParams<double> ep, const std::vector<int>& h_nred,
+                 const std::vector<int>& h_order, bool s_double) {
+    const int nS = ep.n_jobs, n_chunks = ceil_div(nS, SPLIT_JOBS), per = ceil_div(nS, n_chunks);
+    const size_t nn = (size_t)ep.ws_stride;
+    ep.ws_a = ws_a.as<cplx<double>>(per * nn);
+    ep.ws_l = ws_l.as<cplx<double>>(per * nn);
+    ep.ws_z = ws_z.as<double>(per * nn);
+    const EigSplitSizes z = eig_split_sizes(per, ep.nmax);
+    const EigSplitBuffers b{split_c.as<cplx<double>>(z.cplx_elems), split_r.as<double>(z.real_elems),
+                            split_i.as<int>(z.int_elems)};
+    const int* order0 = ep.order;
+    for (int k = 0; k < nS; k += per) {
+      ep.order = order0 + k;
+      ep.n_jobs = std::min(per, nS - k);
+      // largest first: the chunk's first sample has its largest reduced size
+      launch_eig_split(ep, b, h_nred[h_order[k]], ctx.n_cu, s_double, ctx.stream);
     }
   }
 

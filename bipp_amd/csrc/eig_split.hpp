@@ -1,0 +1,619 @@
+// Phase-split form of the batched generalized eigensolver (float64): one launch per phase over
+// all samples of a batch instead of one workgroup per sample for all phases.
+//
+// The persistent kernel (eig_kernel) gives a sample one CU, so a batch of fewer samples than
+// CUs leaves the rest of the chip idle and a sample takes its single-CU time: 55 ms for twelve
+// 400..512-antenna samples, 64 ms for 96 of them (tridiagonalisation 23, back-transform 17,
+// whitening 3.9, un-whitening 3.0, load 1.3 ms per sample).  Here the dense phases run on tiles
+// or column groups of every sample, and the tridiagonalisation, whose column steps depend on
+// each other, takes one launch per column with several workgroups per sample.  The Cholesky
+// inverse and the divide and conquer keep a workgroup per sample (the phases of eig_kernel).
+//
+// Buffers (leading dimension nmax): p.z_out[sample] holds the reduced S, then C, then the
+// reflectors and T factors, and in the end the eigenvectors; p.ws_l[job] G, then W = L^-1;
+// p.ws_a[job] scratch (W S, the divide and conquer's arrays, the back-transformed vectors);
+// p.ws_z[job] the eigenvectors of the tridiagonal.  job: position in p.order.
+#pragma once
+
+// Job and unit of a workgroup when `per_job` units of each job are to run on one XCD (workgroup
+// x runs on XCD x mod 8): a job's operands then stay in that XCD's L2.
+struct SplitUnit {
+  int job, unit;
+};
+__device__ __forceinline__ SplitUnit split_unit(int per_job, int n_jobs) {
+  const int n_units = per_job * n_jobs, per_xcd = (n_units + 7) / 8;
+  const int u = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if (static_cast<int>(blockIdx.x >> 3) >= per_xcd || u >= n_units) return {-1, 0};
+  return {u / per_job, u % per_job};
+}
+inline unsigned split_grid(int per_job, int n_jobs) {
+  return static_cast<unsigned>(8 * ((static_cast<long long>(per_job) * n_jobs + 7) / 8));
+}
+
+// The reduced pencil: S (full) into z_out, G into ws_l.  Workgroup: 16 columns of one job.
+template <typename TIn>
+__global__ __launch_bounds__(256) void split_load_kernel(EigParams<double> p) {
+  const int job = blockIdx.y, sid = p.order[job], n = p.n_red[sid];
+  const int j1 = min(n, static_cast<int>(blockIdx.x) * 16 + 16);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int* idx = p.idx + (size_t)sid * p.idx_stride;
+  const cplx<TIn>* S = reinterpret_cast<const cplx<TIn>*>(p.s) + (size_t)sid * p.stride_s;
+  const double* xyz = p.xyz + (size_t)sid * p.stride_xyz;
+  const cplx<double>* Gin = p.g_in ? p.g_in + (size_t)sid * p.stride_g : nullptr;
+  cplx<double>* A = p.z_out + (size_t)sid * p.stride_z;
+  cplx<double>* L = p.ws_l + (size_t)job * p.ws_stride;
+  const double wl = p.wl[sid];
+  for (int j = blockIdx.x * 16 + wave; j < j1; j += 4) {
+    const int bj = idx[j];
+    for (int i = lane; i < n; i += 64) {
+      const int bi = idx[i];
+      cplx<TIn> sv = (bi >= bj) ? S[bi + (size_t)bj * p.lds] : conj(S[bj + (size_t)bi * p.lds]);
+      cplx<double> a = cvt<double>(sv);
+      if (i == j) a.im = 0;
+      A[i + (size_t)j * p.ldz] = a;
+      cplx<double> g;
+      if (Gin) {
+        g = Gin[i + (size_t)j * p.ld_g];
+      } else if (i == j) {
+        g = mk<double>(p.gram_prefactor, 0);
+      } else {
+        const double dx = xyz[bi] - xyz[bj], dy = xyz[bi + p.ldxyz] - xyz[bj + p.ldxyz],
+                     dz = xyz[bi + 2 * p.ldxyz] - xyz[bj + 2 * p.ldxyz];
+        const double x = 2.0 * sqrt(dx * dx + dy * dy + dz * dz) / wl;
+        const double sc = x != 0.0 ? sinpi(x) / (3.14159265358979323846 * x) : 1.0;
+        g = mk<double>(p.gram_prefactor * sc, 0);
+      }
+      L[i + (size_t)j * p.ws_ld] = g;
+    }
+  }
+}
+
+// W = L^-1 of G = L L^H in place (scratch ws_a); info and, where there is nothing to solve,
+// the eigenvalues.  Workgroup per job.
+template <int NMAX>
+__global__ __launch_bounds__(EigCfg<NMAX>::NT) void split_chol_kernel(EigParams<double> p) {
+  const int job = blockIdx.x, sid = p.order[job], n = p.n_red[sid], tid = threadIdx.x;
+  int info = 0;
+  if (n > 0) {
+    const int bad = chol_phase<double, NMAX>(n, p.ws_l + (size_t)job * p.ws_stride, p.ws_ld,
+                                             p.ws_a + (size_t)job * p.ws_stride, p.ws_ld, nullptr);
+    // leading minor bad + 1 of G is not positive definite: ?hegv reports info = n + bad + 1
+    if (bad >= 0) info = n + bad + 1;
+  }
+  if (n <= 0 || info)
+    for (int j = tid; j < p.nmax; j += EigCfg<NMAX>::NT) p.d_out[(size_t)sid * p.stride_d + j] = 0;
+  if (tid == 0) p.info[sid] = info;
+}
+
+// Dense products on 64 x 64 tiles, a wavefront per 32 x 32 quadrant (2 x 2 blocks of
+// v_mfma_f64_16x16x4f64, four per complex product), operands straight from global memory with
+// the next four k in flight: an MFMA takes 64 cycles, so a CU reads 16 bytes per cycle, a
+// quarter of what its L1 delivers, and neither LDS nor barriers are needed.  D[j][i] is
+// formed (A operand: rows j, B operand: rows i), so stores write 16 consecutive rows.
+//   MODE 0: ws_a = W S       = sum_{k <= i} W[i,k] conj(S[j,k])          (S Hermitian)
+//   MODE 1: z_out = ws_a W^H = sum_{k <= j} X[i,k] conj(W[j,k]), lower triangle, real diagonal
+//   MODE 2: z_out = W^H ws_a = sum_{k >= i} conj(W[k,i]) X[k,j]
+template <int MODE>
+__global__ __launch_bounds__(256) void split_gemm_kernel(EigParams<double> p, int tiles_side) {
+  typedef double f64x4 __attribute__((ext_vector_type(4)));
+  const int n_tiles = MODE == 1 ? tiles_side * (tiles_side + 1) / 2 : tiles_side * tiles_side;
+  const SplitUnit u = split_unit(n_tiles, p.n_jobs);
+  if (u.job < 0) return;
+  const int sid = p.order[u.job], n = p.n_red[sid];
+  if (p.info[sid] != 0) return;
+  int ti, tj;
+  if (MODE == 1) {
+    ti = 0;
+    while ((ti + 1) * (ti + 2) / 2 <= u.unit) ++ti;
+    tj = u.unit - ti * (ti + 1) / 2;
+  } else {
+    ti = u.unit % tiles_side;
+    tj = u.unit / tiles_side;
+  }
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int ib = 64 * ti + 32 * (wave & 1), jb = 64 * tj + 32 * (wave >> 1);
+  if (ib >= n || jb >= n || (MODE == 1 && jb > ib + 31)) return;
+  const int ld = p.ws_ld;
+  const cplx<double>* W = p.ws_l + (size_t)u.job * p.ws_stride;
+  cplx<double>* X = p.ws_a + (size_t)u.job * p.ws_stride;
+  cplx<double>* A = p.z_out + (size_t)sid * p.stride_z;
+  const int lr = lane & 15, lk = lane >> 4;
+  const int jr[2] = {jb + lr, jb + 16 + lr}, ir[2] = {ib + lr, ib + 16 + lr};
+  const int k0 = MODE == 2 ? ib : 0;
+  const int k1 = MODE == 0 ? min(n, ib + 32) : (MODE == 1 ? min(n, jb + 32) : n);
+  f64x4 dr[2][2], di[2][2];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      dr[a][b] = f64x4{0, 0, 0, 0};
+      di[a][b] = f64x4{0, 0, 0, 0};
+    }
+  auto load = [&](int k, cplx<double>* P, cplx<double>* Q) {
+    const int e = k + lk;
+    const bool ok = e < k1;
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const int j = jr[b], i = ir[b];
+      P[b] = Q[b] = mk<double>(0, 0);
+      if (MODE == 0) {
+        if (ok && j < n) P[b] = A[j + (size_t)e * ld];
+        if (ok && i < n && e <= i) Q[b] = W[i + (size_t)e * ld];
+      } else if (MODE == 1) {
+        if (ok && j < n && e <= j) P[b] = W[j + (size_t)e * ld];
+        if (ok && i < n) Q[b] = X[i + (size_t)e * ld];
+      } else {
+        if (ok && j < n) P[b] = X[e + (size_t)j * ld];
+        if (ok && i < n && e >= i) Q[b] = W[e + (size_t)i * ld];
+      }
+    }
+  };
+  cplx<double> P[2], Q[2];
+  load(k0, P, Q);
+  for (int k = k0; k < k1; k += 4) {
+    cplx<double> Pn[2], Qn[2];
+    load(k + 4, Pn, Qn);
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        // conj(P) Q: re Pr Qr + Pi Qi, im Pr Qi - Pi Qr (MODE 2: P conj(Q), the conjugate)
+        dr[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(P[a].re, Q[b].re, dr[a][b], 0, 0, 0);
+        dr[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(P[a].im, Q[b].im, dr[a][b], 0, 0, 0);
+        di[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(P[a].re, Q[b].im, di[a][b], 0, 0, 0);
+        di[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(-P[a].im, Q[b].re, di[a][b], 0, 0, 0);
+      }
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      P[b] = Pn[b];
+      Q[b] = Qn[b];
+    }
+  }
+  cplx<double>* out = MODE == 0 ? X : A;
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int j = jb + 16 * a + lk + 4 * r, i = ir[b];
+        if (i >= n || j >= n || (MODE == 1 && i < j)) continue;
+        double im = MODE == 2 ? -di[a][b][r] : di[a][b][r];
+        if (MODE == 1 && i == j) im = 0;
+        out[i + (size_t)j * ld] = mk<double>(dr[a][b][r], im);
+      }
+}
+
+// --------------------------------------------------------------------------------------
+// Tridiagonalisation, one launch per column c (zhetd2 order, lower triangle).
+//
+// State between launches (parity c & 1): the reflector v_c and tau_c, and y = A v_c over the
+// trailing matrix as per-workgroup row sums plus the column sums.  Launch c
+//   - forms w_{c-1} from y, v_{c-1}, tau_{c-1}, the updated column c and its reflector v_c (every
+//     workgroup of the sample for itself, from the same operands in the same order, so all
+//     hold the same bits; workgroup 0 records d_c, e_c, v_c, tau_c and puts v_{c-1} into its
+//     column of A);
+//   - applies the pending update A -= v w^H + w v^H (of c - 1) to its columns of the trailing
+//     matrix and adds their part of A v_c from the updated lower triangle.
+// Bound: the launches follow each other (a prologue of two workgroup sums and the round trip
+// through the last-level cache per launch), then, for many samples, the last-level cache (the
+// trailing triangle read and written once per column).  Lanes hold 16 rows x 4 columns, so a
+// column's sum takes four lane moves for four columns at once, and row sums over the columns
+// of a wavefront stay in registers.  Column tiles of 4 are dealt to the sample's wavefronts in
+// turn, which keeps them balanced while the trailing matrix shrinks.
+// --------------------------------------------------------------------------------------
+constexpr int TRI_NT = 512, TRI_NW = TRI_NT / 64, TRI_GMAX = 8;
+
+struct TriWork {
+  cplx<double>* v;     // [job][2][nmax]
+  cplx<double>* tau;   // [job][2]
+  cplx<double>* col;   // [job][2][nmax] column sums
+  cplx<double>* row;   // [job][2][TRI_GMAX][nmax] row sums of each workgroup
+  double* de;          // [job][nmax][2] diagonal, subdiagonal
+  int* perm;           // [job][nmax]
+};
+
+struct TriShared {
+  cplx<double> v[TRI_NT], w[TRI_NT], vn[TRI_NT];
+  cplx<double> xw[TRI_NW][TRI_NT];  // a wavefront's row sums
+  double red[2][2 * TRI_NW];
+  cplx<double> yc, alpha;
+};
+
+// Sum of (re, im) over the four 16-lane rows: lane rows 0 and 1 return the real total, rows 2
+// and 3 the imaginary one.  permlane32_swap leaves both operands' lower halves in the first
+// result and their upper halves in the second; permlane16_swap does so with each pair of rows.
+__device__ __forceinline__ double rows_total(double re, double im) {
+  auto swap32 = [](unsigned a, unsigned b) {
+    return __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  };
+  auto swap16 = [](unsigned a, unsigned b) {
+    return __builtin_amdgcn_permlane16_swap(a, b, false, false);
+  };
+  auto mk64 = [](unsigned lo, unsigned hi) {
+    return __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi) << 32) | lo));
+  };
+  const unsigned long long r = __double_as_longlong(re), q = __double_as_longlong(im);
+  const auto lo = swap32(static_cast<unsigned>(r), static_cast<unsigned>(q));
+  const auto hi = swap32(static_cast<unsigned>(r >> 32), static_cast<unsigned>(q >> 32));
+  const double z = mk64(lo[0], hi[0]) + mk64(lo[1], hi[1]);
+  const unsigned long long zz = __double_as_longlong(z);
+  const auto l2 = swap16(static_cast<unsigned>(zz), static_cast<unsigned>(zz));
+  const auto h2 = swap16(static_cast<unsigned>(zz >> 32), static_cast<unsigned>(zz >> 32));
+  return mk64(l2[0], h2[0]) + mk64(l2[1], h2[1]);
+}
+
+// sums of a and b over the workgroup in a fixed order; one barrier (slots alternate)
+__device__ __forceinline__ void tri_sum2(double& a, double& b, double* red) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  a = wave_total(a);
+  b = wave_total(b);
+  if (lane == 0) {
+    red[wave] = a;
+    red[TRI_NW + wave] = b;
+  }
+  __syncthreads();
+  a = 0;
+  b = 0;
+#pragma unroll
+  for (int w = 0; w < TRI_NW; ++w) {
+    a += red[w];
+    b += red[TRI_NW + w];
+  }
+}
+
+// NCT: column tiles of a wavefront taken together (a tile's row operands are read once)
+template <int NCT>
+__global__ __launch_bounds__(TRI_NT) void tri_column_kernel(EigParams<double> p, TriWork tw, int c) {
+  __shared__ TriShared sh;
+  const int job = blockIdx.y, g = blockIdx.x, G = gridDim.x;
+  const int sid = p.order[job], n = p.n_red[sid];
+  if (c >= n || p.info[sid] != 0 || (c == n - 1 && g != 0)) return;  // uniform
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ld = p.ldz, nmax = p.nmax;
+  cplx<double>* A = p.z_out + (size_t)sid * p.stride_z;
+  const int cur = c & 1, prv = cur ^ 1;
+  const size_t j2 = (size_t)job * 2;
+  const bool apply = c > 0;
+
+  // ---- w_{c-1}, column c, its reflector; thread i holds row i ----------------------------
+  const int i = tid;
+  const bool live = i >= c && i < n;
+  cplx<double> a = mk<double>(0, 0), v = a, y = a, w = a, tau = a;
+  if (live) {
+    a = A[i + (size_t)c * ld];
+    if (apply) {
+      v = tw.v[(j2 + prv) * nmax + i];
+      y = tw.col[(j2 + prv) * nmax + i];
+      for (int q = 0; q < G; ++q) y = y + tw.row[((j2 + prv) * TRI_GMAX + q) * nmax + i];
+    }
+  }
+  if (apply) {
+    tau = tw.tau[j2 + prv];
+    if (i == c) sh.yc = y;
+    const cplx<double> x = tau * y;
+    const cplx<double> dt = cmul_conj_a(x, v);
+    double pr = dt.re, pi = dt.im;
+    tri_sum2(pr, pi, sh.red[0]);
+    const cplx<double> alpha2 = tau * mk<double>(-0.5 * pr, -0.5 * pi);
+    w = x + alpha2 * v;
+    const cplx<double> wc = tau * sh.yc + alpha2;  // row c, where v is 1
+    if (live) a = a - (v * conj(wc) + w);
+  }
+  sh.v[i] = v;
+  sh.w[i] = w;
+  if (i == c + 1) sh.alpha = a;
+  double part = live && i >= c + 2 ? abs2(a) : 0.0, unused = 0;
+  tri_sum2(part, unused, sh.red[1]);
+  if (g == 0 && live) {
+    if (apply) {
+      if (i > c)
+        A[i + (size_t)(c - 1) * ld] = v;
+      else
+        A[(c - 1) + (size_t)(c - 1) * ld] = tau;  // the diagonal slot keeps tau
+    }
+    if (i == c) {
+      tw.de[((size_t)job * nmax + c) * 2] = a.re;
+      if (c == n - 1) {
+        tw.de[((size_t)job * nmax + c) * 2 + 1] = 0;
+        A[c + (size_t)c * ld] = mk<double>(0, 0);  // no reflector for the last column
+      }
+    }
+  }
+  if (c == n - 1) return;
+  const cplx<double> alpha = sh.alpha;
+  cplx<double> tn, scal;
+  double beta;
+  if (part == 0.0 && alpha.im == 0.0) {
+    tn = mk<double>(0, 0);
+    beta = alpha.re;
+    scal = mk<double>(0, 0);
+  } else {
+    const double nrm = sqrt(alpha.re * alpha.re + alpha.im * alpha.im + part);
+    beta = alpha.re >= 0.0 ? -nrm : nrm;
+    tn = mk<double>((beta - alpha.re) / beta, -alpha.im / beta);
+    scal = crecip(mk<double>(alpha.re - beta, alpha.im));
+  }
+  const cplx<double> vn = i == c + 1 ? mk<double>(1, 0) : (live && i >= c + 2 ? a * scal : mk<double>(0, 0));
+  sh.vn[i] = vn;
+  if (g == 0) {
+    if (live && i > c) tw.v[(j2 + cur) * nmax + i] = vn;
+    if (i == c) {
+      tw.tau[j2 + cur] = tn;
+      tw.de[((size_t)job * nmax + c) * 2 + 1] = beta;
+    }
+  }
+  // ---- pass over this wavefront's column tiles ------------------------------------------
+  const int i0 = c + 1;
+  for (int r = (i0 & ~63) + lane; r < n; r += 64) sh.xw[wave][r] = mk<double>(0, 0);
+  __syncthreads();
+  const int lr = lane & 15, lc = lane >> 4;
+  const int W = G * TRI_NW, gw = g * TRI_NW + wave;
+  const int ct_end = (n + 3) >> 2, rt_end = (n + 15) >> 4;
+  int ct = i0 >> 2;
+  ct += (gw - ct % W + W) % W;  // first tile at or after column i0 that is this wavefront's
+  constexpr int RU = 8 / NCT;   // row tiles loaded together: eight elements in flight per lane
+  for (; ct < ct_end; ct += NCT * W) {
+    int jc[NCT];
+    cplx<double> cv[NCT], cw[NCT], cn[NCT], cs[NCT];
+#pragma unroll
+    for (int u = 0; u < NCT; ++u) {
+      const int j = 4 * (ct + u * W) + lc;
+      jc[u] = j >= i0 && j < n ? j : n;  // n: no such column (every row test fails)
+      const int jj = min(jc[u], TRI_NT - 1);
+      cv[u] = conj(sh.v[jj]);
+      cw[u] = conj(sh.w[jj]);
+      cn[u] = sh.vn[jj];
+      cs[u] = mk<double>(0, 0);
+    }
+    cplx<double> x[RU][NCT], xn[RU][NCT];
+    auto load = [&](int rt, cplx<double>(&o)[RU][NCT]) {
+#pragma unroll
+      for (int k = 0; k < RU; ++k)
+#pragma unroll
+        for (int u = 0; u < NCT; ++u) {
+          const int r = 16 * (rt + k) + lr;
+          o[k][u] = r < n && r >= jc[u] ? A[r + (size_t)jc[u] * ld] : mk<double>(0, 0);
+        }
+    };
+    const int rt0 = ct >> 2;
+    load(rt0, x);
+    for (int rt = rt0; rt < rt_end; rt += RU) {
+      if (rt + RU < rt_end) load(rt + RU, xn);
+#pragma unroll
+      for (int k = 0; k < RU; ++k) {
+        const int r = 16 * (rt + k) + lr;
+        if (16 * (rt + k) >= n) break;  // uniform
+        const int rr = min(r, TRI_NT - 1);
+        const cplx<double> vi = sh.v[rr], wi = sh.w[rr], ni = sh.vn[rr];
+        cplx<double> acc = mk<double>(0, 0);
+#pragma unroll
+        for (int u = 0; u < NCT; ++u) {
+          if (r < n && r >= jc[u]) {
+            cplx<double> e = x[k][u];
+            if (apply) {
+              e = e - (vi * cw[u] + wi * cv[u]);
+              A[r + (size_t)jc[u] * ld] = e;
+            }
+            acc = acc + e * cn[u];
+            if (r > jc[u]) cs[u] = cs[u] + cmul_conj_a(e, ni);
+          }
+        }
+        const double t = rows_total(acc.re, acc.im);
+        if (!(lc & 1) && r < n) {
+          double* o = reinterpret_cast<double*>(&sh.xw[wave][r]) + (lc >> 1);
+          *o += t;
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < RU; ++k)
+#pragma unroll
+        for (int u = 0; u < NCT; ++u) x[k][u] = xn[k][u];
+    }
+#pragma unroll
+    for (int u = 0; u < NCT; ++u) {
+      const cplx<double> s = mk<double>(sum16(cs[u].re), sum16(cs[u].im));
+      if (lr == 0 && jc[u] < n) tw.col[(j2 + cur) * nmax + jc[u]] = s;
+    }
+  }
+  __syncthreads();
+  if (i >= i0 && i < n) {
+    cplx<double> s = sh.xw[0][i];
+#pragma unroll
+    for (int q = 1; q < TRI_NW; ++q) s = s + sh.xw[q][i];
+    tw.row[((j2 + cur) * TRI_GMAX + g) * nmax + i] = s;
+  }
+}
+
+// Eigenpairs of the tridiagonal (dc_phase, scratch ws_a), ascending order: eigenvalues to
+// d_out, the column order to perm.  Workgroup per job.
+template <int NMAX>
+__global__ __launch_bounds__(EigCfg<NMAX>::NT) void split_dc_kernel(EigParams<double> p, TriWork tw) {
+  EigShared<double, NMAX>& sh = eig_sh<double, NMAX>;
+  constexpr int NT_ = EigCfg<NMAX>::NT;
+  const int job = blockIdx.x, sid = p.order[job], n = p.n_red[sid], tid = threadIdx.x;
+  if (n <= 0 || p.info[sid] != 0) return;
+  for (int i = tid; i < n; i += NT_) {
+    sh.de[i].x = tw.de[((size_t)job * p.nmax + i) * 2];
+    sh.de[i].y = tw.de[((size_t)job * p.nmax + i) * 2 + 1];
+  }
+  __syncthreads();
+  dc_phase<double, NMAX>(n, p.ws_z + (size_t)job * p.ws_stride, p.ws_ld,
+                         reinterpret_cast<double*>(p.ws_a + (size_t)job * p.ws_stride), nullptr);
+  rank_order<double, NMAX>(n, sh);
+  for (int j = tid; j < p.nmax; j += NT_) {
+    p.d_out[(size_t)sid * p.stride_d + j] = j < n ? sh.de[sh.perm[j]].x : 0.0;
+    if (j < n) tw.perm[(size_t)job * p.nmax + j] = sh.perm[j];
+  }
+}
+
+// --------------------------------------------------------------------------------------
+// Back-transform ws_a = Q Z[:, perm] in compact-WY blocks of 16 reflectors on
+// v_mfma_f64_16x16x4f64 (the scheme and layouts of back_transform_mfma), over workgroups of
+// 16 eigenvector columns: four wavefronts take alternate 16-row blocks of them (in registers
+// for the whole phase) and exchange one partial product per reflector block through LDS.  The
+// reflectors come straight from A (they are read by every column group of the sample, all
+// on one XCD); an MFMA takes 64 cycles, so their loads cost a CU 16 bytes per cycle.
+// --------------------------------------------------------------------------------------
+// v_{cs + q} at row i (1 at its unit entry, 0 above it and for cs + q < 0)
+__device__ __forceinline__ cplx<double> wy_elem(const cplx<double>* A, int ld, int n, int col, int i) {
+  if (col < 0 || i <= col || i >= n) return mk<double>(0, 0);
+  return i == col + 1 ? mk<double>(1, 0) : A[i + (size_t)col * ld];
+}
+
+// T factor of one block of reflectors into the strict upper triangle of A: entry (p, q),
+// p <= q, at A[cs + p, cs + q + 1].
+__global__ __launch_bounds__(256) void split_tfac_kernel(EigParams<double> p) {
+  typedef double f64x4 __attribute__((ext_vector_type(4)));
+  __shared__ double red[4][64][8];
+  __shared__ cplx<double> gm[16][16], t[16][16], tau[16];
+  const int b = blockIdx.x, sid = p.order[blockIdx.y], n = p.n_red[sid];
+  const int nblk = (n - 1 + 15) / 16;
+  if (b >= nblk || p.info[sid] != 0) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lr = lane & 15, lk = lane >> 4;
+  cplx<double>* A = p.z_out + (size_t)sid * p.stride_z;
+  const int ld = p.ldz, cs = n - 2 - 16 * b - 15;
+  const int rb0 = (max(cs, 0) + 1) / 16, rb1 = (n + 15) / 16;
+  f64x4 gr = {0, 0, 0, 0}, gi = {0, 0, 0, 0};
+  for (int rb = rb0 + wave; rb < rb1; rb += 4)
+#pragma unroll
+    for (int s4 = 0; s4 < 4; ++s4) {
+      const cplx<double> v = wy_elem(A, ld, n, cs + lr, rb * 16 + 4 * s4 + lk);
+      gr = __builtin_amdgcn_mfma_f64_16x16x4f64(v.re, v.re, gr, 0, 0, 0);
+      gr = __builtin_amdgcn_mfma_f64_16x16x4f64(v.im, v.im, gr, 0, 0, 0);
+      gi = __builtin_amdgcn_mfma_f64_16x16x4f64(v.re, v.im, gi, 0, 0, 0);
+      gi = __builtin_amdgcn_mfma_f64_16x16x4f64(-v.im, v.re, gi, 0, 0, 0);
+    }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    red[wave][lane][r] = gr[r];
+    red[wave][lane][4 + r] = gi[r];
+  }
+  if (tid < 16) tau[tid] = cs + tid >= 0 ? A[(cs + tid) + (size_t)(cs + tid) * ld] : mk<double>(0, 0);
+  __syncthreads();
+  if (wave != 0) return;  // no workgroup barrier below
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    gm[lk + 4 * r][lr] = mk<double>(
+        (red[0][lane][r] + red[1][lane][r]) + (red[2][lane][r] + red[3][lane][r]),
+        (red[0][lane][4 + r] + red[1][lane][4 + r]) + (red[2][lane][4 + r] + red[3][lane][4 + r]));
+  wave_sync();
+  for (int i = 0; i < 16; ++i) {
+    if (lane < 16) {
+      cplx<double> val = mk<double>(0, 0);
+      if (lane == i) {
+        val = tau[i];
+      } else if (lane < i) {
+        cplx<double> acc = mk<double>(0, 0);
+        for (int q = lane; q < i; ++q) acc = acc + t[lane][q] * gm[q][i];
+        val = mk<double>(0, 0) - tau[i] * acc;
+      }
+      t[lane][i] = val;
+    }
+    wave_sync();
+  }
+  for (int e = lane; e < 256; e += 64) {
+    const int pr = e / 16, q = e % 16;
+    if (pr <= q && cs + pr >= 0) A[(cs + pr) + (size_t)(cs + q + 1) * ld] = t[pr][q];
+  }
+}
+
+template <int NMAX>
+__global__ __launch_bounds__(256) void split_bt_kernel(EigParams<double> p, TriWork tw, int groups) {
+  typedef double f64x4 __attribute__((ext_vector_type(4)));
+  constexpr int NWV = 4, RBW = NMAX / 16 / NWV;
+  __shared__ double red[2][NWV][64][8];
+  const SplitUnit u = split_unit(groups, p.n_jobs);
+  if (u.job < 0) return;
+  const int sid = p.order[u.job], n = p.n_red[sid];
+  if (16 * u.unit >= n || p.info[sid] != 0) return;
+  const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lk = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ld = p.ldz;
+  const cplx<double>* A = p.z_out + (size_t)sid * p.stride_z;
+  const double* Z = p.ws_z + (size_t)u.job * p.ws_stride;
+  cplx<double>* X = p.ws_a + (size_t)u.job * p.ws_stride;
+  const int col = 16 * u.unit + lr;
+  const int pc = col < n ? tw.perm[(size_t)u.job * p.nmax + col] : 0;
+  const f64x4 z4 = {0, 0, 0, 0};
+  f64x4 xr[RBW], xi[RBW];  // row block wave + 4 t, register r: row lk + 4 r
+#pragma unroll
+  for (int t = 0; t < RBW; ++t) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = (wave + NWV * t) * 16 + lk + 4 * r;
+      xr[t][r] = row < n && col < n ? Z[row + (size_t)pc * ld] : 0.0;
+    }
+    xi[t] = z4;
+  }
+  const int nblk = (n - 1 + 15) / 16;
+  for (int b = 0; b < nblk; ++b) {
+    const int cs = n - 2 - 16 * b - 15, rb0 = (max(cs, 0) + 1) / 16;
+    f64x4 wr = z4, wi = z4;
+#pragma unroll
+    for (int t = 0; t < RBW; ++t) {
+      const int rb = wave + NWV * t;
+      if (rb < rb0 || 16 * rb >= n) continue;  // uniform over the wavefront
+      cplx<double> v[4];
+#pragma unroll
+      for (int s4 = 0; s4 < 4; ++s4) v[s4] = wy_elem(A, ld, n, cs + lr, rb * 16 + 4 * s4 + lk);
+#pragma unroll
+      for (int s4 = 0; s4 < 4; ++s4) {
+        wr = __builtin_amdgcn_mfma_f64_16x16x4f64(v[s4].re, xr[t][s4], wr, 0, 0, 0);
+        wi = __builtin_amdgcn_mfma_f64_16x16x4f64(v[s4].re, xi[t][s4], wi, 0, 0, 0);
+        wr = __builtin_amdgcn_mfma_f64_16x16x4f64(v[s4].im, xi[t][s4], wr, 0, 0, 0);
+        wi = __builtin_amdgcn_mfma_f64_16x16x4f64(-v[s4].im, xr[t][s4], wi, 0, 0, 0);
+      }
+    }
+    cplx<double> tv[4];
+#pragma unroll
+    for (int s4 = 0; s4 < 4; ++s4) {
+      const int q = 4 * s4 + lk;
+      tv[s4] = lr <= q && cs + lr >= 0 ? A[(cs + lr) + (size_t)(cs + q + 1) * ld] : mk<double>(0, 0);
+    }
+    double(*rd)[64][8] = red[b & 1];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      rd[wave][lane][r] = wr[r];
+      rd[wave][lane][4 + r] = wi[r];
+    }
+    // one barrier per block: the other buffer is next written after the next barrier
+    __syncthreads();
+    f64x4 w1r, w1i, w2r = z4, w2i = z4;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      w1r[r] = (rd[0][lane][r] + rd[1][lane][r]) + (rd[2][lane][r] + rd[3][lane][r]);
+      w1i[r] = (rd[0][lane][4 + r] + rd[1][lane][4 + r]) + (rd[2][lane][4 + r] + rd[3][lane][4 + r]);
+    }
+#pragma unroll
+    for (int s4 = 0; s4 < 4; ++s4) {
+      w2r = __builtin_amdgcn_mfma_f64_16x16x4f64(tv[s4].re, w1r[s4], w2r, 0, 0, 0);
+      w2i = __builtin_amdgcn_mfma_f64_16x16x4f64(tv[s4].re, w1i[s4], w2i, 0, 0, 0);
+      w2r = __builtin_amdgcn_mfma_f64_16x16x4f64(-tv[s4].im, w1i[s4], w2r, 0, 0, 0);
+      w2i = __builtin_amdgcn_mfma_f64_16x16x4f64(tv[s4].im, w1r[s4], w2i, 0, 0, 0);
+    }
+#pragma unroll
+    for (int t = 0; t < RBW; ++t) {
+      const int rb = wave + NWV * t;
+      if (rb < rb0 || 16 * rb >= n) continue;  // uniform over the wavefront
+      cplx<double> v[4];
+#pragma unroll
+      for (int s4 = 0; s4 < 4; ++s4) v[s4] = wy_elem(A, ld, n, cs + 4 * s4 + lk, rb * 16 + lr);
+#pragma unroll
+      for (int s4 = 0; s4 < 4; ++s4) {
+        xr[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(-v[s4].re, w2r[s4], xr[t], 0, 0, 0);
+        xi[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(-v[s4].re, w2i[s4], xi[t], 0, 0, 0);
+        xr[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(v[s4].im, w2i[s4], xr[t], 0, 0, 0);
+        xi[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(-v[s4].im, w2r[s4], xi[t], 0, 0, 0);
+      }
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < RBW; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = (wave + NWV * t) * 16 + lk + 4 * r;
+      if (row < n && col < n) X[row + (size_t)col * ld] = mk<double>(xr[t][r], xi[t][r]);
+    }
+}

@@ -23,6 +23,7 @@
 #include "chol_inv.hpp"
 #include "tridiag_dc.hpp"
 
+#include <algorithm>
 #include <limits>
 #include <type_traits>
 
@@ -986,6 +987,25 @@ __device__ __noinline__ void back_transform_mfma(int n, cplx<double>* A_, int ld
   __syncthreads();
 }
 
+// Rank sort of the eigenvalues sh.de[i].x: sh.perm[k] is the index of the k-th smallest (NaN
+// ordered as +inf, ties by index: the ranks always form a permutation of [0, n)).  Ends with
+// a barrier.
+template <typename R, int NMAX>
+__device__ __forceinline__ void rank_order(int n, EigShared<R, NMAX>& sh) {
+  for (int i = threadIdx.x; i < n; i += EigCfg<NMAX>::NT) {
+    const R di0 = sh.de[i].x;
+    const R di = di0 == di0 ? di0 : std::numeric_limits<R>::infinity();
+    int rank = 0;
+    for (int j = 0; j < n; ++j) {
+      const R dj0 = sh.de[j].x;
+      const R dj = dj0 == dj0 ? dj0 : std::numeric_limits<R>::infinity();
+      rank += (dj < di) || (dj == di && j < i);
+    }
+    sh.perm[rank] = i;
+  }
+  __syncthreads();
+}
+
 template <typename R, typename TIn, int NMAX>
 __device__ void solve_one(const EigParams<R>& p, int sid, EigShared<R, NMAX>& sh) {
   constexpr int NT_ = EigCfg<NMAX>::NT, NW_ = EigCfg<NMAX>::NW, RM = EigCfg<NMAX>::RM,
@@ -1110,20 +1130,8 @@ __device__ void solve_one(const EigParams<R>& p, int sid, EigShared<R, NMAX>& sh
                     p.prof ? p.prof + (size_t)sid * EIG_PROF_SLOTS + 8 : nullptr);
   eig_mark(p, sid, 5);
 
-  // ---- ascending order: rank sort --------------------------------------------------
-  // (NaN ordered as +inf, ties by index: the ranks always form a permutation of [0, n))
-  for (int i = tid; i < n; i += NT_) {
-    const R di0 = sh.de[i].x;
-    const R di = di0 == di0 ? di0 : std::numeric_limits<R>::infinity();
-    int rank = 0;
-    for (int j = 0; j < n; ++j) {
-      const R dj0 = sh.de[j].x;
-      const R dj = dj0 == dj0 ? dj0 : std::numeric_limits<R>::infinity();
-      rank += (dj < di) || (dj == di && j < i);
-    }
-    sh.perm[rank] = i;
-  }
-  __syncthreads();
+  // ---- ascending order ----------------------------------------------------------------
+  rank_order<R, NMAX>(n, sh);
   for (int j = tid; j < nmax; j += NT_) dout[j] = j < n ? sh.de[sh.perm[j]].x : R(0);
 
   // ---- back-transform X = Q Z[:, perm] ------------------------------------------------
@@ -1290,6 +1298,8 @@ __global__ __launch_bounds__(EigCfg<NMAX>::NT) void eig_kernel(EigParams<R> p) {
   }
 }
 
+#include "eig_split.hpp"
+
 // --------------------------------------------------------------------------------------
 // Flag live entries and compact kept beams (src/eigensolver.cpp:145-168).
 // One workgroup per sample.
@@ -1421,6 +1431,76 @@ void launch_eig(const EigParams<R>& p, int n_slots, bool in_double, hipStream_t 
   BIPP_EIG_CASE(512)
 #undef BIPP_EIG_CASE
   check_launch("eig_kernel");
+}
+
+int eig_split_groups(int n_jobs, int n_cu) {
+  // workgroups per sample of a column launch: one per CU over all samples; at most eight,
+  // since every workgroup reads the row sums of all of them (G^2 vectors per sample)
+  return std::max(1, std::min(TRI_GMAX, n_cu / std::max(1, n_jobs)));
+}
+
+EigSplitSizes eig_split_sizes(int n_jobs, int nmax) {
+  EigSplitSizes z;
+  const size_t jn = (size_t)n_jobs * nmax;
+  z.cplx_elems = jn * (2 + 2 + 2 * TRI_GMAX) + 2 * (size_t)n_jobs;
+  z.real_elems = 2 * jn;
+  z.int_elems = jn;
+  return z;
+}
+
+void launch_eig_split(const EigParams<double>& p, const EigSplitBuffers& b, int n_max, int n_cu,
+                      bool in_double, hipStream_t stream) {
+  if (p.n_jobs <= 0) return;
+  if (eig_nmax_bucket<double>(p.nmax) != 512 || p.n_jobs > 65535 || n_max > p.nmax || !p.order ||
+      p.standard || p.ldz != p.ws_ld || p.stride_z != p.ws_stride)
+    fail(BIPP_INTERNAL_ERROR, "phase-split eigensolve arguments");
+  const int jobs = p.n_jobs;
+  const size_t jn = (size_t)jobs * p.nmax;
+  TriWork tw;
+  tw.v = b.cplx_buf;
+  tw.col = tw.v + 2 * jn;
+  tw.row = tw.col + 2 * jn;
+  tw.tau = tw.row + 2 * TRI_GMAX * jn;
+  tw.de = b.real_buf;
+  tw.perm = b.int_buf;
+  constexpr int NM = 512;
+  if (n_max > 0) {
+    const dim3 lg(ceil_div(n_max, 16), jobs);
+    if (in_double)
+      split_load_kernel<double><<<lg, 256, 0, stream>>>(p);
+    else
+      split_load_kernel<float><<<lg, 256, 0, stream>>>(p);
+    check_launch("split_load_kernel");
+  }
+  split_chol_kernel<NM><<<jobs, EigCfg<NM>::NT, 0, stream>>>(p);
+  check_launch("split_chol_kernel");
+  if (n_max <= 0) return;
+  const int side = ceil_div(n_max, 64);
+  split_gemm_kernel<0><<<split_grid(side * side, jobs), 256, 0, stream>>>(p, side);
+  check_launch("split_gemm_kernel");
+  split_gemm_kernel<1><<<split_grid(side * (side + 1) / 2, jobs), 256, 0, stream>>>(p, side);
+  check_launch("split_gemm_kernel");
+  const int G = eig_split_groups(jobs, n_cu);
+  for (int c = 0; c < n_max; ++c) {
+    // column tiles of a wavefront taken together: a sample's up to 128 tiles over its 8 G
+    // wavefronts are two each for G = 8
+    if (G >= 4)
+      tri_column_kernel<2><<<dim3(G, jobs), TRI_NT, 0, stream>>>(p, tw, c);
+    else
+      tri_column_kernel<4><<<dim3(G, jobs), TRI_NT, 0, stream>>>(p, tw, c);
+  }
+  check_launch("tri_column_kernel");
+  split_dc_kernel<NM><<<jobs, EigCfg<NM>::NT, 0, stream>>>(p, tw);
+  check_launch("split_dc_kernel");
+  if (n_max > 1) {
+    split_tfac_kernel<<<dim3((n_max + 14) / 16, jobs), 256, 0, stream>>>(p);
+    check_launch("split_tfac_kernel");
+  }
+  const int groups = ceil_div(n_max, 16);
+  split_bt_kernel<NM><<<split_grid(groups, jobs), 256, 0, stream>>>(p, tw, groups);
+  check_launch("split_bt_kernel");
+  split_gemm_kernel<2><<<split_grid(side * side, jobs), 256, 0, stream>>>(p, side);
+  check_launch("split_gemm_kernel");
 }
 
 template <typename R>
