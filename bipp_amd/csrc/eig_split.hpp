@@ -202,7 +202,8 @@ __global__ __launch_bounds__(256) void split_gemm_kernel(EigParams<double> p, in
 // of a wavefront stay in registers.  Column tiles of 4 are dealt to the sample's wavefronts in
 // turn, which keeps them balanced while the trailing matrix shrinks.
 // --------------------------------------------------------------------------------------
-constexpr int TRI_NT = 512, TRI_NW = TRI_NT / 64, TRI_GMAX = 8;
+constexpr int TRI_N = 512;   // largest reduced size
+constexpr int TRI_GMAX = 8;  // workgroups per sample of a launch
 
 struct TriWork {
   cplx<double>* v;     // [job][2][nmax]
@@ -213,10 +214,11 @@ struct TriWork {
   int* perm;           // [job][nmax]
 };
 
+template <int NW>
 struct TriShared {
-  cplx<double> v[TRI_NT], w[TRI_NT], vn[TRI_NT];
-  cplx<double> xw[TRI_NW][TRI_NT];  // a wavefront's row sums
-  double red[2][2 * TRI_NW];
+  cplx<double> v[TRI_N], w[TRI_N], vn[TRI_N];
+  cplx<double> xw[NW][TRI_N];  // a wavefront's row sums
+  double red[2][2 * NW];
   cplx<double> yc, alpha;
 };
 
@@ -244,28 +246,30 @@ __device__ __forceinline__ double rows_total(double re, double im) {
 }
 
 // sums of a and b over the workgroup in a fixed order; one barrier (slots alternate)
+template <int NW>
 __device__ __forceinline__ void tri_sum2(double& a, double& b, double* red) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   a = wave_total(a);
   b = wave_total(b);
   if (lane == 0) {
     red[wave] = a;
-    red[TRI_NW + wave] = b;
+    red[NW + wave] = b;
   }
   __syncthreads();
   a = 0;
   b = 0;
 #pragma unroll
-  for (int w = 0; w < TRI_NW; ++w) {
+  for (int w = 0; w < NW; ++w) {
     a += red[w];
-    b += red[TRI_NW + w];
+    b += red[NW + w];
   }
 }
 
 // NCT: column tiles of a wavefront taken together (a tile's row operands are read once)
-template <int NCT>
-__global__ __launch_bounds__(TRI_NT) void tri_column_kernel(EigParams<double> p, TriWork tw, int c) {
-  __shared__ TriShared sh;
+template <int NT, int NCT>
+__global__ __launch_bounds__(NT) void tri_column_kernel(EigParams<double> p, TriWork tw, int c) {
+  constexpr int NW = NT / 64, RPT = TRI_N / NT;
+  __shared__ TriShared<NW> sh;
   const int job = blockIdx.y, g = blockIdx.x, G = gridDim.x;
   const int sid = p.order[job], n = p.n_red[sid];
   if (c >= n || p.info[sid] != 0 || (c == n - 1 && g != 0)) return;  // uniform
@@ -277,47 +281,103 @@ __global__ __launch_bounds__(TRI_NT) void tri_column_kernel(EigParams<double> p,
   const size_t j2 = (size_t)job * 2;
   const bool apply = c > 0;
 
-  // ---- w_{c-1}, column c, its reflector; thread i holds row i ----------------------------
-  const int i = tid;
-  const bool live = i >= c && i < n;
-  cplx<double> a = mk<double>(0, 0), v = a, y = a, w = a, tau = a;
-  if (live) {
-    a = A[i + (size_t)c * ld];
-    if (apply) {
-      v = tw.v[(j2 + prv) * nmax + i];
-      y = tw.col[(j2 + prv) * nmax + i];
-      for (int q = 0; q < G; ++q) y = y + tw.row[((j2 + prv) * TRI_GMAX + q) * nmax + i];
+  const int i0 = c + 1;
+  const int lr = lane & 15, lc = lane >> 4;
+  const int W = G * NW, gw = g * NW + wave;
+  const int ct_end = (n + 3) >> 2, rt_end = (n + 15) >> 4;
+  constexpr int RU = 8 / NCT;  // row tiles loaded together: eight elements in flight per lane
+  int ct = i0 >> 2;
+  ct += (gw - ct % W + W) % W;  // first tile at or after column i0 that is this wavefront's
+  int jc[NCT];
+  auto tiles = [&]() {
+#pragma unroll
+    for (int u = 0; u < NCT; ++u) {
+      const int j = 4 * (ct + u * W) + lc;
+      jc[u] = j >= i0 && j < n ? j : n;  // n: no such column (every row test fails)
+    }
+  };
+  cplx<double> x[RU][NCT], xn[RU][NCT];
+  auto load = [&](int rt, cplx<double>(&o)[RU][NCT]) {
+#pragma unroll
+    for (int k = 0; k < RU; ++k)
+#pragma unroll
+      for (int u = 0; u < NCT; ++u) {
+        const int r = 16 * (rt + k) + lr;
+        o[k][u] = mk<double>(0, 0);
+        if (r < n && r >= jc[u]) o[k][u] = A[r + (size_t)jc[u] * ld];
+      }
+  };
+  // the first elements of the pass are in flight during the prologue
+  tiles();
+  load(ct >> 2, x);
+
+  // ---- w_{c-1}, column c, its reflector; a thread holds rows tid + NT q ----------------
+  cplx<double> a[RPT], v[RPT], y[RPT], tau = mk<double>(0, 0);
+  bool live[RPT];
+#pragma unroll
+  for (int q = 0; q < RPT; ++q) {
+    const int i = tid + NT * q;
+    live[q] = i >= c && i < n;
+    a[q] = v[q] = y[q] = mk<double>(0, 0);
+    if (live[q]) {
+      a[q] = A[i + (size_t)c * ld];
+      if (apply) {
+        v[q] = tw.v[(j2 + prv) * nmax + i];
+        y[q] = tw.col[(j2 + prv) * nmax + i];
+        for (int k = 0; k < G; ++k) y[q] = y[q] + tw.row[((j2 + prv) * TRI_GMAX + k) * nmax + i];
+      }
+      if (i == c) sh.yc = y[q];
     }
   }
+  cplx<double> w[RPT];
+#pragma unroll
+  for (int q = 0; q < RPT; ++q) w[q] = mk<double>(0, 0);
   if (apply) {
     tau = tw.tau[j2 + prv];
-    if (i == c) sh.yc = y;
-    const cplx<double> x = tau * y;
-    const cplx<double> dt = cmul_conj_a(x, v);
-    double pr = dt.re, pi = dt.im;
-    tri_sum2(pr, pi, sh.red[0]);
-    const cplx<double> alpha2 = tau * mk<double>(-0.5 * pr, -0.5 * pi);
-    w = x + alpha2 * v;
-    const cplx<double> wc = tau * sh.yc + alpha2;  // row c, where v is 1
-    if (live) a = a - (v * conj(wc) + w);
-  }
-  sh.v[i] = v;
-  sh.w[i] = w;
-  if (i == c + 1) sh.alpha = a;
-  double part = live && i >= c + 2 ? abs2(a) : 0.0, unused = 0;
-  tri_sum2(part, unused, sh.red[1]);
-  if (g == 0 && live) {
-    if (apply) {
-      if (i > c)
-        A[i + (size_t)(c - 1) * ld] = v;
-      else
-        A[(c - 1) + (size_t)(c - 1) * ld] = tau;  // the diagonal slot keeps tau
+    double pr = 0, pi = 0;
+#pragma unroll
+    for (int q = 0; q < RPT; ++q) {
+      w[q] = tau * y[q];
+      const cplx<double> dt = cmul_conj_a(w[q], v[q]);
+      pr += dt.re;
+      pi += dt.im;
     }
-    if (i == c) {
-      tw.de[((size_t)job * nmax + c) * 2] = a.re;
-      if (c == n - 1) {
-        tw.de[((size_t)job * nmax + c) * 2 + 1] = 0;
-        A[c + (size_t)c * ld] = mk<double>(0, 0);  // no reflector for the last column
+    tri_sum2<NW>(pr, pi, sh.red[0]);
+    const cplx<double> alpha2 = tau * mk<double>(-0.5 * pr, -0.5 * pi);
+    const cplx<double> wc = tau * sh.yc + alpha2;  // row c, where v is 1
+#pragma unroll
+    for (int q = 0; q < RPT; ++q) {
+      w[q] = w[q] + alpha2 * v[q];
+      if (live[q]) a[q] = a[q] - (v[q] * conj(wc) + w[q]);
+    }
+  }
+  double part = 0, unused = 0;
+#pragma unroll
+  for (int q = 0; q < RPT; ++q) {
+    const int i = tid + NT * q;
+    sh.v[i] = v[q];
+    sh.w[i] = w[q];
+    if (i == c + 1) sh.alpha = a[q];
+    if (live[q] && i >= c + 2) part += abs2(a[q]);
+  }
+  tri_sum2<NW>(part, unused, sh.red[1]);
+  if (g == 0) {
+#pragma unroll
+    for (int q = 0; q < RPT; ++q) {
+      const int i = tid + NT * q;
+      if (!live[q]) continue;
+      if (apply) {
+        if (i > c)
+          A[i + (size_t)(c - 1) * ld] = v[q];
+        else
+          A[(c - 1) + (size_t)(c - 1) * ld] = tau;  // the diagonal slot keeps tau
+      }
+      if (i == c) {
+        tw.de[((size_t)job * nmax + c) * 2] = a[q].re;
+        if (c == n - 1) {
+          tw.de[((size_t)job * nmax + c) * 2 + 1] = 0;
+          A[c + (size_t)c * ld] = mk<double>(0, 0);  // no reflector for the last column
+        }
       }
     }
   }
@@ -335,57 +395,46 @@ __global__ __launch_bounds__(TRI_NT) void tri_column_kernel(EigParams<double> p,
     tn = mk<double>((beta - alpha.re) / beta, -alpha.im / beta);
     scal = crecip(mk<double>(alpha.re - beta, alpha.im));
   }
-  const cplx<double> vn = i == c + 1 ? mk<double>(1, 0) : (live && i >= c + 2 ? a * scal : mk<double>(0, 0));
-  sh.vn[i] = vn;
-  if (g == 0) {
-    if (live && i > c) tw.v[(j2 + cur) * nmax + i] = vn;
-    if (i == c) {
-      tw.tau[j2 + cur] = tn;
-      tw.de[((size_t)job * nmax + c) * 2 + 1] = beta;
+#pragma unroll
+  for (int q = 0; q < RPT; ++q) {
+    const int i = tid + NT * q;
+    cplx<double> vn = mk<double>(i == c + 1 ? 1.0 : 0.0, 0);
+    if (live[q] && i >= c + 2) vn = a[q] * scal;
+    sh.vn[i] = vn;
+    if (g == 0) {
+      if (live[q] && i > c) tw.v[(j2 + cur) * nmax + i] = vn;
+      if (i == c) {
+        tw.tau[j2 + cur] = tn;
+        tw.de[((size_t)job * nmax + c) * 2 + 1] = beta;
+      }
     }
   }
   // ---- pass over this wavefront's column tiles ------------------------------------------
-  const int i0 = c + 1;
   for (int r = (i0 & ~63) + lane; r < n; r += 64) sh.xw[wave][r] = mk<double>(0, 0);
   __syncthreads();
-  const int lr = lane & 15, lc = lane >> 4;
-  const int W = G * TRI_NW, gw = g * TRI_NW + wave;
-  const int ct_end = (n + 3) >> 2, rt_end = (n + 15) >> 4;
-  int ct = i0 >> 2;
-  ct += (gw - ct % W + W) % W;  // first tile at or after column i0 that is this wavefront's
-  constexpr int RU = 8 / NCT;   // row tiles loaded together: eight elements in flight per lane
+  bool first = true;
   for (; ct < ct_end; ct += NCT * W) {
-    int jc[NCT];
+    if (!first) {
+      tiles();
+      load(ct >> 2, x);
+    }
+    first = false;
     cplx<double> cv[NCT], cw[NCT], cn[NCT], cs[NCT];
 #pragma unroll
     for (int u = 0; u < NCT; ++u) {
-      const int j = 4 * (ct + u * W) + lc;
-      jc[u] = j >= i0 && j < n ? j : n;  // n: no such column (every row test fails)
-      const int jj = min(jc[u], TRI_NT - 1);
+      const int jj = min(jc[u], TRI_N - 1);
       cv[u] = conj(sh.v[jj]);
       cw[u] = conj(sh.w[jj]);
       cn[u] = sh.vn[jj];
       cs[u] = mk<double>(0, 0);
     }
-    cplx<double> x[RU][NCT], xn[RU][NCT];
-    auto load = [&](int rt, cplx<double>(&o)[RU][NCT]) {
-#pragma unroll
-      for (int k = 0; k < RU; ++k)
-#pragma unroll
-        for (int u = 0; u < NCT; ++u) {
-          const int r = 16 * (rt + k) + lr;
-          o[k][u] = r < n && r >= jc[u] ? A[r + (size_t)jc[u] * ld] : mk<double>(0, 0);
-        }
-    };
-    const int rt0 = ct >> 2;
-    load(rt0, x);
-    for (int rt = rt0; rt < rt_end; rt += RU) {
+    for (int rt = ct >> 2; rt < rt_end; rt += RU) {
       if (rt + RU < rt_end) load(rt + RU, xn);
 #pragma unroll
       for (int k = 0; k < RU; ++k) {
         const int r = 16 * (rt + k) + lr;
         if (16 * (rt + k) >= n) break;  // uniform
-        const int rr = min(r, TRI_NT - 1);
+        const int rr = min(r, TRI_N - 1);
         const cplx<double> vi = sh.v[rr], wi = sh.w[rr], ni = sh.vn[rr];
         cplx<double> acc = mk<double>(0, 0);
 #pragma unroll
@@ -418,10 +467,13 @@ __global__ __launch_bounds__(TRI_NT) void tri_column_kernel(EigParams<double> p,
     }
   }
   __syncthreads();
-  if (i >= i0 && i < n) {
+#pragma unroll
+  for (int q = 0; q < RPT; ++q) {
+    const int i = tid + NT * q;
+    if (i < i0 || i >= n) continue;
     cplx<double> s = sh.xw[0][i];
 #pragma unroll
-    for (int q = 1; q < TRI_NW; ++q) s = s + sh.xw[q][i];
+    for (int k = 1; k < NW; ++k) s = s + sh.xw[k][i];
     tw.row[((j2 + cur) * TRI_GMAX + g) * nmax + i] = s;
   }
 }

@@ -1433,12 +1433,6 @@ void launch_eig(const EigParams<R>& p, int n_slots, bool in_double, hipStream_t 
   check_launch("eig_kernel");
 }
 
-int eig_split_groups(int n_jobs, int n_cu) {
-  // workgroups per sample of a column launch: one per CU over all samples; at most eight,
-  // since every workgroup reads the row sums of all of them (G^2 vectors per sample)
-  return std::max(1, std::min(TRI_GMAX, n_cu / std::max(1, n_jobs)));
-}
-
 EigSplitSizes eig_split_sizes(int n_jobs, int nmax) {
   EigSplitSizes z;
   const size_t jn = (size_t)n_jobs * nmax;
@@ -1480,14 +1474,18 @@ void launch_eig_split(const EigParams<double>& p, const EigSplitBuffers& b, int 
   check_launch("split_gemm_kernel");
   split_gemm_kernel<1><<<split_grid(side * (side + 1) / 2, jobs), 256, 0, stream>>>(p, side);
   check_launch("split_gemm_kernel");
-  const int G = eig_split_groups(jobs, n_cu);
+  // Column launches: one 512-thread workgroup per CU over all samples while that gives a sample
+  // at least four (at most eight: every workgroup reads the row sums of all of them, G^2
+  // vectors per sample), else two 256-thread ones per CU, whose prologues and passes overlap.
+  // Whole batch of 400..512 beams: 12 samples 15.7 ms (17.0 with 256 threads), 32 samples 20.0
+  // (20.8), 96 samples 32.5 against 30.9 with 256 threads.
+  const bool wide = n_cu / jobs >= 4;
+  const int G = std::max(1, std::min(TRI_GMAX, (wide ? n_cu : 2 * n_cu) / jobs));
   for (int c = 0; c < n_max; ++c) {
-    // column tiles of a wavefront taken together: a sample's up to 128 tiles over its 8 G
-    // wavefronts are two each for G = 8
-    if (G >= 4)
-      tri_column_kernel<2><<<dim3(G, jobs), TRI_NT, 0, stream>>>(p, tw, c);
+    if (wide)
+      tri_column_kernel<512, 2><<<dim3(G, jobs), 512, 0, stream>>>(p, tw, c);
     else
-      tri_column_kernel<4><<<dim3(G, jobs), TRI_NT, 0, stream>>>(p, tw, c);
+      tri_column_kernel<256, 2><<<dim3(G, jobs), 256, 0, stream>>>(p, tw, c);
   }
   check_launch("tri_column_kernel");
   split_dc_kernel<NM><<<jobs, EigCfg<NM>::NT, 0, stream>>>(p, tw);
