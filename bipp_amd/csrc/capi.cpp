@@ -36,7 +36,7 @@ struct BippSynthesisImpl {
   // steering buffers
   DevBuf n_eig, n_ant_used, pos, afrag, wts;
   // direct-sum buffers
-  DevBuf wdense, vfull, vv, vv32, uvw;
+  DevBuf wdense, vfull, vv, uvw;
   // type-3 NUFFT state
   N3Options n3opt;
   double pix_lo[3] = {0, 0, 0}, pix_hi[3] = {0, 0, 0};
@@ -172,8 +172,9 @@ struct BippSynthesisImpl {
       sp.img_ld = n_pix;
       launch_steer(sp, mode, st);
       BIPP_HIP(hipEventRecord(ev[3], st));
-    } else if (imager == 2) {
-      // virtual visibilities + type-3 NUFFT over all samples and levels of the batch
+    } else if (imager == 2 || compute != BIPP_COMPUTE_FP32) {
+      // virtual visibilities + type-3 NUFFT or direct sum over all samples and levels of the
+      // batch
       R* wd = wdense.as<R>((size_t)nS * n_levels * n_beam);
       launch_level_weights<R>(nS, n_levels, filter, d_int, er.d_n_red(), er.d_d(), n_beam, n_beam,
                               er.d_n_vis(), wd, (long long)n_levels * n_beam, st);
@@ -224,7 +225,14 @@ struct BippSynthesisImpl {
       src.pos_stride = pp.pos_stride;
       src.apad = apad;
       const double* l64 = static_cast<const double*>(lmn64.p);
-      if (compute == BIPP_COMPUTE_FP64) {
+      if (imager == 1) {
+        if (compute == BIPP_COMPUTE_FP64)
+          n3d.direct<R>(c, src, nS, n_levels, n_beam, pp.z, pp.stride_z, pp.ldz, wd, l64, n_pix,
+                        static_cast<double*>(img.p));
+        else
+          n3f.direct<R>(c, src, nS, n_levels, n_beam, pp.z, pp.stride_z, pp.ldz, wd, l64, n_pix,
+                        static_cast<float*>(img.p));
+      } else if (compute == BIPP_COMPUTE_FP64) {
         n3d.values<R>(c, nS, n_levels, n_beam, rows_max, pp.n_ant, pp.z, pp.stride_z, pp.ldz, wd);
         n3d.image(c, src, nS, n_levels, n3opt, pix_lo, pix_hi, l64, n_pix, img.p, false);
       } else {
@@ -232,10 +240,10 @@ struct BippSynthesisImpl {
         n3f.image(c, src, nS, n_levels, n3opt, pix_lo, pix_hi, l64, n_pix, img.p,
                   compute == BIPP_COMPUTE_FP32);
       }
-      n3_timed = true;
+      n3_timed = imager == 2;
       BIPP_HIP(hipEventRecord(ev[3], st));
-    } else {
-      // virtual visibilities + direct NUFT sum, per sample and level
+    } else if constexpr (sizeof(R) == 4) {
+      // float32 form: virtual visibilities + direct NUFT sum, per sample and level
       R* wd = wdense.as<R>((size_t)nS * n_levels * n_beam);
       launch_level_weights<R>(nS, n_levels, filter, d_int, er.d_n_red(), er.d_d(), n_beam, n_beam,
                               er.d_n_vis(), wd, (long long)n_levels * n_beam, st);
@@ -263,29 +271,17 @@ struct BippSynthesisImpl {
       std::vector<double> h_wl(nS);
       BIPP_HIP(hipMemcpyAsync(h_wl.data(), wl, sizeof(double) * nS, hipMemcpyDeviceToHost, st));
       BIPP_HIP(hipStreamSynchronize(st));
-      const bool mixed = compute == BIPP_COMPUTE_MIXED;
       for (int k = 0; k < nS; ++k) {
         const double uvw_scale = 2.0 * 3.14159265358979323846 / h_wl[k];
         const double* xk = xyz + (size_t)k * stride_xyz;
         for (int lv = 0; lv < n_levels; ++lv) {
           launch_virtual_vis<R>(1, n_ant, n_beam, vf + (size_t)k * n_ant * n_beam, n_ant, 0,
                                 wd + ((size_t)k * n_levels + lv) * n_beam, 0, vvb, 0, st);
-          if (mixed) {
-            double* u = uvw.as<double>(3 * (size_t)nn);
-            launch_baselines<double>(n_ant, xk, ldxyz, uvw_scale, u, u + nn, u + 2 * nn, st);
-            cplx<float>* v32 = vv32.as<cplx<float>>((size_t)nn);
-            launch_copy_cast<R, float>(1, (int)nn, 1, vvb, nn, 0, v32, nn, 0, st);
-            const double* l = static_cast<const double*>(lmn64.p);
-            launch_nuft_sum_mixed(1.0, (int)nn, v32, u, u + nn, u + 2 * nn, n_pix, l, l + n_pix,
-                                  l + 2 * (size_t)n_pix, static_cast<float*>(img.p) + (size_t)lv * n_pix,
-                                  st);
-          } else {
-            R* u = uvw.as<R>(3 * (size_t)nn);
-            launch_baselines<R>(n_ant, xk, ldxyz, uvw_scale, u, u + nn, u + 2 * nn, st);
-            const R* l = sizeof(R) == 8 ? static_cast<const R*>(lmn64.p) : static_cast<const R*>(lmn32.p);
-            launch_nuft_sum<R>(R(1), (int)nn, vvb, u, u + nn, u + 2 * nn, n_pix, l, l + n_pix,
-                               l + 2 * (size_t)n_pix, static_cast<R*>(img.p) + (size_t)lv * n_pix, st);
-          }
+          R* u = uvw.as<R>(3 * (size_t)nn);
+          launch_baselines<R>(n_ant, xk, ldxyz, uvw_scale, u, u + nn, u + 2 * nn, st);
+          const R* l = static_cast<const R*>(lmn32.p);
+          launch_nuft_sum<R>(R(1), (int)nn, vvb, u, u + nn, u + 2 * nn, n_pix, l, l + n_pix,
+                             l + 2 * (size_t)n_pix, static_cast<R*>(img.p) + (size_t)lv * n_pix, st);
         }
       }
       BIPP_HIP(hipEventRecord(ev[3], st));

@@ -37,7 +37,7 @@ struct BippImagerImpl {
   double pix_lo[3] = {0, 0, 0}, pix_hi[3] = {0, 0, 0};
   PinnedBuf h_uvw, h_v, h_d, h_sc, h_wl;
   DevBuf d_uvw, d_v, d_d, d_sc, d_wl, v_r, w_r, uvw_scale, antisym, lmn64, lmn32, img;
-  DevBuf vv, vv32, uvw_r;
+  DevBuf vv, uvw_r;
   N3Runner<float> n3f;
   N3Runner<double> n3d;
 
@@ -131,46 +131,45 @@ struct BippImagerImpl {
     pp.uvw_scale = uvw_scale.as<double>(nS);
     launch_eigpair_prep<R>(pp, nS, st);
     const double* l64 = static_cast<const double*>(lmn64.p);
-    if (imager == 2) {
-      n3.template values<R>(c, nS, n_img, n_beam, n_ant, nullptr, pp.v_out,
-                            (long long)n_ant * n_beam, n_ant, pp.w_out);
-      N3Source src;
-      src.mode = N3_SRC_UVW;
-      src.n_ant_max = n_ant;
-      src.n_rows_const = n_ant;
-      src.uvw = du;
-      src.uvw_stride = 3LL * nn();
-      src.lduvw = (long long)nn();
-      src.uvw_scale = pp.uvw_scale;
+    N3Source src;
+    src.mode = N3_SRC_UVW;
+    src.n_ant_max = n_ant;
+    src.n_rows_const = n_ant;
+    src.uvw = du;
+    src.uvw_stride = 3LL * nn();
+    src.lduvw = (long long)nn();
+    src.uvw_scale = pp.uvw_scale;
+    if (imager == 2 || compute != BIPP_COMPUTE_FP32) {
       unsigned char* anti = antisym.as<unsigned char>(nS);
       src.antisym = anti;
       launch_uvw_antisym(src, nS, anti, st);
+    }
+    if (imager == 2) {
+      n3.template values<R>(c, nS, n_img, n_beam, n_ant, nullptr, pp.v_out,
+                            (long long)n_ant * n_beam, n_ant, pp.w_out);
       n3.image(c, src, nS, n_img, opt, pix_lo, pix_hi, l64, n_pix, img.p,
                compute == BIPP_COMPUTE_FP32);
       return;
     }
-    // direct sum per (sample, image) of the reference's arithmetic (src/host/kernels/nuft_sum.cpp)
-    const long long n2 = (long long)nn();
-    cplx<R>* vvb = vv.as<cplx<R>>(n2);
-    for (int k = 0; k < nS; ++k) {
-      const double sc = 2.0 * 3.14159265358979323846 / static_cast<double>(hwl[k]);
-      const float* uk = du + (size_t)k * 3 * n2;
-      for (int l = 0; l < n_img; ++l) {
-        launch_virtual_vis<R>(1, n_ant, n_beam, pp.v_out + (size_t)k * n_ant * n_beam, n_ant, 0,
-                              pp.w_out + ((size_t)k * n_img + l) * n_beam, 0, vvb, 0, st);
-        if (compute == BIPP_COMPUTE_MIXED) {
-          double* u = uvw_r.as<double>(3 * n2);
-          launch_scale_uvw<double>(n2, uk, n2, sc, u, u + n2, u + 2 * n2, st);
-          cplx<float>* v32 = vv32.as<cplx<float>>(n2);
-          launch_copy_cast<R, float>(1, (int)n2, 1, vvb, n2, 0, v32, n2, 0, st);
-          launch_nuft_sum_mixed(1.0, (int)n2, v32, u, u + n2, u + 2 * n2, n_pix, l64, l64 + n_pix,
-                                l64 + 2 * (size_t)n_pix,
-                                static_cast<float*>(img.p) + (size_t)l * n_pix, st);
-        } else {
-          R* u = uvw_r.as<R>(3 * n2);
+    if (compute != BIPP_COMPUTE_FP32) {
+      n3.template direct<R>(c, src, nS, n_img, n_beam, pp.v_out, (long long)n_ant * n_beam, n_ant,
+                            pp.w_out, l64, n_pix, static_cast<TG*>(img.p));
+      return;
+    }
+    // float32 direct sum per (sample, image) of the reference's arithmetic, float32 phases
+    // (src/host/kernels/nuft_sum.cpp)
+    if constexpr (sizeof(R) == 4) {
+      const long long n2 = (long long)nn();
+      cplx<R>* vvb = vv.as<cplx<R>>(n2);
+      const R* lm = static_cast<const R*>(lmn32.p);
+      for (int k = 0; k < nS; ++k) {
+        const double sc = 2.0 * 3.14159265358979323846 / static_cast<double>(hwl[k]);
+        const float* uk = du + (size_t)k * 3 * n2;
+        R* u = uvw_r.as<R>(3 * n2);
+        for (int l = 0; l < n_img; ++l) {
+          launch_virtual_vis<R>(1, n_ant, n_beam, pp.v_out + (size_t)k * n_ant * n_beam, n_ant, 0,
+                                pp.w_out + ((size_t)k * n_img + l) * n_beam, 0, vvb, 0, st);
           launch_scale_uvw<R>(n2, uk, n2, sc, u, u + n2, u + 2 * n2, st);
-          const R* lm = sizeof(R) == 8 ? reinterpret_cast<const R*>(lmn64.p)
-                                       : reinterpret_cast<const R*>(lmn32.p);
           launch_nuft_sum<R>(R(1), (int)n2, vvb, u, u + n2, u + 2 * n2, n_pix, lm, lm + n_pix,
                              lm + 2 * (size_t)n_pix, static_cast<R*>(img.p) + (size_t)l * n_pix, st);
         }

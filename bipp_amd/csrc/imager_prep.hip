@@ -58,7 +58,5 @@ void launch_scale_uvw(long long n, const float* uvw, long long lduvw, double sca
 }
 template void launch_scale_uvw<float>(long long, const float*, long long, double, float*, float*,
                                       float*, hipStream_t);
-template void launch_scale_uvw<double>(long long, const float*, long long, double, double*,
-                                       double*, double*, hipStream_t);
 
 }  // namespace bippamd

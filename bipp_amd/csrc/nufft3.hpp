@@ -214,6 +214,26 @@ struct N3VVParams {
   long long ld_vv;
 };
 
+// Direct sum over the points of a source: img[lv][q] += Re sum_points v_lv exp(i u . x_q) for
+// levels [lv0, lv0 + n_levels), n_levels <= 8.  chunks > 1: the slots are split over that
+// many workgroups per pixel block, their sums go through part ([chunks][n_levels][n_pix]).
+template <typename R>
+struct N3DirectParams {
+  N3Source src;
+  long long n_slots;        // slots_per_sample * samples
+  const cplx<R>* vv;        // [nS][n_levels_total][vv_stride], trace in slot (0, 1)
+  long long vv_stride;
+  int n_levels_total, lv0, n_levels;
+  int n_pix;
+  const double* lmn;        // [3][n_pix]
+  int chunks;
+  R* part;
+  R* img;                   // [n_levels_total][n_pix]
+};
+int direct_chunks(long long n_slots, int n_pix, int n_cu);
+template <typename R>
+void launch_direct_sum(const N3DirectParams<R>& p, hipStream_t st);
+
 void launch_pos_range(int n_samples, const double* pos, long long pos_stride, int apad,
                       const int* n_rows, int n_rows_const, double* out, hipStream_t st);
 // 1 per sample whose nAnt^2 x 3 uvw is antisymmetric with a zero diagonal, else 0

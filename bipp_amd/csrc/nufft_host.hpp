@@ -521,6 +521,7 @@ struct N3Runner {
   DevBuf grid, sorted, sorted_vals;
   DevBuf bin_count, bin_start, bin_rank, scan_tmp, vv, deconv, gl, twid, prof_buf;
   DevBuf group_of, group_count, group_start, group_fill, group_tmp, slot_list, ranges;
+  DevBuf direct_part;
   std::vector<cplx<TG>> htw;
   std::vector<TG> hdec;
   N3Plan plan;
@@ -599,6 +600,45 @@ struct N3Runner {
     BIPP_HIP(hipEventRecord(ev_vv[1], st));
   }
   static bool merge_auto(int rows_max) { return rows_max >= 2; }
+
+  // Direct sum of a batch instead of the transform: virtual visibilities of as many samples
+  // as fit 1 GiB at a time, then every level (eight per launch) at every pixel.
+  template <typename RE>
+  void direct(ContextImpl& c, const N3Source& src_all, int nS, int L, int n_cols, const cplx<RE>* z,
+              long long stride_z, int ldz, const RE* wd, const double* lmn64, int n_pix, TG* img) {
+    const int rows = src_all.n_ant_max;
+    const long long mat = (long long)rows * rows * L * (long long)sizeof(cplx<TG>);
+    const int per = static_cast<int>(std::max<long long>(1, std::min<long long>(nS, (1LL << 30) / mat)));
+    for (int k = 0; k < nS; k += per) {
+      const int m = std::min(per, nS - k);
+      N3Source src = src_all;
+      if (src.n_rows) src.n_rows += k;
+      if (src.pos) src.pos += (size_t)k * src.pos_stride;
+      if (src.uvw) src.uvw += (size_t)k * src.uvw_stride;
+      if (src.uvw_scale) src.uvw_scale += k;
+      if (src.antisym) src.antisym += k;
+      values<RE>(c, m, L, n_cols, rows, src.n_rows, z + (size_t)k * stride_z, stride_z, ldz,
+                 wd + (size_t)k * L * n_cols);
+      src.merge_auto = merge_auto(rows) ? 1 : 0;
+      src.ld_vv = ld_vv;
+      N3DirectParams<TG> dp;
+      dp.src = src;
+      dp.n_slots = src.slots_per_sample() * m;
+      dp.vv = static_cast<const cplx<TG>*>(vv.p);
+      dp.vv_stride = vv_stride;
+      dp.n_levels_total = L;
+      dp.n_pix = n_pix;
+      dp.lmn = lmn64;
+      dp.chunks = direct_chunks(dp.n_slots, n_pix, c.n_cu);
+      dp.part = dp.chunks > 1 ? direct_part.as<TG>((size_t)dp.chunks * std::min(L, 8) * n_pix) : nullptr;
+      dp.img = img;
+      for (int l = 0; l < L; l += 8) {
+        dp.lv0 = l;
+        dp.n_levels = std::min(8, L - l);
+        launch_direct_sum<TG>(dp, c.stream);
+      }
+    }
+  }
 
   // levels transformed together by the current plan: as many as the grid memory bound of
   // one box holds, at least one

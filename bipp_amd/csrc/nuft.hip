@@ -317,9 +317,6 @@ void launch_baselines(int n_ant, const double* xyz, long long ldxyz, double scal
 }
 template void launch_baselines<float>(int, const double*, long long, double, float*, float*,
                                       float*, hipStream_t);
-template void launch_baselines<double>(int, const double*, long long, double, double*, double*,
-                                       double*, hipStream_t);
-
 template <typename TS, typename TD>
 void launch_copy_cast(int n_batch, int rows, int cols, const void* src, long long lds,
                       long long stride_s, void* dst, long long ldd, long long stride_d,

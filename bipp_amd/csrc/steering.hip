@@ -441,30 +441,6 @@ __global__ __launch_bounds__(SteerCfg<MODE>::NT) void steer_kernel(SteerParams p
 // --------------------------------------------------------------------------------------
 // BF16X3 contraction
 // --------------------------------------------------------------------------------------
-// cos and sin of f turns, f in [-1/2, 1/2]: reduced to a quarter turn (exactly: 4 f and its
-// distance g to the nearest integer are representable), then minimax polynomials in g^2 of
-// sin(pi/2 g) / g (error 4.8e-9) and cos(pi/2 g) (error 4.7e-11), both below float rounding,
-// fitted by exchange on [0, 1/4].
-__device__ __forceinline__ void cossin_turn(float f, float& c, float& s) {
-  const float u = 4.0f * f;
-  const float q = rintf(u);
-  const float g = u - q;
-  const float y = g * g;
-  float ps = fmaf(y, -0.00460217700f, 0.0796802281f);
-  ps = fmaf(y, ps, -0.645963479f);
-  ps = fmaf(y, ps, 1.57079632f);
-  float pc = fmaf(y, 0.000903631703f, -0.0208600713f);
-  pc = fmaf(y, pc, 0.253669204f);
-  pc = fmaf(y, pc, -1.23370054f);
-  pc = fmaf(y, pc, 1.0f);
-  ps *= g;
-  const unsigned qi = static_cast<unsigned>(static_cast<int>(q));
-  const bool odd = qi & 1u;
-  const float a = odd ? ps : pc, b = odd ? pc : ps;
-  c = __uint_as_float(__float_as_uint(a) ^ (((qi + 1u) & 2u) << 30));
-  s = __uint_as_float(__float_as_uint(b) ^ ((qi & 2u) << 30));
-}
-
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ unsigned pack_bf16(float a, float b) {
