@@ -16,8 +16,8 @@ from typing import Dict, Iterable, List, Optional, Sequence, Tuple
 import numpy as np
 
 from . import _capi
-from ._capi import (GenericError, call, check, lib, ptr, COMPUTE, FILTERS, IMAGERS,  # noqa: F401
-                    PRECISION, PU)
+from ._capi import (GenericError, call, check, lib, ptr, typed_ptr, COMPUTE,  # noqa: F401
+                    FILTERS, IMAGERS, PRECISION, PU)
 from .levels import Filter, apply_filter, centroid_to_intervals, infer_intervals  # noqa: F401
 from .dataset import (Dataset, ImageData, ImageProp, InMemoryDataset,  # noqa: F401
                       InMemoryImageData, InMemoryImageProp)
@@ -204,19 +204,18 @@ def _eigh_common(gram: bool, wl, s, w, xyz=None):
     v = np.zeros((n_ant, n_beam), dtype=cdt, order="F")
     nr = C.c_size_t()
     sc = (C.c_float if single else C.c_double)()
-    rp = C.POINTER(C.c_float if single else C.c_double)
     if gram:
         xyz = _fortran(xyz, rdt)
         if xyz.shape != (n_ant, 3):
             raise _capi._EXC[3]("xyz must be (nAntenna, 3)")
         fn = lib().bipp_eigh_gram_s if single else lib().bipp_eigh_gram_d
         check(fn(rdt(wl), n_ant, n_beam, ptr(s), n_beam, ptr(w), n_ant,
-                 xyz.ctypes.data_as(rp), n_ant, d.ctypes.data_as(rp), ptr(v), n_ant,
+                 typed_ptr(xyz), n_ant, typed_ptr(d), ptr(v), n_ant,
                  C.byref(nr), C.byref(sc)))
     else:
         fn = lib().bipp_eigh_s if single else lib().bipp_eigh_d
         check(fn(rdt(wl), n_ant, n_beam, ptr(s), n_beam, ptr(w), n_ant,
-                 d.ctypes.data_as(rp), ptr(v), n_ant, C.byref(nr), C.byref(sc)))
+                 typed_ptr(d), ptr(v), n_ant, C.byref(nr), C.byref(sc)))
     return v, d, rdt(sc.value)
 
 
@@ -261,8 +260,8 @@ class NufftSynthesis:
         h = C.c_void_p()
         check(lib().bipp_synthesis_create(
             ctx.handle, COMPUTE[compute], IMAGERS[imager], self.n_antenna, self.n_beam,
-            self.n_levels, iv.ctypes.data_as(C.POINTER(C.c_double)), FILTERS[filter_name],
-            self.n_pixel, lmn.ctypes.data_as(C.POINTER(C.c_float)), self.n_pixel,
+            self.n_levels, typed_ptr(iv), FILTERS[filter_name],
+            self.n_pixel, typed_ptr(lmn), self.n_pixel,
             1 if batched else 0, C.byref(h)))
         self._h = h
         if tolerance is not None:
@@ -284,7 +283,7 @@ class NufftSynthesis:
         check(lib().bipp_synthesis_nufft_tuning(self._h, shape, 0, None, C.byref(n)))
         cand = np.zeros(5 * max(n.value, 1))
         check(lib().bipp_synthesis_nufft_tuning(self._h, shape, n.value,
-                                                cand.ctypes.data_as(C.POINTER(C.c_double)),
+                                                typed_ptr(cand),
                                                 C.byref(n)))
         rows = [(dict(zip(keys, (int(x) for x in cand[5 * k:5 * k + 4]))), float(cand[5 * k + 4]))
                 for k in range(n.value)]
@@ -313,7 +312,7 @@ class NufftSynthesis:
         cdt = np.complex128 if s.dtype == np.complex128 else np.complex64
         prec = PRECISION["double" if cdt == np.complex128 else "single"]
         # column-major per sample == row-major of the transpose
-        s_cm = np.ascontiguousarray(np.swapaxes(s, 1, 2).astype(cdt))
+        s_cm = np.ascontiguousarray(np.swapaxes(s, 1, 2), dtype=cdt)
         xyz = np.asarray(xyz, dtype=np.float64)
         if xyz.ndim == 2:
             xyz = np.broadcast_to(xyz, (n_s,) + xyz.shape)
@@ -322,14 +321,12 @@ class NufftSynthesis:
         w_cm, ldw, sw = None, 0, 0
         if w is not None:
             w = np.asarray(w)
-            if w.ndim == 2:
-                w = np.broadcast_to(w, (n_s,) + w.shape)
-            w_cm = np.ascontiguousarray(np.swapaxes(w, 1, 2).astype(cdt))
-            ldw, sw = self.n_antenna, self.n_antenna * self.n_beam
-        dpp = C.POINTER(C.c_double)
+            w_cm = np.ascontiguousarray(np.swapaxes(w, -1, -2), dtype=cdt)
+            # one matrix for all samples: stride 0
+            ldw, sw = self.n_antenna, self.n_antenna * self.n_beam if w.ndim == 3 else 0
         check(lib().bipp_synthesis_collect_host(
-            self._h, n_s, wl.ctypes.data_as(dpp), prec, ptr(s_cm), self.n_beam,
-            self.n_beam * self.n_beam, ptr(w_cm), ldw, sw, x_cm.ctypes.data_as(dpp),
+            self._h, n_s, typed_ptr(wl), prec, ptr(s_cm), self.n_beam,
+            self.n_beam * self.n_beam, ptr(w_cm), ldw, sw, typed_ptr(x_cm),
             self.n_antenna, 3 * self.n_antenna))
 
     def collect_device(self, n_samples: int, wl_dev: int, s_dev: int, s_double: bool,
@@ -358,7 +355,7 @@ class NufftSynthesis:
     def get(self, level: int, normalize: bool = True) -> np.ndarray:
         out = np.empty(self.n_pixel, dtype=np.float32)
         check(lib().bipp_synthesis_get(self._h, int(level), 1 if normalize else 0,
-                                       out.ctypes.data_as(C.POINTER(C.c_float))))
+                                       typed_ptr(out)))
         return out
 
     def images(self, normalize: bool = True) -> np.ndarray:
@@ -382,7 +379,7 @@ class NufftSynthesis:
     def timings(self, reset: bool = False) -> Dict[str, float]:
         """GPU milliseconds per stage accumulated over collect calls (HIP events)."""
         ms = np.zeros(9)
-        check(lib().bipp_synthesis_timings(self._h, ms.ctypes.data_as(C.POINTER(C.c_double)),
+        check(lib().bipp_synthesis_timings(self._h, typed_ptr(ms),
                                            1 if reset else 0))
         keys = ("eigensolve_ms", "prep_ms", "image_ms", "batches", "nufft_vv_ms",
                 "nufft_sort_ms", "nufft_spread_ms", "nufft_fft_ms", "nufft_interp_ms")
@@ -396,8 +393,8 @@ class NufftSynthesis:
         d = np.zeros((n.value, self.n_beam), dtype=np.float64)
         nr = np.zeros(n.value, dtype=np.int32)
         check(lib().bipp_synthesis_last_eigenvalues(
-            self._h, n.value, d.ctypes.data_as(C.POINTER(C.c_double)),
-            nr.ctypes.data_as(C.POINTER(C.c_int32)), None))
+            self._h, n.value, typed_ptr(d),
+            typed_ptr(nr), None))
         return d, nr
 
     def __del__(self) -> None:

@@ -10,6 +10,8 @@ import os
 import re
 from typing import Dict
 
+import numpy as np
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 LIB_PATH = os.path.join(HERE, "libbipp_amd.so")
@@ -148,6 +150,16 @@ def check(code: int) -> None:
 
 def call(name: str, *args) -> None:
     check(getattr(lib(), name)(*args))
+
+
+_EMPTY = {np.dtype(t): c * 0 for t, c in (("f4", C.c_float), ("f8", C.c_double), ("i4", i32))}
+
+
+def typed_ptr(a):
+    """A numpy array as a typed pointer argument.  (`ndarray.ctypes.data_as` builds a reference
+    cycle per call, and collecting the cycles of a few hundred calls walks every object of the
+    program: 45 ms with torch loaded.)  The caller keeps the array."""
+    return _EMPTY[a.dtype].from_address(a.ctypes.data)
 
 
 def ptr(a) -> int:

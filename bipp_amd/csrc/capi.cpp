@@ -649,6 +649,7 @@ void eigh_host(bool gram, T wl, size_t nAntenna, size_t nBeam, const void* s, si
     dflt = c.release();
   }
   ContextImpl& c = *dflt->impl;
+  PoolScope scope(c.pool);
   hipStream_t st = c.stream;
   constexpr bool dbl = sizeof(T) == 8;
   const size_t ce = 2 * sizeof(T);
@@ -875,7 +876,8 @@ BippError bipp_synthesis_collect_host(BippSynthesis h, size_t nSamples, const do
     BIPP_HIP(hipMemcpyAsync(sd, s, sb, hipMemcpyHostToDevice, st));
     const void* wd = nullptr;
     if (w) {
-      const size_t wb = es * strideW * nSamples;
+      // strideW == 0: one matrix for all samples
+      const size_t wb = es * (strideW ? strideW * nSamples : ldw * h->n_beam);
       void* p = h->st_w.get(wb);
       BIPP_HIP(hipMemcpyAsync(p, w, wb, hipMemcpyHostToDevice, st));
       wd = p;

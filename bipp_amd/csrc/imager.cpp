@@ -31,7 +31,8 @@ struct BippImagerImpl {
   int n_ant = 0, n_beam = 0, n_img = 0, n_pix = 0;
   N3Options opt;
   size_t batch_req = 0;  // requested samples per batch, 0: automatic
-  size_t batch = 0;      // samples per batch of the current staging buffers
+  size_t batch = 0;      // samples per batch
+  size_t staged = 0;     // samples that the staging buffers hold
   size_t count = 0;      // staged samples
   size_t n_added = 0;
   double pix_lo[3] = {0, 0, 0}, pix_hi[3] = {0, 0, 0};
@@ -48,22 +49,35 @@ struct BippImagerImpl {
            sizeof(float) * ((size_t)n_img * n_beam + 2);
   }
 
+  // Room for one more staged sample.  The buffers grow with the samples that come (pinning a
+  // whole batch of several hundred MB for a few samples took most of a call).
   void ensure_staging() {
-    if (batch) return;
-    size_t b = batch_req;
-    if (b == 0) {
-      // the reference's automatic batch: about 2 GB of points at 20 bytes per baseline
-      b = std::max<size_t>(1, 2000000000ULL / (20ULL * nn()));
-      b = std::min<size_t>(b, 4096);
+    if (!batch) {
+      size_t b = batch_req;
+      if (b == 0) {
+        // the reference's automatic batch: about 2 GB of points at 20 bytes per baseline
+        b = std::max<size_t>(1, 2000000000ULL / (20ULL * nn()));
+        b = std::min<size_t>(b, 4096);
+      }
+      // staging stays within 1 GiB of pinned memory
+      batch = std::max<size_t>(1, std::min<size_t>(b, (1ULL << 30) / sample_bytes()));
+      staged = std::min(staged, batch);
     }
-    // staging stays within 1 GiB of pinned memory
-    b = std::max<size_t>(1, std::min<size_t>(b, (1ULL << 30) / sample_bytes()));
-    batch = b;
-    h_uvw.get(sizeof(float) * 3 * nn() * b);
-    h_v.get(8 * (size_t)n_ant * n_beam * b);
-    h_d.get(sizeof(float) * (size_t)n_img * n_beam * b);
-    h_sc.get(sizeof(float) * b);
-    h_wl.get(sizeof(float) * b);
+    if (count < staged) return;
+    staged = std::min(batch, std::max<size_t>(16, 2 * staged));
+    grow(h_uvw, sizeof(float) * 3 * nn());
+    grow(h_v, 8 * (size_t)n_ant * n_beam);
+    grow(h_d, sizeof(float) * (size_t)n_img * n_beam);
+    grow(h_sc, sizeof(float));
+    grow(h_wl, sizeof(float));
+  }
+  // `b` with room for `staged` samples of `bytes` each, the first `count` kept
+  void grow(PinnedBuf& b, size_t bytes) {
+    if (b.cap >= bytes * staged) return;
+    PinnedBuf n;
+    n.get(bytes * staged);
+    if (count) std::memcpy(n.p, b.p, bytes * count);
+    n.swap(b);
   }
 
   void add(float wl, float scale, const float* uvw, size_t lduvw, const void* v, size_t ldv,
@@ -200,6 +214,7 @@ BippError bipp_imager_create(BippContext ctx, BippCompute compute, int imager, s
     require(compute == BIPP_COMPUTE_FP64 || compute == BIPP_COMPUTE_FP32 ||
                 compute == BIPP_COMPUTE_MIXED,
             BIPP_INVALID_PARAMETER_ERROR, "unknown compute mode");
+    PoolScope scope(ctx->impl->pool);
     auto h = std::make_unique<BippImagerImpl>();
     h->ctx = ctx;
     h->compute = compute;
@@ -209,22 +224,34 @@ BippError bipp_imager_create(BippContext ctx, BippCompute compute, int imager, s
     h->n_img = (int)nImages;
     h->n_pix = (int)nPixel;
     hipStream_t st = ctx->impl->stream;
-    std::vector<double> l64(3 * nPixel);
-    std::vector<float> l32(3 * nPixel);
-    for (size_t c3 = 0; c3 < 3; ++c3)
-      for (size_t q = 0; q < nPixel; ++q) {
-        l32[c3 * nPixel + q] = lmn[q + c3 * ldlmn];
-        l64[c3 * nPixel + q] = static_cast<double>(lmn[q + c3 * ldlmn]);
-      }
+    // eight running extremes per component (the compiler keeps them in a vector register);
+    // each starts from the first pixel and moves on a strict comparison
     for (int c3 = 0; c3 < 3; ++c3) {
-      const auto mm = std::minmax_element(l64.begin() + c3 * nPixel, l64.begin() + (c3 + 1) * nPixel);
-      h->pix_lo[c3] = *mm.first;
-      h->pix_hi[c3] = *mm.second;
+      const float* v = lmn + c3 * ldlmn;
+      float lo[8], hi[8];
+      for (int k = 0; k < 8; ++k) lo[k] = hi[k] = v[0];
+      size_t q = 0;
+      for (; q + 8 <= nPixel; q += 8)
+        for (int k = 0; k < 8; ++k) {
+          lo[k] = v[q + k] < lo[k] ? v[q + k] : lo[k];
+          hi[k] = v[q + k] > hi[k] ? v[q + k] : hi[k];
+        }
+      for (; q < nPixel; ++q) {
+        lo[0] = v[q] < lo[0] ? v[q] : lo[0];
+        hi[0] = v[q] > hi[0] ? v[q] : hi[0];
+      }
+      for (int k = 1; k < 8; ++k) {
+        lo[0] = lo[k] < lo[0] ? lo[k] : lo[0];
+        hi[0] = hi[k] > hi[0] ? hi[k] : hi[0];
+      }
+      h->pix_lo[c3] = lo[0];
+      h->pix_hi[c3] = hi[0];
     }
-    double* d64 = h->lmn64.as<double>(l64.size());
-    float* d32 = h->lmn32.as<float>(l32.size());
-    BIPP_HIP(hipMemcpyAsync(d64, l64.data(), sizeof(double) * l64.size(), hipMemcpyHostToDevice, st));
-    BIPP_HIP(hipMemcpyAsync(d32, l32.data(), sizeof(float) * l32.size(), hipMemcpyHostToDevice, st));
+    float* d32 = h->lmn32.as<float>(3 * nPixel);
+    for (int c3 = 0; c3 < 3; ++c3)
+      BIPP_HIP(hipMemcpyAsync(d32 + c3 * nPixel, lmn + c3 * ldlmn, sizeof(float) * nPixel,
+                              hipMemcpyHostToDevice, st));
+    launch_widen(d32, h->lmn64.as<double>(3 * nPixel), 3LL * nPixel, st);
     const size_t isz = h->img_double() ? 8 : 4;
     void* im = h->img.get(isz * nImages * nPixel);
     BIPP_HIP(hipMemsetAsync(im, 0, isz * nImages * nPixel, st));
@@ -277,6 +304,7 @@ BippError bipp_imager_add(BippImager h, float wl, float scale, const float* uvw,
     require(lduvw >= h->nn() && ldv >= (size_t)h->n_ant && lddScaled >= (size_t)h->n_beam,
             BIPP_INVALID_PARAMETER_ERROR, "leading dimension too small");
     require(wl > 0, BIPP_INVALID_PARAMETER_ERROR, "wavelength must be positive");
+    PoolScope scope(h->ctx->impl->pool);
     h->add(wl, scale, uvw, lduvw, v, ldv, dScaled, lddScaled);
   });
 }
@@ -286,6 +314,7 @@ BippError bipp_imager_get(BippImager h, size_t imgIdx, float* image) {
     require(h != nullptr, BIPP_INVALID_HANDLE_ERROR, "null handle");
     require(image != nullptr, BIPP_INVALID_POINTER_ERROR, "null image");
     require(imgIdx < (size_t)h->n_img, BIPP_INVALID_PARAMETER_ERROR, "image index out of range");
+    PoolScope scope(h->ctx->impl->pool);
     h->flush();
     hipStream_t st = h->ctx->impl->stream;
     if (h->img_double()) {

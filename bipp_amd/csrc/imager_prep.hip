@@ -37,7 +37,18 @@ __global__ void scale_uvw_kernel(long long n, const float* uvw, long long lduvw,
   w[i] = static_cast<R>(scale * static_cast<double>(uvw[i + 2 * lduvw]));
 }
 
+__global__ void widen_kernel(const float* in, double* out, long long n) {
+  const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+  if (i < n) out[i] = static_cast<double>(in[i]);
+}
+
 }  // namespace
+
+void launch_widen(const float* in, double* out, long long n, hipStream_t st) {
+  if (n <= 0) return;
+  widen_kernel<<<static_cast<unsigned>((n + 255) / 256), 256, 0, st>>>(in, out, n);
+  check_launch("widen_kernel");
+}
 
 template <typename R>
 void launch_eigpair_prep(const EigPairPrep<R>& p, int n_samples, hipStream_t st) {

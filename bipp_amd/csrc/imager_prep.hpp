@@ -19,6 +19,7 @@ struct EigPairPrep {
 
 template <typename R>
 void launch_eigpair_prep(const EigPairPrep<R>& p, int n_samples, hipStream_t st);
+void launch_widen(const float* in, double* out, long long n, hipStream_t st);
 template <typename R>
 void launch_scale_uvw(long long n, const float* uvw, long long lduvw, double scale, R* u, R* v,
                       R* w, hipStream_t st);

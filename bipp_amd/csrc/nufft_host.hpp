@@ -179,10 +179,34 @@ std::vector<double> es_ft_weights(double beta, const std::vector<double>& x,
   for (size_t i = 0; i < x.size(); ++i) ew[i] = w[i] * std::exp(beta * (std::sqrt(1 - x[i] * x[i]) - 1));
   return ew;
 }
-double es_ft_host(double xi, const std::vector<double>& x, const std::vector<double>& ew) {
-  double s = 0;
-  for (size_t i = 0; i < x.size(); ++i) s += ew[i] * std::cos(xi * x[i]);
-  return 2 * s;
+// phi(xi0 + j dxi) for j < n.  The cosines of a node step by a rotation, started afresh from
+// cos and sin every 16 entries (rounding of a few 1e-15): a tolerance's tables took 3 ms with
+// a cosine per node and entry.
+std::vector<double> es_ft_table(double xi0, double dxi, int n, const std::vector<double>& x,
+                                const std::vector<double>& ew) {
+  const size_t m = x.size();
+  std::vector<double> out(n), c(m), s(m), cd(m), sd(m);
+  for (size_t i = 0; i < m; ++i) {
+    cd[i] = std::cos(dxi * x[i]);
+    sd[i] = std::sin(dxi * x[i]);
+  }
+  for (int j = 0; j < n; ++j) {
+    if (j % 16 == 0)
+      for (size_t i = 0; i < m; ++i) {
+        const double a = (xi0 + j * dxi) * x[i];
+        c[i] = std::cos(a);
+        s[i] = std::sin(a);
+      }
+    double sum = 0;
+    for (size_t i = 0; i < m; ++i) {
+      sum += ew[i] * c[i];
+      const double t = c[i] * cd[i] - s[i] * sd[i];
+      s[i] = s[i] * cd[i] + c[i] * sd[i];
+      c[i] = t;
+    }
+    out[j] = 2 * sum;
+  }
+  return out;
 }
 
 }  // namespace
@@ -300,10 +324,9 @@ struct N3Plan {
       if (new_kernel || dec_nf1[d] != nf1[d] || dec_nf2[d] != nf2[d]) {
         deconv[d].resize(nf1[d]);
         const double a2 = 0.5 * w * h2[d];
-        for (int i = 0; i < nf1[d]; ++i) {
-          const int l = i - nf1[d] / 2;
-          deconv[d][i] = 1.0 / (a2 * es_ft_host(l * a2, gl_x, gl_ew));
-        }
+        const int half = nf1[d] / 2;  // phi is even; nf1 is even
+        const std::vector<double> phi = es_ft_table(0.0, a2, half + 1, gl_x, gl_ew);
+        for (int i = 0; i < nf1[d]; ++i) deconv[d][i] = 1.0 / (a2 * phi[std::abs(i - half)]);
         dec_nf1[d] = nf1[d];
         dec_nf2[d] = nf2[d];
       }
@@ -315,8 +338,7 @@ struct N3Plan {
       constexpr int NFT = 2048;
       const double xi_max = 1.05 * 3.14159265358979323846 * w / (2 * sigma) + 1e-3;
       const double delta = xi_max / NFT;
-      ft_tab.resize(NFT + 3);
-      for (int j = 0; j < NFT + 3; ++j) ft_tab[j] = es_ft_host(std::fabs((j - 1) * delta), gl_x, gl_ew);
+      ft_tab = es_ft_table(-delta, delta, NFT + 3, gl_x, gl_ew);  // phi is even
       ft_inv_delta = 1.0 / delta;
       tab_w = w;
     }
@@ -539,9 +561,8 @@ struct N3Runner {
   bool autotune = false;
   N3Tuning last_tuning;
   std::vector<std::pair<N3Tuning, float>> tune_log;  // candidates and ms of the last tuning
-  double* h_buf = nullptr;  // pinned: ranges, counts and starts read back by the host
+  PinnedBuf h_buf;          // ranges, counts and starts read back by the host
   double max_bytes_ = 0;    // grid memory bound of one box (bytes)
-  size_t h_cap = 0;
 
   N3Runner() = default;
   N3Runner(const N3Runner&) = delete;
@@ -549,18 +570,9 @@ struct N3Runner {
     for (auto e : evs) (void)hipEventDestroy(e);
     for (auto e : ev_vv)
       if (e) (void)hipEventDestroy(e);
-    if (h_buf) (void)hipHostFree(h_buf);
   }
 
-  double* host_buf(size_t n) {
-    if (h_cap < n) {
-      if (h_buf) BIPP_HIP(hipHostFree(h_buf));
-      h_buf = nullptr;
-      BIPP_HIP(hipHostMalloc(reinterpret_cast<void**>(&h_buf), sizeof(double) * n));
-      h_cap = n;
-    }
-    return h_buf;
-  }
+  double* host_buf(size_t n) { return h_buf.as<double>(n); }
   hipEvent_t pass_event(int pass, int stage, int edge) {
     const size_t i = ((size_t)pass * 4 + stage) * 2 + edge;
     while (evs.size() <= i) {

@@ -16,7 +16,7 @@ from typing import Dict, Iterable, List, Optional, Sequence, Tuple, Union
 import numpy as np
 
 from . import _capi
-from ._capi import COMPUTE, IMAGERS, check, lib
+from ._capi import COMPUTE, IMAGERS, check, lib, typed_ptr
 from .dataset import Dataset, ImageData, ImageProp, InMemoryImageData
 
 
@@ -45,7 +45,7 @@ class EigenpairImager:
         h = C.c_void_p()
         check(lib().bipp_imager_create(ctx.handle, COMPUTE[compute], IMAGERS[imager],
                                        self.n_antenna, self.n_beam, self.n_images, self.n_pixel,
-                                       lmn.ctypes.data_as(C.POINTER(C.c_float)), self.n_pixel,
+                                       typed_ptr(lmn), self.n_pixel,
                                        C.byref(h)))
         self._h = h
         check(lib().bipp_imager_set_tolerance(h, float(tolerance)))
@@ -63,13 +63,12 @@ class EigenpairImager:
         na, nb = self.n_antenna, self.n_beam
         if uvw.shape != (na * na, 3) or v.shape != (na, nb) or d.shape != (self.n_images, nb):
             raise _bad("sample arrays do not match the imager's antenna, beam and image counts")
-        fpp = C.POINTER(C.c_float)
-        check(lib().bipp_imager_add(self._h, float(wl), float(scale), uvw.ctypes.data_as(fpp),
-                                    na * na, v.ctypes.data, na, d.ctypes.data_as(fpp), nb))
+        check(lib().bipp_imager_add(self._h, float(wl), float(scale), typed_ptr(uvw),
+                                    na * na, v.ctypes.data, na, typed_ptr(d), nb))
 
     def get(self, index: int) -> np.ndarray:
         out = np.empty(self.n_pixel, dtype=np.float32)
-        check(lib().bipp_imager_get(self._h, int(index), out.ctypes.data_as(C.POINTER(C.c_float))))
+        check(lib().bipp_imager_get(self._h, int(index), typed_ptr(out)))
         return out
 
     @property

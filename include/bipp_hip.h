@@ -151,7 +151,8 @@ BippError bipp_synthesis_collect_graph(BippSynthesis h, size_t nSamples, const d
                                        size_t strideXyz);
 /* Graph captures and launches of bipp_synthesis_collect_graph on this handle. */
 BippError bipp_synthesis_graph_info(BippSynthesis h, long long* captures, long long* launches);
-/* Same as bipp_synthesis_collect with host arrays (copied to the device first). */
+/* Same as bipp_synthesis_collect with host arrays (copied to the device first).  strideW 0: one
+ * matrix W for all samples. */
 BippError bipp_synthesis_collect_host(BippSynthesis h, size_t nSamples, const double* wl,
                                       BippPrecision sPrec, const void* s, size_t lds,
                                       size_t strideS, const void* w, size_t ldw, size_t strideW,
