@@ -222,29 +222,6 @@ struct TriShared {
   cplx<double> yc, alpha;
 };
 
-// Sum of (re, im) over the four 16-lane rows: lane rows 0 and 1 return the real total, rows 2
-// and 3 the imaginary one.  permlane32_swap leaves both operands' lower halves in the first
-// result and their upper halves in the second; permlane16_swap does so with each pair of rows.
-__device__ __forceinline__ double rows_total(double re, double im) {
-  auto swap32 = [](unsigned a, unsigned b) {
-    return __builtin_amdgcn_permlane32_swap(a, b, false, false);
-  };
-  auto swap16 = [](unsigned a, unsigned b) {
-    return __builtin_amdgcn_permlane16_swap(a, b, false, false);
-  };
-  auto mk64 = [](unsigned lo, unsigned hi) {
-    return __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi) << 32) | lo));
-  };
-  const unsigned long long r = __double_as_longlong(re), q = __double_as_longlong(im);
-  const auto lo = swap32(static_cast<unsigned>(r), static_cast<unsigned>(q));
-  const auto hi = swap32(static_cast<unsigned>(r >> 32), static_cast<unsigned>(q >> 32));
-  const double z = mk64(lo[0], hi[0]) + mk64(lo[1], hi[1]);
-  const unsigned long long zz = __double_as_longlong(z);
-  const auto l2 = swap16(static_cast<unsigned>(zz), static_cast<unsigned>(zz));
-  const auto h2 = swap16(static_cast<unsigned>(zz >> 32), static_cast<unsigned>(zz >> 32));
-  return mk64(l2[0], h2[0]) + mk64(l2[1], h2[1]);
-}
-
 // sums of a and b over the workgroup in a fixed order; one barrier (slots alternate)
 template <int NW>
 __device__ __forceinline__ void tri_sum2(double& a, double& b, double* red) {

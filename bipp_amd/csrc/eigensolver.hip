@@ -120,6 +120,17 @@ struct alignas(2 * sizeof(R)) RPair {
   R x, y;
 };
 
+// The resident tridiagonalisation (eig_resident.hpp, float64 up to 256 beams) keeps 12 row tiles
+// of 64 elements per wavefront in LDS at 256 beams.
+template <typename R>
+constexpr bool tri_resident(int nmax) {
+  return std::is_same<R, double>::value && nmax <= 256;
+}
+template <typename R>
+constexpr int tri_lds_elems(int nmax) {
+  return tri_resident<R>(nmax) && nmax == 256 ? 12 * 64 * (EigCfg<256>::NT / 64) : 1;
+}
+
 template <typename R, int NMAX>
 struct EigShared {
   static constexpr int NW_ = EigCfg<NMAX>::NW;
@@ -133,7 +144,11 @@ struct EigShared {
     R dct[DcCfg<NMAX>::TILE_ELEMS];  // product tiles of the tridiagonal divide and conquer
   };
   union {
-    cplx<R> xw[NW_][NMAX];  // per-wave partial sums of the matrix-vector passes
+    struct {
+      cplx<R> xw[NW_][NMAX];  // per-wave partial sums of the matrix-vector passes
+      cplx<R> cx[NMAX];       // the column of the next reflector (resident form)
+      cplx<R> tt[tri_lds_elems<R>(NMAX)];  // column tiles of the resident form kept in LDS
+    };
     GemmTiles<R> gt;        // operand tiles of the GEMM passes
     BackTile<R, NMAX> bt;   // reflectors of the back-transform
     typename std::conditional<std::is_same<R, double>::value && bt_mfma(NMAX), BtBlock<R, NMAX>,
@@ -749,6 +764,35 @@ __device__ __noinline__ void tridiag_phase(int n, cplx<R>* __restrict__ A, int l
   __syncthreads();
 }
 
+// Sums over the four 16-lane rows of a wavefront by lane swaps: permlane32_swap leaves both
+// operands' lower halves in the first result and their upper halves in the second;
+// permlane16_swap does so with each pair of rows.
+__device__ __forceinline__ double swap_add32(double a, double b) {
+  const unsigned long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+  const auto lo = __builtin_amdgcn_permlane32_swap(static_cast<unsigned>(x), static_cast<unsigned>(y), false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap(static_cast<unsigned>(x >> 32), static_cast<unsigned>(y >> 32), false, false);
+  return __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi[0]) << 32) | lo[0])) +
+         __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi[1]) << 32) | lo[1]));
+}
+__device__ __forceinline__ double swap_add16(double a, double b) {
+  const unsigned long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+  const auto lo = __builtin_amdgcn_permlane16_swap(static_cast<unsigned>(x), static_cast<unsigned>(y), false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap(static_cast<unsigned>(x >> 32), static_cast<unsigned>(y >> 32), false, false);
+  return __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi[0]) << 32) | lo[0])) +
+         __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi[1]) << 32) | lo[1]));
+}
+// totals of a complex value: lane rows 0 and 1 return the real one, rows 2 and 3 the imaginary
+__device__ __forceinline__ double rows_total(double re, double im) {
+  const double z = swap_add32(re, im);
+  return swap_add16(z, z);
+}
+// of two complex values: lane rows 0 to 3 return Re a, Re b, Im a, Im b
+__device__ __forceinline__ double rows_total2(cplx<double> a, cplx<double> b) {
+  return swap_add16(swap_add32(a.re, a.im), swap_add32(b.re, b.im));
+}
+
+#include "eig_resident.hpp"
+
 // W = L^-1 of the Cholesky factor of G (chol_inv.hpp), out of line; -1 or the failing column.
 template <typename R, int NMAX>
 __device__ __noinline__ int chol_phase(int n, cplx<R>* L, int ld, cplx<R>* T, int ldt,
@@ -1119,6 +1163,8 @@ __device__ void solve_one(const EigParams<R>& p, int sid, EigShared<R, NMAX>& sh
       sh.de[0].y = 0;
     }
     __syncthreads();
+  } else if constexpr (tri_resident<R>(NMAX)) {
+    tridiag_resident<NMAX>(n, A, ld, p.prof ? p.prof + (size_t)sid * EIG_PROF_SLOTS + 16 : nullptr);
   } else {
     tridiag_phase<R, NMAX>(n, A, ld, p.prof ? p.prof + (size_t)sid * EIG_PROF_SLOTS + 16 : nullptr);
   }

@@ -71,6 +71,22 @@ def test_split_sizes(ctx, n, live):
             break
 
 
+@pytest.mark.parametrize("n,live", [(64, [2, 3, 4, 5, 15, 16, 17, 33, 63, 64]),
+                                    (128, [1, 65, 66, 97, 127, 128]),
+                                    (256, [129, 159, 160, 161, 191, 192, 193, 223, 255, 256])])
+def test_resident_sizes(ctx, n, live):
+    """The tridiagonalisation with the trailing matrix in registers (up to 256 beams): sizes on
+    both sides of its row tiles, and of the columns kept in registers (160) and LDS (192)."""
+    samples = make(n, live, n)
+    print(f"resident eigensolve n={n} live={live}", flush=True)
+    d, v, nr = solve(ctx, samples, n)
+    for k, smp in enumerate(samples):
+        vo, do, _, _ = O.eigh_gram(smp.wl, smp.s.astype(np.complex64), None, smp.xyz)
+        assert nr[k] == live[k]
+        assert np.abs(d[k] - do).max() < 1e-10 * np.abs(do).max()
+        assert rel((v[k] * d[k]) @ v[k].conj().T, (vo * do) @ vo.conj().T) < 1e-10
+
+
 def test_split_general_w(ctx):
     r = np.random.default_rng(5)
     na, nb = 300, 260
