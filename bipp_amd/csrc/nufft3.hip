@@ -678,6 +678,29 @@ __device__ __forceinline__ cplx<R> root_const(int m) {
     constexpr double ts[4] = {0, H2, 1, H2};
     c = tc[m];
     s = ts[m];
+  } else if constexpr (N == 10) {
+    constexpr double C = 0.809016994374947424102, D = 0.309016994374947424102,
+                     E = 0.587785252292473129169, F = 0.951056516295153572116;
+    constexpr double tc[5] = {1, C, D, -D, -C};
+    constexpr double ts[5] = {0, E, F, F, E};
+    c = tc[m];
+    s = ts[m];
+  } else if constexpr (N == 12) {
+    constexpr double tc[7] = {1, H3, 0.5, 0, -0.5, -H3, -1};
+    constexpr double ts[7] = {0, 0.5, H3, 1, H3, 0.5, 0};
+    c = tc[m];
+    s = ts[m];
+  } else if constexpr (N == 15) {
+    constexpr double tc[9] = {1, 0.913545457642600895502, 0.669130606358858213826,
+                              0.309016994374947424102, -0.104528463267653471400, -0.5,
+                              -0.809016994374947424102, -0.978147600733805637929,
+                              -0.978147600733805637929};
+    constexpr double ts[9] = {0, 0.406736643075800207754, 0.743144825477394235015,
+                              0.951056516295153572116, 0.994521895368273336923, H3,
+                              0.587785252292473129169, 0.207911690817759337102,
+                              -0.207911690817759337102};
+    c = tc[m];
+    s = ts[m];
   } else {
     static_assert(N == 6, "roots of the composite radices");
     constexpr double tc[3] = {1, 0.5, -0.5};
@@ -751,10 +774,16 @@ __device__ __forceinline__ void dft_small(cplx<R>* v) {
     dft_ct<R, 2, 4>(v);
   } else if constexpr (RAD == 9) {
     dft_ct<R, 3, 3>(v);
+  } else if constexpr (RAD == 10) {
+    dft_ct<R, 2, 5>(v);
+  } else if constexpr (RAD == 12) {
+    dft_ct<R, 3, 4>(v);
+  } else if constexpr (RAD == 15) {
+    dft_ct<R, 3, 5>(v);
   } else if constexpr (RAD == 16) {
     dft_ct<R, 4, 4>(v);
   } else {
-    static_assert(RAD == 5, "radix 2, 3, 4, 5, 6, 8, 9 or 16");
+    static_assert(RAD == 5, "radix 2, 3, 4, 5, 6, 8, 9, 10, 12, 15 or 16");
     // radix 5, roots w^k = exp(+2 pi i k / 5) = c_k + i s_k with w^4 = conj(w), w^3 =
     // conj(w^2): with t1 = x1 + x4, t2 = x2 + x3, t3 = x1 - x4, t4 = x2 - x3,
     //   y1, y4 = x0 + c1 t1 + c2 t2 +- i (s1 t3 + s2 t4)
@@ -1807,7 +1836,7 @@ void go_pass_rr(const N3PassParams<R>& p, hipStream_t st) {
   X(2, 1) X(2, 2) X(3, 1) X(3, 2) X(3, 3) X(4, 1) X(4, 2) X(4, 3) X(4, 4) X(5, 1) X(5, 2)   \
   X(5, 3) X(5, 4) X(5, 5) X(6, 1) X(6, 2) X(6, 3) X(6, 4) X(6, 5) X(6, 6) X(8, 1) X(8, 2)   \
   X(8, 3) X(8, 4) X(8, 5) X(8, 6) X(8, 8) X(9, 1) X(9, 2) X(9, 3) X(9, 4) X(9, 5) X(9, 6)   \
-  X(9, 8) X(9, 9) X(16, 1) X(16, 2) X(16, 3) X(16, 4) X(16, 5) X(16, 6) X(16, 8)
+  X(9, 8) X(9, 9) X(10, 5) X(10, 6) X(10, 9) X(10, 10) X(12, 9) X(12, 10) X(15, 5) X(16, 1) X(16, 2) X(16, 3) X(16, 4) X(16, 5) X(16, 6) X(16, 8)
 
 template <typename R>
 bool launch_fft_pass_rr(const N3PassParams<R>& p, hipStream_t st) {

@@ -1,0 +1,46 @@
+"""Type-3 NUFFT on grids whose strided axes take the register passes of radices 10 and 12 (60,
+100, 108, 120 points in one pass, 180 = 90 * 2, 200 = 100 * 2 and 240 = 120 * 2 in two), against
+the float64 oracle.  The array is scaled until the plan has the wanted y length (twice an even
+2^a 3^b 5^c)."""
+import math
+
+import numpy as np
+import pytest
+
+import bipp_amd
+from bipp_amd import synthetic
+from oracle import bipp_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("length", [48, 60, 100, 108, 120, 180, 200, 240])
+def test_fft_lengths(ctx, length):
+    compute, tol, bound = "mixed", 1e-5, 1e-4
+    r = np.random.default_rng(length)
+    n = 9
+    src, flux = synthetic.zenith_cap_sources(r, 5, 5.0)
+    p0 = synthetic.disk_positions(r, n, 1.0) + np.array([0, 0, 0.3]) * r.normal(size=(n, 1))
+    lmn = synthetic.make_lmn_grid(21, math.radians(20))
+    # nf2 = smooth(2 smooth(4 / pi X S + w + 1)); X: half extent of 2 pi (p_a - p_b) over a > b
+    w = math.ceil(math.log10(1 / tol)) + 1
+    a, b = np.tril_indices(n)
+    u = 2 * np.pi * (p0[a, 1] - p0[b, 1])
+    xs = 0.5 * (u.max() - u.min()) * 0.5 * (lmn[:, 1].max() - lmn[:, 1].min())
+    for want in np.arange(length / 2, length / 2 - 12, -0.25):
+        scale = (want - w - 1) / (4 / math.pi * xs)
+        if scale <= 0:
+            break
+        xyz = p0 * scale
+        s = synthetic.visibilities(xyz, 1.0, src, flux, 0.1)
+        syn = bipp_amd.NufftSynthesis(ctx, n, n, [[0.0, 3e38]], lmn, compute=compute,
+                                      imager="nufft", tolerance=tol)
+        syn.collect(1.0, s, xyz)
+        if syn.nufft_grid()[1] == length:
+            break
+    assert syn.nufft_grid()[1] == length
+    ref, _ = O.synthesize([synthetic.Sample(0, 0, 1.0, xyz, s, np.ones(n, bool))],
+                          np.array([[0.0, 3e38]]), lmn)
+    err = O.rel_l2(syn.images()[0], ref[0])
+    print(f"grid {syn.nufft_grid()} {compute}: rel L2 {err:.2e}", flush=True)
+    assert err <= bound     # the bound of the other mixed NUFFT tests
