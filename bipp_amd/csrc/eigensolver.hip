@@ -1360,44 +1360,78 @@ __device__ inline T norm_unfused(T re, T im) {
   return a + b;
 }
 
+// Bound: the latency of reading S through one CU, so sixteen wavefronts take four columns each
+// with all their loads in flight (512 beams: 0.048 ms; four wavefronts, a column at a time: 0.35 ms;
+// 256 beams, 300 samples: 0.035 against 0.11 ms).
+constexpr int FLAG_NT = 1024, FLAG_NW = FLAG_NT / 64;
 template <typename TIn>
-__global__ __launch_bounds__(NT) void flag_kernel(FlagParams p) {
+__global__ __launch_bounds__(FLAG_NT) void flag_kernel(FlagParams p) {
   extern __shared__ int flag_sh[];
-  __shared__ unsigned long long cnt_sh[NW];
+  __shared__ unsigned long long cnt_sh[FLAG_NW];
+  __shared__ int kept_sh[FLAG_NW];
   const int sid = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int nb = p.n_beam;
   const cplx<TIn>* S = reinterpret_cast<const cplx<TIn>*>(p.s) + (size_t)sid * p.stride_s;
   const TIn eps = sizeof(TIn) == 4 ? TIn(1.1920928955078125e-07) : TIn(2.220446049250313e-16);
-  for (int i = tid; i < nb; i += NT) flag_sh[i] = 0;
+  for (int i = tid; i < nb; i += FLAG_NT) flag_sh[i] = 0;
   __syncthreads();
   unsigned long long cnt = 0;
-  for (int c = wave; c < nb; c += NW) {
-    bool any = false;
-    for (int r = c + lane; r < nb; r += 64) {
-      const cplx<TIn> v = S[r + (size_t)c * p.lds];
-      const bool live = p.mode == 0 ? (norm_unfused(v.re, v.im) > eps)
-                                    : (fabs(v.re) >= eps || fabs(v.im) >= eps);
-      if (live) {
-        flag_sh[r] = 1;
-        cnt += 1 + (r != c);
-        any = true;
-      }
+  constexpr int UC = 4, UR = 2;  // columns and 64-row chunks loaded together
+  for (int c0 = wave * UC; c0 < nb; c0 += FLAG_NW * UC) {
+    bool any[UC] = {};
+    for (int r0 = c0 & ~63; r0 < nb; r0 += 64 * UR) {
+      cplx<TIn> v[UC][UR];
+#pragma unroll
+      for (int u = 0; u < UC; ++u)
+#pragma unroll
+        for (int k = 0; k < UR; ++k) {
+          const int c = c0 + u, r = r0 + 64 * k + lane;
+          v[u][k] = mk<TIn>(0, 0);
+          if (c < nb && r >= c && r < nb) v[u][k] = S[r + (size_t)c * p.lds];
+        }
+#pragma unroll
+      for (int u = 0; u < UC; ++u)
+#pragma unroll
+        for (int k = 0; k < UR; ++k) {
+          const int c = c0 + u, r = r0 + 64 * k + lane;
+          const bool live = p.mode == 0 ? (norm_unfused(v[u][k].re, v[u][k].im) > eps)
+                                        : (fabs(v[u][k].re) >= eps || fabs(v[u][k].im) >= eps);
+          if (live) {  // (a lane without an element holds zero, which is not live)
+            flag_sh[r] = 1;
+            cnt += 1 + (r != c);
+            any[u] = true;
+          }
+        }
     }
-    if (__any(any) && lane == 0) flag_sh[c] = 1;
+#pragma unroll
+    for (int u = 0; u < UC; ++u)
+      if (__any(any[u]) && lane == 0) flag_sh[c0 + u] = 1;
   }
   cnt = wave_sum(cnt);
   if (lane == 0) cnt_sh[wave] = cnt;
   __syncthreads();
+  // kept beams in order: 1024 at a time, ranks by ballots
+  int* idx = p.idx + (size_t)sid * p.idx_stride;
+  int base = 0;
+  for (int i0 = 0; i0 < nb; i0 += FLAG_NT) {
+    const bool kept = i0 + tid < nb && flag_sh[i0 + tid];
+    const unsigned long long m = __ballot(kept);
+    if (lane == 0) kept_sh[wave] = __popcll(m);
+    __syncthreads();
+    int at = base + __popcll(m & ((1ull << lane) - 1ull));
+    for (int w = 0; w < FLAG_NW; ++w) {
+      at += w < wave ? kept_sh[w] : 0;
+      base += kept_sh[w];
+    }
+    if (kept) idx[at] = i0 + tid;
+    __syncthreads();
+  }
   if (tid == 0) {
     unsigned long long total = 0;
-    for (int w = 0; w < NW; ++w) total += cnt_sh[w];
+    for (int w = 0; w < FLAG_NW; ++w) total += cnt_sh[w];
     p.n_vis[sid] = total;
-    int nr = 0;
-    int* idx = p.idx + (size_t)sid * p.idx_stride;
-    for (int i = 0; i < nb; ++i)
-      if (flag_sh[i]) idx[nr++] = i;
-    p.n_red[sid] = nr;
+    p.n_red[sid] = base;
   }
 }
 
@@ -1444,9 +1478,9 @@ void launch_flag(const FlagParams& p, int n_samples, bool in_double, hipStream_t
   if (n_samples <= 0) return;
   const size_t shmem = sizeof(int) * (size_t)p.n_beam;
   if (in_double)
-    flag_kernel<double><<<n_samples, NT, shmem, stream>>>(p);
+    flag_kernel<double><<<n_samples, FLAG_NT, shmem, stream>>>(p);
   else
-    flag_kernel<float><<<n_samples, NT, shmem, stream>>>(p);
+    flag_kernel<float><<<n_samples, FLAG_NT, shmem, stream>>>(p);
   check_launch("flag_kernel");
 }
 
