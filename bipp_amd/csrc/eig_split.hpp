@@ -124,7 +124,6 @@ __global__ __launch_bounds__(256) void split_gemm_kernel(EigParams<double> p, in
   cplx<double>* A = p.z_out + (size_t)sid * p.stride_z;
   const int lr = lane & 15, lk = lane >> 4;
   const int jr[2] = {jb + lr, jb + 16 + lr}, ir[2] = {ib + lr, ib + 16 + lr};
-  const int k0 = MODE == 2 ? ib : 0;
   const int k1 = MODE == 0 ? min(n, ib + 32) : (MODE == 1 ? min(n, jb + 32) : n);
   f64x4 dr[2][2], di[2][2];
 #pragma unroll
@@ -134,45 +133,75 @@ __global__ __launch_bounds__(256) void split_gemm_kernel(EigParams<double> p, in
       dr[a][b] = f64x4{0, 0, 0, 0};
       di[a][b] = f64x4{0, 0, 0, 0};
     }
-  auto load = [&](int k, cplx<double>* P, cplx<double>* Q) {
+  // Operands of step k for this lane's k + lk.  Rows past n read row n - 1 (their results are not
+  // stored).  MASK: k past k1 and, in the triangular operand, elements of the other triangle
+  // give zero; the steps between need no test, so their loads are a uniform base plus a fixed
+  // lane offset (with a test and a 64-bit address per load the vector ALU took 10
+  // instructions per MFMA, which the float64 MFMA does not overlap: 1.54 against 1.21 ms for 96
+  // products of 400..512 rows).
+  const unsigned uld = ld;
+  unsigned oj[2], oi[2];
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    const unsigned j = min(jr[b], n - 1), i = min(ir[b], n - 1);
+    oj[b] = MODE == 2 ? lk + j * uld : j + lk * uld;
+    oi[b] = MODE == 2 ? lk + i * uld : i + lk * uld;
+  }
+  auto load = [&](auto mask, int k, cplx<double>* P, cplx<double>* Q) __attribute__((always_inline)) {
+    const cplx<double>* bp = (MODE == 0 ? A : (MODE == 1 ? W : X)) + (MODE == 2 ? (size_t)k : (size_t)k * uld);
+    const cplx<double>* bq = (MODE == 1 ? X : W) + (MODE == 2 ? (size_t)k : (size_t)k * uld);
     const int e = k + lk;
-    const bool ok = e < k1;
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
-      const int j = jr[b], i = ir[b];
+      if (!decltype(mask)::value) {
+        P[b] = bp[oj[b]];
+        Q[b] = bq[oi[b]];
+        continue;
+      }
       P[b] = Q[b] = mk<double>(0, 0);
-      if (MODE == 0) {
-        if (ok && j < n) P[b] = A[j + (size_t)e * ld];
-        if (ok && i < n && e <= i) Q[b] = W[i + (size_t)e * ld];
-      } else if (MODE == 1) {
-        if (ok && j < n && e <= j) P[b] = W[j + (size_t)e * ld];
-        if (ok && i < n) Q[b] = X[i + (size_t)e * ld];
-      } else {
-        if (ok && j < n) P[b] = X[e + (size_t)j * ld];
-        if (ok && i < n && e >= i) Q[b] = W[e + (size_t)i * ld];
+      if (e < k1) {
+        if (MODE != 1 || e <= jr[b]) P[b] = bp[oj[b]];
+        if (MODE == 1 || (MODE == 0 ? e <= ir[b] : e >= ir[b])) Q[b] = bq[oi[b]];
       }
     }
   };
-  cplx<double> P[2], Q[2];
-  load(k0, P, Q);
-  for (int k = k0; k < k1; k += 4) {
-    cplx<double> Pn[2], Qn[2];
-    load(k + 4, Pn, Qn);
+  auto mul = [&](const cplx<double>* P, const cplx<double>* Q) __attribute__((always_inline)) {
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+    for (int a = 0; a < 2; ++a) {
+      const double np = -P[a].im;
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
         // conj(P) Q: re Pr Qr + Pi Qi, im Pr Qi - Pi Qr (MODE 2: P conj(Q), the conjugate)
         dr[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(P[a].re, Q[b].re, dr[a][b], 0, 0, 0);
         dr[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(P[a].im, Q[b].im, dr[a][b], 0, 0, 0);
         di[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(P[a].re, Q[b].im, di[a][b], 0, 0, 0);
-        di[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(-P[a].im, Q[b].re, di[a][b], 0, 0, 0);
+        di[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(np, Q[b].re, di[a][b], 0, 0, 0);
       }
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      P[b] = Pn[b];
-      Q[b] = Qn[b];
     }
+  };
+  auto run = [&](auto mask, int ka, int kb) __attribute__((always_inline)) {
+    if (ka >= kb) return;
+    cplx<double> P[2][2], Q[2][2];
+    load(mask, ka, P[0], Q[0]);
+    for (int k = ka; k < kb; k += 8) {
+      if (k + 4 < kb) load(mask, k + 4, P[1], Q[1]);
+      mul(P[0], Q[0]);
+      if (k + 4 >= kb) break;
+      if (k + 8 < kb) load(mask, k + 8, P[0], Q[0]);
+      mul(P[1], Q[1]);
+    }
+  };
+  constexpr std::true_type MASKED{};
+  constexpr std::false_type PLAIN{};
+  if (MODE == 2) {
+    const int k2 = n & ~3;
+    run(MASKED, ib, min(n, ib + 32));
+    run(PLAIN, ib + 32, k2);
+    if (k2 >= ib + 32) run(MASKED, k2, n);
+  } else {
+    const int kd = MODE == 0 ? ib : jb;  // the triangular operand's diagonal blocks begin
+    run(PLAIN, 0, kd);
+    run(MASKED, kd, k1);
   }
   cplx<double>* out = MODE == 0 ? X : A;
 #pragma unroll
