@@ -219,28 +219,40 @@ __global__ __launch_bounds__(256) void split_gemm_kernel(EigParams<double> p, in
 }
 
 // --------------------------------------------------------------------------------------
-// Tridiagonalisation, one launch per column c (zhetd2 order, lower triangle).
+// Tridiagonalisation (zhetd2 order, lower triangle): the first n - TRI_TAIL columns with one
+// launch per column c, the trailing matrix that is left in the registers of one workgroup per
+// sample (split_tail_kernel).
 //
-// State between launches (parity c & 1): the reflector v_c and tau_c, and y = A v_c over the
-// trailing matrix as per-workgroup row sums plus the column sums.  Launch c
+// State between launches: the reflectors v, tau of the last TRI_LAG columns and their w, and
+// y = A v_{c-1} over the trailing matrix as per-workgroup row sums plus the column sums.  Launch c
 //   - forms w_{c-1} from y, v_{c-1}, tau_{c-1}, the updated column c and its reflector v_c (every
 //     workgroup of the sample for itself, from the same operands in the same order, so all
-//     hold the same bits; workgroup 0 records d_c, e_c, v_c, tau_c and puts v_{c-1} into its
-//     column of A);
-//   - applies the pending update A -= v w^H + w v^H (of c - 1) to its columns of the trailing
-//     matrix and adds their part of A v_c from the updated lower triangle.
+//     hold the same bits; workgroup 0 records d_c, e_c, v_c, tau_c, w_{c-1} and puts v_{c-1} into
+//     its column of A);
+//   - applies the P pending updates A -= v w^H + w v^H to its columns of the trailing matrix and
+//     adds their part of A v_c from the updated lower triangle.  The updated elements are
+//     stored in every TRI_LAG-th launch only; the others repeat them from the same operands.
+//   - at c = n - TRI_TAIL forms no reflector and stores what is pending.
 // Bound: the launches follow each other (a prologue of two workgroup sums and the round trip
 // through the last-level cache per launch), then, for many samples, the last-level cache (the
-// trailing triangle read and written once per column).  Lanes hold 16 rows x 4 columns, so a
-// column's sum takes four lane moves for four columns at once, and row sums over the columns
-// of a wavefront stay in registers.  Column tiles of 4 are dealt to the sample's wavefronts in
-// turn, which keeps them balanced while the trailing matrix shrinks.
+// trailing triangle read once per column and written once per TRI_LAG).  Lanes hold 16 rows x 4
+// columns, so a column's sum takes four lane moves for four columns at once, and row sums over
+// the columns of a wavefront stay in registers.  Column tiles of 4 are dealt to the sample's
+// wavefronts in turn, which keeps them balanced while the trailing matrix shrinks.
+// Measured, batches of 400..512 beams: 96 samples 28.3 to 24.8 ms, 12 samples 15.4 to 14.1 ms against
+// launches for all columns that store every time; over the first 256 columns of 96 samples a
+// storing launch takes 43 us on average, one that does not 30 us, the tail kernel 1.84 ms.  (Longer
+// lags could save a sixth of a launch at most and take the LDS of the second workgroup.)
 // --------------------------------------------------------------------------------------
 constexpr int TRI_N = 512;   // largest reduced size
 constexpr int TRI_GMAX = 8;  // workgroups per sample of a launch
+constexpr int TRI_TAIL = 256;  // columns left to split_tail_kernel
+constexpr int TRI_LAG = 2;   // columns per store of the trailing matrix
+constexpr int TRI_RING = TRI_LAG + 1;
 
 struct TriWork {
-  cplx<double>* v;     // [job][2][nmax]
+  cplx<double>* v;     // [job][TRI_RING][nmax], column c in slot c mod TRI_RING
+  cplx<double>* w;     // [job][TRI_RING][nmax]
   cplx<double>* tau;   // [job][2]
   cplx<double>* col;   // [job][2][nmax] column sums
   cplx<double>* row;   // [job][2][TRI_GMAX][nmax] row sums of each workgroup
@@ -248,12 +260,13 @@ struct TriWork {
   int* perm;           // [job][nmax]
 };
 
-template <int NW>
+template <int NW, int P>
 struct TriShared {
-  cplx<double> v[TRI_N], w[TRI_N], vn[TRI_N];
+  cplx<double> v[P ? P : 1][TRI_N], w[P ? P : 1][TRI_N];  // pending updates, newest first
+  cplx<double> vn[TRI_N];
   cplx<double> xw[NW][TRI_N];  // a wavefront's row sums
   double red[2][2 * NW];
-  cplx<double> yc, alpha;
+  cplx<double> yc, alpha, vc[P ? P : 1], wc[P ? P : 1];  // row c of y and of the older updates
 };
 
 // sums of a and b over the workgroup in a fixed order; one barrier (slots alternate)
@@ -277,22 +290,26 @@ __device__ __forceinline__ void tri_sum2(double& a, double& b, double* red) {
 }
 
 // NCT: column tiles of a wavefront taken together (a tile's row operands are read once)
-template <int NT, int NCT>
+// P: pending updates, those of columns c - 1 .. c - P
+template <int NT, int NCT, int P>
 __global__ __launch_bounds__(NT) void tri_column_kernel(EigParams<double> p, TriWork tw, int c) {
   constexpr int NW = NT / 64, RPT = TRI_N / NT;
-  __shared__ TriShared<NW> sh;
+  __shared__ TriShared<NW, P> sh;
   const int job = blockIdx.y, g = blockIdx.x, G = gridDim.x;
   const int sid = p.order[job], n = p.n_red[sid];
-  if (c >= n || p.info[sid] != 0 || (c == n - 1 && g != 0)) return;  // uniform
+  const int last = n - TRI_TAIL;  // the column that hands over
+  if (c > last || last <= 0 || p.info[sid] != 0) return;  // uniform
+  const bool hand = c == last, keep = hand || P == TRI_LAG;  // keep: store the updated elements
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ld = p.ldz, nmax = p.nmax;
   cplx<double>* A = p.z_out + (size_t)sid * p.stride_z;
   const int cur = c & 1, prv = cur ^ 1;
   const size_t j2 = (size_t)job * 2;
-  const bool apply = c > 0;
+  const size_t jr = (size_t)job * TRI_RING;
+  auto slot = [&](int col) { return (jr + col % TRI_RING) * nmax; };
 
-  const int i0 = c + 1;
+  const int i0 = hand ? c : c + 1;
   const int lr = lane & 15, lc = lane >> 4;
   const int W = G * NW, gw = g * NW + wave;
   const int ct_end = (n + 3) >> 2, rt_end = (n + 15) >> 4;
@@ -323,51 +340,64 @@ __global__ __launch_bounds__(NT) void tri_column_kernel(EigParams<double> p, Tri
   load(ct >> 2, x);
 
   // ---- w_{c-1}, column c, its reflector; a thread holds rows tid + NT q ----------------
-  cplx<double> a[RPT], v[RPT], y[RPT], tau = mk<double>(0, 0);
+  cplx<double> a[RPT], v[P ? P : 1][RPT], w[P ? P : 1][RPT], y[RPT], tau = mk<double>(0, 0);
   bool live[RPT];
 #pragma unroll
   for (int q = 0; q < RPT; ++q) {
     const int i = tid + NT * q;
     live[q] = i >= c && i < n;
-    a[q] = v[q] = y[q] = mk<double>(0, 0);
+    a[q] = y[q] = mk<double>(0, 0);
+#pragma unroll
+    for (int k = 0; k < (P ? P : 1); ++k) v[k][q] = w[k][q] = mk<double>(0, 0);
     if (live[q]) {
-      a[q] = A[i + (size_t)c * ld];
-      if (apply) {
-        v[q] = tw.v[(j2 + prv) * nmax + i];
+      if (!hand) a[q] = A[i + (size_t)c * ld];  // (at the handover its owner is storing to it)
+#pragma unroll
+      for (int k = 0; k < P; ++k) {
+        v[k][q] = tw.v[slot(c - 1 - k) + i];
+        if (k > 0) w[k][q] = tw.w[slot(c - 1 - k) + i];
+      }
+      if (P > 0) {
         y[q] = tw.col[(j2 + prv) * nmax + i];
         for (int k = 0; k < G; ++k) y[q] = y[q] + tw.row[((j2 + prv) * TRI_GMAX + k) * nmax + i];
       }
-      if (i == c) sh.yc = y[q];
+      if (i == c) {
+        sh.yc = y[q];
+#pragma unroll
+        for (int k = 1; k < P; ++k) sh.vc[k] = v[k][q], sh.wc[k] = w[k][q];
+      }
     }
   }
-  cplx<double> w[RPT];
-#pragma unroll
-  for (int q = 0; q < RPT; ++q) w[q] = mk<double>(0, 0);
-  if (apply) {
+  if (P > 0) {
     tau = tw.tau[j2 + prv];
     double pr = 0, pi = 0;
 #pragma unroll
     for (int q = 0; q < RPT; ++q) {
-      w[q] = tau * y[q];
-      const cplx<double> dt = cmul_conj_a(w[q], v[q]);
+      w[0][q] = tau * y[q];
+      const cplx<double> dt = cmul_conj_a(w[0][q], v[0][q]);
       pr += dt.re;
       pi += dt.im;
     }
     tri_sum2<NW>(pr, pi, sh.red[0]);
     const cplx<double> alpha2 = tau * mk<double>(-0.5 * pr, -0.5 * pi);
-    const cplx<double> wc = tau * sh.yc + alpha2;  // row c, where v is 1
+    const cplx<double> wc = tau * sh.yc + alpha2;  // row c, where v_{c-1} is 1
 #pragma unroll
     for (int q = 0; q < RPT; ++q) {
-      w[q] = w[q] + alpha2 * v[q];
-      if (live[q]) a[q] = a[q] - (v[q] * conj(wc) + w[q]);
+      w[0][q] = w[0][q] + alpha2 * v[0][q];
+      if (!live[q]) continue;
+#pragma unroll
+      for (int k = P - 1; k > 0; --k) a[q] = a[q] - (v[k][q] * conj(sh.wc[k]) + w[k][q] * conj(sh.vc[k]));
+      a[q] = a[q] - (v[0][q] * conj(wc) + w[0][q]);
     }
   }
   double part = 0, unused = 0;
 #pragma unroll
   for (int q = 0; q < RPT; ++q) {
     const int i = tid + NT * q;
-    sh.v[i] = v[q];
-    sh.w[i] = w[q];
+#pragma unroll
+    for (int k = 0; k < P; ++k) {
+      sh.v[k][i] = v[k][q];
+      sh.w[k][i] = w[k][q];
+    }
     if (i == c + 1) sh.alpha = a[q];
     if (live[q] && i >= c + 2) part += abs2(a[q]);
   }
@@ -377,22 +407,16 @@ __global__ __launch_bounds__(NT) void tri_column_kernel(EigParams<double> p, Tri
     for (int q = 0; q < RPT; ++q) {
       const int i = tid + NT * q;
       if (!live[q]) continue;
-      if (apply) {
+      if (P > 0) {
+        tw.w[slot(c - 1) + i] = w[0][q];
         if (i > c)
-          A[i + (size_t)(c - 1) * ld] = v[q];
+          A[i + (size_t)(c - 1) * ld] = v[0][q];
         else
           A[(c - 1) + (size_t)(c - 1) * ld] = tau;  // the diagonal slot keeps tau
       }
-      if (i == c) {
-        tw.de[((size_t)job * nmax + c) * 2] = a[q].re;
-        if (c == n - 1) {
-          tw.de[((size_t)job * nmax + c) * 2 + 1] = 0;
-          A[c + (size_t)c * ld] = mk<double>(0, 0);  // no reflector for the last column
-        }
-      }
+      if (i == c && !hand) tw.de[((size_t)job * nmax + c) * 2] = a[q].re;
     }
   }
-  if (c == n - 1) return;
   const cplx<double> alpha = sh.alpha;
   cplx<double> tn, scal;
   double beta;
@@ -413,7 +437,7 @@ __global__ __launch_bounds__(NT) void tri_column_kernel(EigParams<double> p, Tri
     if (live[q] && i >= c + 2) vn = a[q] * scal;
     sh.vn[i] = vn;
     if (g == 0) {
-      if (live[q] && i > c) tw.v[(j2 + cur) * nmax + i] = vn;
+      if (live[q] && i > c) tw.v[slot(c) + i] = vn;
       if (i == c) {
         tw.tau[j2 + cur] = tn;
         tw.de[((size_t)job * nmax + c) * 2 + 1] = beta;
@@ -430,12 +454,15 @@ __global__ __launch_bounds__(NT) void tri_column_kernel(EigParams<double> p, Tri
       load(ct >> 2, x);
     }
     first = false;
-    cplx<double> cv[NCT], cw[NCT], cn[NCT], cs[NCT];
+    cplx<double> cv[P ? P : 1][NCT], cw[P ? P : 1][NCT], cn[NCT], cs[NCT];
 #pragma unroll
     for (int u = 0; u < NCT; ++u) {
       const int jj = min(jc[u], TRI_N - 1);
-      cv[u] = conj(sh.v[jj]);
-      cw[u] = conj(sh.w[jj]);
+#pragma unroll
+      for (int q = 0; q < P; ++q) {
+        cv[q][u] = conj(sh.v[q][jj]);
+        cw[q][u] = conj(sh.w[q][jj]);
+      }
       cn[u] = sh.vn[jj];
       cs[u] = mk<double>(0, 0);
     }
@@ -446,18 +473,20 @@ __global__ __launch_bounds__(NT) void tri_column_kernel(EigParams<double> p, Tri
         const int r = 16 * (rt + k) + lr;
         if (16 * (rt + k) >= n) break;  // uniform
         const int rr = min(r, TRI_N - 1);
-        const cplx<double> vi = sh.v[rr], wi = sh.w[rr], ni = sh.vn[rr];
+        const cplx<double> ni = sh.vn[rr];
+        cplx<double> vi[P ? P : 1], wi[P ? P : 1];
+#pragma unroll
+        for (int q = 0; q < P; ++q) vi[q] = sh.v[q][rr], wi[q] = sh.w[q][rr];
         cplx<double> acc = mk<double>(0, 0);
 #pragma unroll
         for (int u = 0; u < NCT; ++u) {
           if (r < n && r >= jc[u]) {
             cplx<double> e = x[k][u];
-            if (apply) {
-              e = e - (vi * cw[u] + wi * cv[u]);
-              A[r + (size_t)jc[u] * ld] = e;
-            }
-            acc = acc + e * cn[u];
-            if (r > jc[u]) cs[u] = cs[u] + cmul_conj_a(e, ni);
+#pragma unroll
+            for (int q = P - 1; q >= 0; --q) e = sub_mul2(e, vi[q], cw[q][u], wi[q], cv[q][u]);
+            if (keep) A[r + (size_t)jc[u] * ld] = e;
+            acc = add_mul(acc, e, cn[u]);
+            if (r > jc[u]) cs[u] = add_mul_conj(cs[u], e, ni);
           }
         }
         const double t = rows_total(acc.re, acc.im);
@@ -486,6 +515,29 @@ __global__ __launch_bounds__(NT) void tri_column_kernel(EigParams<double> p, Tri
 #pragma unroll
     for (int k = 1; k < NW; ++k) s = s + sh.xw[k][i];
     tw.row[((j2 + cur) * TRI_GMAX + g) * nmax + i] = s;
+  }
+}
+
+// The trailing matrix from column n - TRI_TAIL on (all of a smaller one).  Workgroup per job.
+__global__ __launch_bounds__(EigCfg<TRI_TAIL>::NT) void split_tail_kernel(EigParams<double> p, TriWork tw) {
+  EigShared<double, TRI_TAIL>& sh = eig_sh<double, TRI_TAIL>;
+  const int job = blockIdx.x, sid = p.order[job], n = p.n_red[sid], ld = p.ldz;
+  if (n <= 0 || p.info[sid] != 0) return;
+  const int c0 = max(0, n - TRI_TAIL), m = n - c0;
+  cplx<double>* A = p.z_out + (size_t)sid * p.stride_z + c0 + (size_t)c0 * ld;
+  if (m > 1) {
+    tridiag_resident<TRI_TAIL>(m, A, ld, nullptr);
+  } else {
+    if (threadIdx.x == 0) {
+      sh.de[0].x = A[0].re;
+      sh.de[0].y = 0;
+      A[0] = mk<double>(0, 0);
+    }
+    __syncthreads();
+  }
+  for (int i = threadIdx.x; i < m; i += EigCfg<TRI_TAIL>::NT) {
+    tw.de[((size_t)job * p.nmax + c0 + i) * 2] = sh.de[i].x;
+    tw.de[((size_t)job * p.nmax + c0 + i) * 2 + 1] = sh.de[i].y;
   }
 }
 

@@ -1516,7 +1516,7 @@ void launch_eig(const EigParams<R>& p, int n_slots, bool in_double, hipStream_t 
 EigSplitSizes eig_split_sizes(int n_jobs, int nmax) {
   EigSplitSizes z;
   const size_t jn = (size_t)n_jobs * nmax;
-  z.cplx_elems = jn * (2 + 2 + 2 * TRI_GMAX) + 2 * (size_t)n_jobs;
+  z.cplx_elems = jn * (2 * TRI_RING + 2 + 2 * TRI_GMAX) + 2 * (size_t)n_jobs;
   z.real_elems = 2 * jn;
   z.int_elems = jn;
   return z;
@@ -1532,7 +1532,8 @@ void launch_eig_split(const EigParams<double>& p, const EigSplitBuffers& b, int 
   const size_t jn = (size_t)jobs * p.nmax;
   TriWork tw;
   tw.v = b.cplx_buf;
-  tw.col = tw.v + 2 * jn;
+  tw.w = tw.v + TRI_RING * jn;
+  tw.col = tw.w + TRI_RING * jn;
   tw.row = tw.col + 2 * jn;
   tw.tau = tw.row + 2 * TRI_GMAX * jn;
   tw.de = b.real_buf;
@@ -1561,13 +1562,25 @@ void launch_eig_split(const EigParams<double>& p, const EigSplitBuffers& b, int 
   // (20.8), 96 samples 32.5 against 30.9 with 256 threads.
   const bool wide = n_cu / jobs >= 4;
   const int G = std::max(1, std::min(TRI_GMAX, (wide ? n_cu : 2 * n_cu) / jobs));
-  for (int c = 0; c < n_max; ++c) {
+  auto column = [&](auto pending, int c) {
+    constexpr int P = decltype(pending)::value;
     if (wide)
-      tri_column_kernel<512, 2><<<dim3(G, jobs), 512, 0, stream>>>(p, tw, c);
+      tri_column_kernel<512, 2, P><<<dim3(G, jobs), 512, 0, stream>>>(p, tw, c);
     else
-      tri_column_kernel<256, 2><<<dim3(G, jobs), 256, 0, stream>>>(p, tw, c);
+      tri_column_kernel<256, 2, P><<<dim3(G, jobs), 256, 0, stream>>>(p, tw, c);
+  };
+  for (int c = 0; c <= n_max - TRI_TAIL; ++c) {
+    if (c == 0)
+      column(std::integral_constant<int, 0>{}, c);
+    else if (c % TRI_LAG)
+      column(std::integral_constant<int, 1>{}, c);
+    else
+      column(std::integral_constant<int, 2>{}, c);
   }
+  static_assert(TRI_LAG == 2, "one launch for each count of pending updates");
   check_launch("tri_column_kernel");
+  split_tail_kernel<<<jobs, EigCfg<TRI_TAIL>::NT, 0, stream>>>(p, tw);
+  check_launch("split_tail_kernel");
   split_dc_kernel<NM><<<jobs, EigCfg<NM>::NT, 0, stream>>>(p, tw);
   check_launch("split_dc_kernel");
   if (n_max > 1) {

@@ -87,6 +87,21 @@ def test_resident_sizes(ctx, n, live):
         assert rel((v[k] * d[k]) @ v[k].conj().T, (vo * do) @ vo.conj().T) < 1e-10
 
 
+def test_handover_sizes(ctx):
+    """The tridiagonalisation hands the last 256 columns from the column launches to one workgroup
+    per sample: with one and with two updates pending (odd and even counts of columns before
+    it), and samples that have no column before it."""
+    n, live = 259, [256, 257, 258, 259, 255, 3]
+    samples = make(n, live, 7)
+    print(f"split eigensolve n={n} live={live}", flush=True)
+    d, v, nr = solve(ctx, samples, n)
+    for k, smp in enumerate(samples):
+        vo, do, _, _ = O.eigh_gram(smp.wl, smp.s.astype(np.complex64), None, smp.xyz)
+        assert nr[k] == live[k]
+        assert np.abs(d[k] - do).max() < 1e-10 * np.abs(do).max()
+        assert rel((v[k] * d[k]) @ v[k].conj().T, (vo * do) @ vo.conj().T) < 1e-10
+
+
 def test_split_general_w(ctx):
     r = np.random.default_rng(5)
     na, nb = 300, 260
