@@ -389,9 +389,9 @@ def main() -> None:
                              "kernel_ms": kern_ms, "fine_grid": list(nf), "spread_grid": nf1,
                              "points": m_pts, "algorithmic_bytes_per_launch": nufft_bytes}
         # measured HBM bytes of the chain: per-dispatch counters times dispatches per step
-        # (one spread launch per 4 levels; strided axes above 128 points take two passes)
+        # (one spread launch per 6 levels; strided axes above 128 points take two passes)
         launches = {"n3_points_kernel": 2,
-                    "n3_spread_kernel": (L + 3) // 4, "fft_lines_kernel": 1,
+                    "n3_spread_kernel": (L + 5) // 6, "fft_lines_kernel": 1,
                     "fft_pass_rr_kernel": sum(2 if x > 128 else 1 for x in nf[1:]),
                     "n3_interp_kernel": 1}
         per_kernel = {}

@@ -32,7 +32,6 @@ namespace bippamd {
 namespace {
 
 constexpr int SP_BIN = 8;    // spread block edge: one wavefront per 8^3 block
-constexpr int SP_LG = 4;     // levels per spread launch (sums kept in registers)
 constexpr int SP_WMAX = 16;  // largest kernel width
 constexpr int SP_MAXR = 9;   // neighbour bin ranges per block: (nback + 1)^2 with nback <= 2
 constexpr int FFT_NT = 512;  // FFT workgroup: ~2 radix-4 butterflies per thread per stage
@@ -386,76 +385,108 @@ __global__ void scan_add_kernel(unsigned* out, const unsigned* block_offsets, in
 
 
 // --------------------------------------------------------------------------------------
-// Spreading with output ownership.  One workgroup owns an 8^3 block (cells l + nf1/2 in
-// [8 b, 8 b + 8) per axis); in each of its wavefronts lane t owns the x-row
-// (y = t mod 8, z = t / 8) and keeps its 8 cells for SP_LG levels in registers.  The points of
-// the bins that can reach the block (a point of bin c covers cells [l0, l0 + w), l0 in bin c)
-// are taken 64 at a time, batch k by wavefront k mod (wavefronts): each point that meets the block
-// is compacted into the wavefront's LDS buffers with its kernel weights (the x weights
-// expanded to the block's 8 columns, zero outside the support) and its values; then every
-// lane whose row lies inside a point's y/z support adds it to its 8 cells.  The wavefronts'
-// sums are reduced through LDS and the block is written once, times the deconvolution
-// factors, with plain stores: no atomics on the grid, and every cell of [-nf1/2, nf1/2)^3
-// written by exactly one workgroup (no zero pass over the grid).  The sums follow the order
-// of the points inside their bins, which the counting pass ranks in arrival order (the
-// values an atomic counter returns): float images agree between runs to rounding, not bit
-// for bit.
+// Spreading with output ownership.  One wavefront owns an 8^3 block (cells l + nf1/2 in
+// [8 b, 8 b + 8) per axis) or, where blocks are few, one of gridDim.y shares of its points.
+// The points of the bins that can reach the block (a point of bin c covers cells [l0, l0 + w),
+// l0 in bin c) are tested 64 at a time; the ones that meet the block are kept until there are
+// 64 of them, then expanded in LDS: kernel weights of the block's 8 columns, rows and slabs
+// (zero outside the support) and values.
+//
+// Over the points q the block is the product C[(y, z)][(x, re/im), level] =
+// sum_q A[(y, z)][q] B[q][(x, re/im), level] with A = wy wz and B = wx v, taken four points at
+// a time by 16x16x4 matrix instructions: tile m of A holds the rows (y, z = 2 m) and
+// (y, z = 2 m + 1), tile lv of B the level lv, and a lane forms its operands from a few LDS
+// reads.  The 64 points are placed in the order of their first z, so that four neighbours
+// reach about the same z pairs, and the tiles of the others are passed over (about 0.4 of
+// them at w = 6).  The kernel is bound by the matrix instructions (32 cycles each in float,
+// 16 per four points of 4 levels before the passed-over ones) and, behind them, the weights.
+// Measured against sums on the vector ALU (a lane per row, four wavefronts per block, weights
+// for every tested point): 500 samples of 256 antennas, 4 levels, w = 6: 9.43 to 4.27 ms (6.98
+// before the kept points and the z order, 4.62 with three wavefronts per SIMD instead of four);
+// two or four wavefronts per block 5.88 and 5.53 ms against 4.62, their last points filling
+// fewer lanes.  12 samples of 512 antennas, 6 levels in one launch: 10.7 to 3.4 ms.
+//
+// The block is written once, times the deconvolution factors, with plain stores: no atomics on
+// the grid, and every cell of [-nf1/2, nf1/2)^3 written by exactly one wavefront (no zero pass
+// over the grid).  The sums follow the order of the points inside their bins, which the
+// counting pass ranks in arrival order (the values an atomic counter returns): float images
+// agree between runs to rounding, not bit for bit.
 // --------------------------------------------------------------------------------------
-template <typename R>
-struct SpreadBatch {
-  R pwx[64][SP_BIN];      // kernel weight of each block column (x), row (y) and slab (z),
-  R pwy[64][SP_BIN];      // zero outside the point's support
-  R pwz[64][SP_BIN];
-  R pv[64][SP_LG][2];     // values of the levels of this launch
-};
-static_assert(SP_BIN == 8 && SP_LG * 2 == 8, "batch rows are moved as 8 values");
-
-// Rows of 8 values moved with 16-byte LDS accesses: a wavefront's row stores (rows 32 or 64
-// bytes apart) conflict at most 2-way instead of 8-way for 4-byte stores, and a row read
-// is two or four instructions.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef double f64x2 __attribute__((ext_vector_type(2)));
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+template <typename R>
+struct SpreadMfma;
+template <>
+struct SpreadMfma<float> {
+  typedef f32x4 V4;
+  static constexpr int levels = 6;  // most levels per launch: 16 result registers each
+  static __device__ __forceinline__ V4 mul(float a, float b, V4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  // row of result register r in lanes 16 k .. 16 k + 15
+  static __device__ __forceinline__ int row(int k, int r) { return 4 * k + r; }
+};
+template <>
+struct SpreadMfma<double> {
+  typedef f64x4 V4;
+  static constexpr int levels = 4;  // 32 result registers each
+  static __device__ __forceinline__ V4 mul(double a, double b, V4 c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int k, int r) { return k + 4 * r; }
+};
+
+// rows of 8 values moved with 16-byte LDS accesses
 __device__ __forceinline__ void st_row8(float* dst, const float (&v)[8]) {
   reinterpret_cast<f32x4*>(dst)[0] = f32x4{v[0], v[1], v[2], v[3]};
   reinterpret_cast<f32x4*>(dst)[1] = f32x4{v[4], v[5], v[6], v[7]};
 }
 __device__ __forceinline__ void st_row8(double* dst, const double (&v)[8]) {
-#pragma unroll
-  for (int k = 0; k < 4; ++k) reinterpret_cast<f64x2*>(dst)[k] = f64x2{v[2 * k], v[2 * k + 1]};
-}
-__device__ __forceinline__ void ld_row8(const float* src, float (&v)[8]) {
-  const f32x4 a = reinterpret_cast<const f32x4*>(src)[0];
-  const f32x4 b = reinterpret_cast<const f32x4*>(src)[1];
-  v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-  v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-}
-__device__ __forceinline__ void ld_row8(const double* src, double (&v)[8]) {
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const f64x2 a = reinterpret_cast<const f64x2*>(src)[k];
-    v[2 * k] = a.x;
-    v[2 * k + 1] = a.y;
-  }
+  reinterpret_cast<f64x4*>(dst)[0] = f64x4{v[0], v[1], v[2], v[3]};
+  reinterpret_cast<f64x4*>(dst)[1] = f64x4{v[4], v[5], v[6], v[7]};
 }
 
-// wavefronts per spread block (batches split between them); static LDS stays under 64 KiB
-template <typename R>
-struct SpreadWaves {
-  static constexpr int value = sizeof(R) == 8 ? 2 : 4;
+template <typename R, int LG>
+struct SpreadBatch {
+  static constexpr int VS = LG <= 2 ? LG : LG <= 4 ? 4 : 8;  // levels of a row of values
+  R pwx[64][SP_BIN];        // rows from the number of points up to a multiple of 4 are zero
+  R pwy[64][SP_BIN];
+  R pwz[64][SP_BIN];        // [z % 2][z / 2]
+  R pv[64][2][VS];          // re, then im of the levels
+  unsigned pend[128];       // points that meet the block, not yet added
+  unsigned char tiles[64];  // z pairs that the point of a row reaches
 };
 
-template <typename R, typename TV>
-__global__ __launch_bounds__(256) void n3_spread_kernel(N3SpreadParams<R> p) {
-  constexpr int B = SP_BIN, PB = 64, NWV = SpreadWaves<R>::value;
-  // per-wavefront batch buffers; reused at the end for the reduction of the row sums
-  __shared__ __align__(16) union {
-    SpreadBatch<R> batch[NWV];
-    R red[NWV - 1][64][(B / 2) * SP_LG * 2];  // half of a lane's cells at a time
-  } sh;
+// result register r of tile m (s: its levels), deconvolved, into the grid: 16 lanes store
+// consecutive re and im.  Cells outside [-nf1/2, nf1/2)^3 are left out.
+template <typename R, int LG>
+__device__ __forceinline__ void spread_store(const N3SpreadParams<R>& p, const int (&org)[3], int m,
+                                             int r, int lane, const R (&s)[LG]) {
+  const int row = SpreadMfma<R>::row(lane >> 4, r);
+  const int ix = org[0] + ((lane & 15) >> 1), iy = org[1] + (row & 7),
+            iz = org[2] + 2 * m + (row >> 3);
+  if (ix >= p.nf1[0] || iy >= p.nf1[1] || iz >= p.nf1[2]) return;
+  int gx = ix - p.nf1[0] / 2, gy = iy - p.nf1[1] / 2, gz = iz - p.nf1[2] / 2;
+  gx += gx < 0 ? p.nf2[0] : 0;
+  gy += gy < 0 ? p.nf2[1] : 0;
+  gz += gz < 0 ? p.nf2[2] : 0;
+  const R f = p.fx[ix] * (p.fy[iy] * p.fz[iz]);
+  R* g = reinterpret_cast<R*>(p.grid + ((size_t)gz * p.nf2[1] + gy) * p.nf2[0] + gx) + (lane & 1);
+#pragma unroll
+  for (int lv = 0; lv < LG; ++lv)
+    g[2 * (size_t)(p.lv0 - p.lv_begin + lv) * p.grid_stride] = s[lv] * f;
+}
+
+// registers for four wavefronts per SIMD in float up to 4 levels, three above, two in double
+template <typename R, int LG>
+__global__ __launch_bounds__(64, sizeof(R) == 8 ? 2 : LG <= 4 ? 4 : 3) void n3_spread_kernel(N3SpreadParams<R> p) {
+  constexpr int B = SP_BIN, PB = 64;
+  typedef SpreadMfma<R> M;
+  typedef typename M::V4 V4;
+  __shared__ __align__(32) SpreadBatch<R, LG> sb;
   const int w = p.w;
-  const int L = p.n_levels;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  SpreadBatch<R>& sb = sh.batch[wave];
+  const int lane = threadIdx.x;
   // Workgroups go to the 8 XCDs in turn (workgroup i to XCD i mod 8).  With xcd_chunk > 0,
   // runs of xcd_chunk consecutive blocks go to one XCD (neighbouring blocks read overlapping
   // point ranges and then share an L2), the runs dealt to the XCDs in turn.
@@ -469,12 +500,11 @@ __global__ __launch_bounds__(256) void n3_spread_kernel(N3SpreadParams<R> p) {
   const int by = (bin / p.nbins[0]) % p.nbins[1];
   const int bz = bin / (p.nbins[0] * p.nbins[1]);
   const int org[3] = {bx * B, by * B, bz * B};
-  const int cy = lane & 7, cz = lane >> 3;
-  R acc[B][SP_LG][2];
+  V4 acc[4][LG];
 #pragma unroll
-  for (int c = 0; c < B; ++c)
+  for (int m = 0; m < 4; ++m)
 #pragma unroll
-    for (int lv = 0; lv < SP_LG; ++lv) acc[c][lv][0] = acc[c][lv][1] = R(0);
+    for (int lv = 0; lv < LG; ++lv) acc[m][lv] = V4{R(0), R(0), R(0), R(0)};
   const unsigned long long t_start = p.prof ? wall_clock64() : 0;
   unsigned long long n_hit = 0;
   const R two_over_w = R(2) / R(w);
@@ -495,159 +525,173 @@ __global__ __launch_bounds__(256) void n3_spread_kernel(N3SpreadParams<R> p) {
       ++nr;
     }
   const unsigned n_batches = (total_pts + PB - 1) / PB;
-  // wavefronts that own at least one batch (the others reach the barriers below idle)
-  const int n_active = static_cast<int>(min<unsigned>(n_batches, NWV));
-  for (unsigned bi = wave; bi < n_batches; bi += NWV) {
-    const unsigned b0 = bi * PB;
-    const int nb = min<unsigned>(PB, total_pts - b0);
-    bool hit = false;
+  // operand rows and columns of the lane: A row i = lane % 16 is y = i % 8, z = 2 m + i / 8,
+  // B column j = lane % 16 is x = j / 2, re or im = j % 2; both take point q0 + lane / 16
+  const int i16 = lane & 15, kq = lane >> 4;
+
+  // the first `total` (at most 64) pending points added to the sums
+  auto add_pending = [&](int total) {
+    const bool hit = lane < total;
     N3Point pt;
+    cplx<R> vals[LG];
     int rel[3] = {0, 0, 0};
-    TV vals[SP_LG];
-    if (lane < nb) {
-      unsigned v = b0 + lane;
-      int r = 0;
-      while (v >= rlen[r]) v -= rlen[r++];
-      pt = p.pts[rbeg[r] + v];
-      hit = true;
+    if (hit) {
+      const unsigned v = sb.pend[lane];
+      pt = p.pts[v];
+      const cplx<R>* pv = p.vals + (size_t)v * p.n_levels_total + p.lv0;
 #pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        rel[d] = pt.l0[d] - org[d];
-        hit = hit && rel[d] < B && rel[d] + w > 0;
-      }
-      if (hit) {
-        // values first: their latency overlaps the compaction and the kernel weights
-        const TV* pv = p.vals + (size_t)(rbeg[r] + v) * p.n_levels_total + p.lv0;
+      for (int lv = 0; lv < LG; ++lv) vals[lv] = pv[lv];
 #pragma unroll
-        for (int lv = 0; lv < SP_LG; ++lv)
-          if (lv < L) vals[lv] = pv[lv];
+      for (int d = 0; d < 3; ++d) rel[d] = pt.l0[d] - org[d];
+    }
+    // rows in the order of the points' first z: four neighbours then share most z pairs
+    int slot = lane;
+    {
+      unsigned long long left = __ballot(hit);
+      const unsigned long long below = (1ull << lane) - 1ull;
+      int base = 0;
+      for (int z = 1 - w; z < B && left; ++z) {
+        const unsigned long long same = __ballot(hit && rel[2] == z);
+        if (hit && rel[2] == z) slot = base + __popcll(same & below);
+        base += __popcll(same);
+        left &= ~same;
       }
     }
-    const unsigned long long mask = __ballot(hit);
-    const int total = __popcll(mask);
-    const int slot = __popcll(mask & ((1ull << lane) - 1ull));
-    wave_sync();  // the previous batch of this wavefront fully consumed
     if (hit) {
-      R row[3][B];
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
         // column c is support offset o = c - rel of the point, at (o - fr) 2 / w: the
         // argument stepped from c = 0, the support test 0 <= o < w as one unsigned compare
         const R x0 = (R(-rel[d]) - R(pt.fr[d])) * two_over_w;
+        R row[B];
 #pragma unroll
         for (int c = 0; c < B; ++c)
-          row[d][c] = static_cast<unsigned>(c - rel[d]) < static_cast<unsigned>(w)
-                          ? es_kernel<R>(x0 + R(c) * two_over_w, beta)
-                          : R(0);
+          row[d < 2 ? c : (c & 1) * 4 + c / 2] =
+              static_cast<unsigned>(c - rel[d]) < static_cast<unsigned>(w)
+                  ? es_kernel<R>(x0 + R(c) * two_over_w, beta)
+                  : R(0);
+        st_row8(d == 0 ? sb.pwx[slot] : d == 1 ? sb.pwy[slot] : sb.pwz[slot], row);
+        __builtin_amdgcn_sched_barrier(0);  // one row held at a time
       }
-      st_row8(sb.pwx[slot], row[0]);
-      st_row8(sb.pwy[slot], row[1]);
-      st_row8(sb.pwz[slot], row[2]);
+      const int z0 = max(rel[2], 0) >> 1, z1 = min(rel[2] + w - 1, B - 1) >> 1;
+      sb.tiles[slot] = static_cast<unsigned char>((2 << z1) - (1 << z0));
       const R pr = R(pt.ph[0]), pim = R(pt.ph[1]);  // multiplicity included
-      R pvr[SP_LG * 2];
 #pragma unroll
-      for (int lv = 0; lv < SP_LG; ++lv) {
-        if (lv < L) {
-          const TV c = vals[lv];
-          pvr[2 * lv] = R(c.re) * pr - R(c.im) * pim;
-          pvr[2 * lv + 1] = R(c.re) * pim + R(c.im) * pr;
-        } else {
-          pvr[2 * lv] = pvr[2 * lv + 1] = R(0);
-        }
+      for (int lv = 0; lv < LG; ++lv) {
+        sb.pv[slot][0][lv] = vals[lv].re * pr - vals[lv].im * pim;
+        sb.pv[slot][1][lv] = vals[lv].re * pim + vals[lv].im * pr;
       }
-      st_row8(&sb.pv[slot][0][0], pvr);
+    }
+    if (lane >= total && lane < ((total + 3) & ~3)) {
+      const R zero[B] = {R(0), R(0), R(0), R(0), R(0), R(0), R(0), R(0)};
+      st_row8(sb.pwx[lane], zero);
+      st_row8(sb.pwy[lane], zero);
+      st_row8(sb.pwz[lane], zero);
+      sb.tiles[lane] = 0;
+#pragma unroll
+      for (int lv = 0; lv < LG; ++lv) sb.pv[lane][0][lv] = sb.pv[lane][1][lv] = R(0);
     }
     wave_sync();
+    unsigned tiles = reinterpret_cast<const unsigned*>(sb.tiles)[lane & 15];  // four rows
+    tiles |= tiles >> 16;
+    tiles |= tiles >> 8;
     n_hit += total;
-    // Branch-free: rows outside a point's support take weight 0 (the expanded y and z
-    // weights are zero there); two points per iteration keep two load chains in flight.
-    auto row_weight = [&](int q) { return sb.pwy[q][cy] * sb.pwz[q][cz]; };
-    auto add_point = [&](int q, R wyz) {
-      R vr[SP_LG], vi[SP_LG], pvq[SP_LG * 2], wxq[B];
-      ld_row8(&sb.pv[q][0][0], pvq);
-      ld_row8(sb.pwx[q], wxq);
+    for (int q0 = 0; q0 < total; q0 += 4) {
+      const int q = q0 + kq;
+      const unsigned act = __builtin_amdgcn_readlane(tiles, q0 >> 2);
+      const R wy = sb.pwy[q][i16 & 7], wx = sb.pwx[q][i16 >> 1];
+      const V4 wz = *reinterpret_cast<const V4*>(&sb.pwz[q][4 * (i16 >> 3)]);
+      R bv[LG];
 #pragma unroll
-      for (int lv = 0; lv < SP_LG; ++lv) {
-        vr[lv] = pvq[2 * lv] * wyz;
-        vi[lv] = pvq[2 * lv + 1] * wyz;
-      }
+      for (int lv = 0; lv < LG; ++lv) bv[lv] = sb.pv[q][i16 & 1][lv] * wx;
 #pragma unroll
-      for (int cx = 0; cx < B; ++cx) {
-        const R wx = wxq[cx];
+      for (int m = 0; m < 4; ++m) {
+        if (!(act >> m & 1u)) continue;
+        const R a = wy * wz[m];
 #pragma unroll
-        for (int lv = 0; lv < SP_LG; ++lv) {
-          acc[cx][lv][0] += wx * vr[lv];
-          acc[cx][lv][1] += wx * vi[lv];
-        }
-      }
-    };
-    int q = 0;
-    for (; q + 1 < total; q += 2) {
-      const R w0 = row_weight(q), w1 = row_weight(q + 1);
-      add_point(q, w0);
-      add_point(q + 1, w1);
-    }
-    if (q < total) add_point(q, row_weight(q));
-  }
-  // ---- reduce the wavefronts' row sums into wavefront 0, half a row at a time ----------
-  if (n_active > 1) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      // every wavefront is done with its batch buffers (h = 0) or wavefront 0 with the
-      // previous half (h = 1)
-      __syncthreads();
-      if (wave > 0 && wave < n_active) {
-        R* dst = sh.red[wave - 1][lane];
-#pragma unroll
-        for (int c = 0; c < B / 2; ++c)
-#pragma unroll
-          for (int lv = 0; lv < SP_LG; ++lv) {
-            dst[(c * SP_LG + lv) * 2 + 0] = acc[h * (B / 2) + c][lv][0];
-            dst[(c * SP_LG + lv) * 2 + 1] = acc[h * (B / 2) + c][lv][1];
-          }
-      }
-      __syncthreads();
-      for (int k = 0; k < n_active - 1 && wave == 0; ++k) {
-        const R* src = sh.red[k][lane];
-#pragma unroll
-        for (int c = 0; c < B / 2; ++c)
-#pragma unroll
-          for (int lv = 0; lv < SP_LG; ++lv) {
-            acc[h * (B / 2) + c][lv][0] += src[(c * SP_LG + lv) * 2 + 0];
-            acc[h * (B / 2) + c][lv][1] += src[(c * SP_LG + lv) * 2 + 1];
-          }
+        for (int lv = 0; lv < LG; ++lv)
+          acc[m][lv] = M::mul(a, bv[lv], acc[m][lv]);
       }
     }
+    wave_sync();  // rows consumed
+  };
+
+  int n_pend = 0;
+  for (unsigned bi = blockIdx.y; bi < n_batches; bi += gridDim.y) {
+    const unsigned b0 = bi * PB;
+    const int nb = min<unsigned>(PB, total_pts - b0);
+    bool hit = false;
+    unsigned v = b0 + lane;
+    if (lane < nb) {
+      int r = 0;
+      while (v >= rlen[r]) v -= rlen[r++];
+      v += rbeg[r];
+      hit = true;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        const int rel = p.pts[v].l0[d] - org[d];
+        hit = hit && rel < B && rel + w > 0;
+      }
+    }
+    const unsigned long long mask = __ballot(hit);
+    if (hit) sb.pend[n_pend + __popcll(mask & ((1ull << lane) - 1ull))] = v;
+    n_pend += __popcll(mask);
+    wave_sync();
+    if (n_pend >= PB) {
+      add_pending(PB);
+      n_pend -= PB;
+      if (lane < n_pend) {
+        const unsigned t = sb.pend[PB + lane];
+        sb.pend[lane] = t;
+      }
+      wave_sync();
+    }
   }
-  if (wave > 0) return;  // no barrier below: wavefront 0 writes the block
-  if (p.prof && lane == 0) {
+  if (n_pend > 0) add_pending(n_pend);
+  if (p.prof && lane == 0 && blockIdx.y == 0) {
     unsigned long long* pr = p.prof + (size_t)bin * 4;
     pr[0] = t_start;
     pr[1] = wall_clock64();
     pr[2] = total_pts;
-    pr[3] = n_hit;  // hits of wavefront 0
+    pr[3] = n_hit;  // hits of the first share
   }
-  // ---- deconvolve and store the owned cells inside [-nf1/2, nf1/2)^3 ------------------
-  const int iy = org[1] + cy, iz = org[2] + cz;
-  if (iy >= p.nf1[1] || iz >= p.nf1[2]) return;
-  int gy = iy - p.nf1[1] / 2, gz = iz - p.nf1[2] / 2;
-  gy += gy < 0 ? p.nf2[1] : 0;
-  gz += gz < 0 ? p.nf2[2] : 0;
-  const R fyz = p.fy[iy] * p.fz[iz];
+  if (gridDim.y > 1) {  // a share's sums: [block][share][tile][result register][level][lane]
+    R* part = p.part + ((size_t)bin * gridDim.y + blockIdx.y) * (16 * LG * 64) + lane;
 #pragma unroll
-  for (int cx = 0; cx < B; ++cx) {
-    const int ix = org[0] + cx;
-    if (ix >= p.nf1[0]) continue;
-    const R f = p.fx[ix] * fyz;
-    int gx = ix - p.nf1[0] / 2;
-    gx += gx < 0 ? p.nf2[0] : 0;
-    cplx<R>* g = p.grid + ((size_t)gz * p.nf2[1] + gy) * p.nf2[0] + gx;
+    for (int m = 0; m < 4; ++m)
 #pragma unroll
-    for (int lv = 0; lv < SP_LG; ++lv)
-      if (lv < L)
-        g[(size_t)(p.lv0 - p.lv_begin + lv) * p.grid_stride] =
-            mk<R>(acc[cx][lv][0] * f, acc[cx][lv][1] * f);
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int lv = 0; lv < LG; ++lv) part[((m * 4 + r) * LG + lv) * 64] = acc[m][lv][r];
+    return;
   }
+#pragma unroll
+  for (int m = 0; m < 4; ++m)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      R s[LG];
+#pragma unroll
+      for (int lv = 0; lv < LG; ++lv) s[lv] = acc[m][lv][r];
+      spread_store<R, LG>(p, org, m, r, lane, s);
+      __builtin_amdgcn_sched_barrier(0);  // no addresses of later stores held meanwhile
+    }
+}
+
+// sums of the shares of a block (blockIdx.x), in their order: wavefront and blockIdx.y take
+// result register and tile
+template <typename R, int LG>
+__global__ __launch_bounds__(256) void n3_spread_sum_kernel(N3SpreadParams<R> p) {
+  const int bin = blockIdx.x, m = blockIdx.y, lane = threadIdx.x & 63, r = threadIdx.x >> 6;
+  const int org[3] = {bin % p.nbins[0] * SP_BIN, bin / p.nbins[0] % p.nbins[1] * SP_BIN,
+                      bin / (p.nbins[0] * p.nbins[1]) * SP_BIN};
+  const R* part = p.part + (size_t)bin * p.shares * (16 * LG * 64) + (m * 4 + r) * LG * 64 + lane;
+  R s[LG];
+#pragma unroll
+  for (int lv = 0; lv < LG; ++lv) s[lv] = R(0);
+  for (int k = 0; k < p.shares; ++k)
+#pragma unroll
+    for (int lv = 0; lv < LG; ++lv) s[lv] += part[(size_t)k * (16 * LG * 64) + lv * 64];
+  spread_store<R, LG>(p, org, m, r, lane, s);
 }
 
 // --------------------------------------------------------------------------------------
@@ -1717,7 +1761,41 @@ void launch_scan(const unsigned* in, unsigned* out, unsigned* tmp, int n, hipStr
 }
 
 
-template <typename R, typename TV>
+namespace {
+template <typename R, int LG>
+void spread_blocks(const N3SpreadParams<R>& p, unsigned blocks, unsigned grid, hipStream_t st) {
+  if constexpr (LG > SpreadMfma<R>::levels) {
+    fail(BIPP_INTERNAL_ERROR, "NUFFT spread level count");
+  } else {
+    n3_spread_kernel<R, LG><<<dim3(grid, p.shares), 64, 0, st>>>(p);
+    check_launch("n3_spread_kernel");
+    if (p.shares > 1) {
+      n3_spread_sum_kernel<R, LG><<<dim3(blocks, 4), 256, 0, st>>>(p);
+      check_launch("n3_spread_sum_kernel");
+    }
+  }
+}
+}  // namespace
+
+int n3_spread_shares(long long n_blocks, const int (&nback)[3], long long n_points) {
+  // Few blocks: their points shared until about 4096 wavefronts (four per SIMD) run or a share
+  // gets fewer than 4 batches of points on average; its sums cost a write and a read of 16 to
+  // 24 KiB.  50 samples of 60 antennas in double precision: 395 us with up to 2048, 220 + 30 us
+  // (the sum) with 4096, 201 + 39 us with 8192; 40 samples of 96 antennas in float, 4096
+  // blocks and more: 97 us without shares, 84 + 72 us with 8192.
+  const long long reach = n_points * (nback[0] + 1) * (nback[1] + 1) * (nback[2] + 1);
+  const long long most = reach / (n_blocks * 256);
+  return static_cast<int>(std::max(1LL, std::min({(4096 + n_blocks - 1) / n_blocks, most, 256LL})));
+}
+
+template <typename R>
+size_t n3_spread_part_elems(long long n_blocks, int shares, int levels) {
+  return (size_t)n_blocks * shares * 1024 * std::min(levels, SpreadMfma<R>::levels);
+}
+template size_t n3_spread_part_elems<float>(long long, int, int);
+template size_t n3_spread_part_elems<double>(long long, int, int);
+
+template <typename R>
 void launch_n3_spread(const N3SpreadParams<R>& p_all, hipStream_t st) {
   const long long n_blocks = (long long)p_all.nbins[0] * p_all.nbins[1] * p_all.nbins[2];
   if (n_blocks <= 0) return;
@@ -1727,23 +1805,36 @@ void launch_n3_spread(const N3SpreadParams<R>& p_all, hipStream_t st) {
     if (p_all.bin_size[d] != SP_BIN || (long long)p_all.nbins[d] * SP_BIN < p_all.nf1[d] ||
         p_all.nback[d] < 0 || p_all.nback[d] > 2)
       fail(BIPP_INTERNAL_ERROR, "NUFFT spread blocks do not cover the grid");
-  // SP_LG levels per launch (the sums of a lane's 8 cells live in registers)
   if (p_all.lv_begin < 0 || p_all.lv_end > p_all.n_levels_total || p_all.lv_begin >= p_all.lv_end)
     fail(BIPP_INTERNAL_ERROR, "NUFFT spread level range");
-  for (int lv0 = p_all.lv_begin; lv0 < p_all.lv_end; lv0 += SP_LG) {
+  if (p_all.shares < 1 || (p_all.shares > 1 && !p_all.part))
+    fail(BIPP_INTERNAL_ERROR, "NUFFT spread shares");
+  // the levels in launches of equal size, at most as many as a kernel keeps sums for
+  constexpr int most = SpreadMfma<R>::levels;
+  const int n_all = p_all.lv_end - p_all.lv_begin;
+  const int launches = (n_all + most - 1) / most;
+  const int per = (n_all + launches - 1) / launches;
+  for (int lv0 = p_all.lv_begin; lv0 < p_all.lv_end; lv0 += per) {
     N3SpreadParams<R> p = p_all;
     p.lv0 = lv0;
-    p.n_levels = std::min(SP_LG, p_all.lv_end - lv0);
+    p.n_levels = std::min(per, p_all.lv_end - lv0);
     // with the XCD order (see the kernel), a multiple of 8 chunks of workgroups; the extra
     // ones exit
     const long long unit = p.xcd_chunk > 0 ? 8LL * p.xcd_chunk : 1;
     const long long grid = (n_blocks + unit - 1) / unit * unit;
-    n3_spread_kernel<R, TV><<<static_cast<unsigned>(grid), 64 * SpreadWaves<R>::value, 0, st>>>(p);
-    check_launch("n3_spread_kernel");
+    const unsigned nb = static_cast<unsigned>(n_blocks), ng = static_cast<unsigned>(grid);
+    switch (p.n_levels) {
+      case 1: spread_blocks<R, 1>(p, nb, ng, st); break;
+      case 2: spread_blocks<R, 2>(p, nb, ng, st); break;
+      case 3: spread_blocks<R, 3>(p, nb, ng, st); break;
+      case 4: spread_blocks<R, 4>(p, nb, ng, st); break;
+      case 5: spread_blocks<R, 5>(p, nb, ng, st); break;
+      default: spread_blocks<R, 6>(p, nb, ng, st); break;
+    }
   }
 }
-template void launch_n3_spread<float, cplx<float>>(const N3SpreadParams<float>&, hipStream_t);
-template void launch_n3_spread<double, cplx<double>>(const N3SpreadParams<double>&, hipStream_t);
+template void launch_n3_spread<float>(const N3SpreadParams<float>&, hipStream_t);
+template void launch_n3_spread<double>(const N3SpreadParams<double>&, hipStream_t);
 
 namespace {
 bool window_ok(const N3Window& w, int n) {

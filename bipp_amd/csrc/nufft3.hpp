@@ -129,6 +129,8 @@ struct N3SpreadParams {
   // optional per-block profile [n_blocks][4]: start, end (wall clock), points, items
   unsigned long long* prof;
   int xcd_chunk;                 // blocks per XCD run (0: blocks in launch order)
+  int shares;                    // wavefronts per block (n3_spread_shares)
+  R* part;                       // their sums (n3_spread_part_elems values) if more than one
 };
 
 // Window of an axis of length n: indices (start + i) mod n for i < count.
@@ -254,7 +256,10 @@ template <typename R>
 void launch_zero(R* p, long long n, hipStream_t st);
 void launch_n3_points(const N3PointsParams& p, int n_samples, hipStream_t st);
 void launch_scan(const unsigned* in, unsigned* out, unsigned* tmp, int n, hipStream_t st);
-template <typename R, typename TV>
+int n3_spread_shares(long long n_blocks, const int (&nback)[3], long long n_points);
+template <typename R>
+size_t n3_spread_part_elems(long long n_blocks, int shares, int levels);
+template <typename R>
 void launch_n3_spread(const N3SpreadParams<R>& p, hipStream_t st);
 template <typename R>
 void launch_fft_lines(const N3LineParams<R>& p, hipStream_t st);

@@ -552,9 +552,10 @@ inline void report_spread_profile(const unsigned long long* dprof, long long nb,
 template <typename TG>
 struct N3Runner {
   DevBuf grid, sorted, sorted_vals;
-  DevBuf bin_count, bin_start, bin_rank, scan_tmp, vv, deconv, gl, twid, prof_buf;
+  DevBuf bin_count, bin_start, bin_rank, scan_tmp, vv, deconv, gl, twid, prof_buf, part_buf;
   DevBuf group_of, group_count, group_start, group_fill, group_tmp, slot_list, ranges;
   DevBuf direct_part;
+  long long n_points = 0;  // slots of the transform under way
   std::vector<cplx<TG>> htw;
   std::vector<TG> hdec;
   N3Plan plan;
@@ -816,7 +817,7 @@ struct N3Runner {
     N3PointsParams pp;
     pp.src = src;
     pp.slot_list = list;
-    pp.n_list = n_list;
+    pp.n_list = n_points = n_list;
     for (int d = 0; d < 3; ++d) {
       pp.C[d] = pl.C[d];
       pp.D[d] = pl.D[d];
@@ -955,7 +956,9 @@ struct N3Runner {
     const bool prof = std::getenv("BIPP_N3_PROFILE") != nullptr;
     sp.prof = prof ? prof_buf.as<unsigned long long>((size_t)nb * 4) : nullptr;
     if (prof) BIPP_HIP(hipMemsetAsync(sp.prof, 0, sizeof(unsigned long long) * nb * 4, st));
-    launch_n3_spread<TG, cplx<TG>>(sp, st);
+    sp.shares = n3_spread_shares(nb, sp.nback, n_points);
+    sp.part = sp.shares > 1 ? part_buf.as<TG>(n3_spread_part_elems<TG>(nb, sp.shares, lg)) : nullptr;
+    launch_n3_spread<TG>(sp, st);
     if (prof) report_spread_profile(sp.prof, nb, pl, st);
   }
 
