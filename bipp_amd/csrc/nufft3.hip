@@ -1273,6 +1273,130 @@ __global__ __launch_bounds__(FFT_NT) void fft_pass_rr_kernel(N3PassParams<R> p, 
   }
 }
 
+// Strided axis of n = n1 n2 points in one pass (the two passes' transforms, windows and output
+// order): 2^tw_shift x positions per workgroup, their lines in LDS between up to four stages of
+// radix r[s] in place, X[K], K = f0 + r0 (f1 + r1 (f2 + ...)), at f0 S0 + f1 S1 + ... with
+// S_s = n / (r0 ... r_s).  The first stage loads from global memory, inside the input window,
+// and the last one stores the frequencies of the output window, so the unpruned middle of the
+// two passes, twice the windows' size each way, stays in the CU.
+// Workgroup i of a round runs on XCD i mod 8 and the tiles of a round are dealt to the XCDs in
+// runs: neighbouring tiles share 128-byte lines (a tile of 4 positions has 32 bytes of each).
+// Bound by LDS exchanges and the transforms' arithmetic between barriers, behind them HBM (7 GB
+// at configuration 4).  500 samples of 256 antennas, y axis of 3456 points, 4 levels: 3.9 + 3.0
+// ms in two passes, 3.7 ms in one (4.3 ms with 512 threads).
+template <typename R, int NT, int RAD, bool FIRST, bool LAST>
+__device__ __forceinline__ void axis_stage(const N3AxisParams<R>& p, int s, cplx<R>* lds, const Twid<R>& tw,
+                                           cplx<R>* base, int xt, int tid) {
+  const int tws = p.tw_shift, TW = 1 << tws;
+  const int S = p.span[s], items = (p.n / RAD) << tws;
+  for (int u = tid; u < items; u += NT) {
+    const int xi = u & (TW - 1), t = u >> tws;
+    const int hi = LAST ? t : FIRST ? 0 : fast_div(t, p.sp_m[s], p.sp_s[s]);
+    const int lo = LAST ? 0 : t - hi * S;
+    cplx<R>* line = lds + xi * p.ld + hi * (RAD * S) + lo;
+    const int j = (xt << tws) + xi;
+    int x = p.xw.start + j;
+    x -= x >= p.nx ? p.nx : 0;
+    cplx<R> v[RAD];
+    if constexpr (FIRST) {
+#pragma unroll
+      for (int r = 0; r < RAD; ++r) {
+        const int ai = lo + r * S;
+        v[r] = j < p.xw.count && in_window(ai, p.in, p.n) ? base[(long long)ai * p.axis_stride + x]
+                                                          : mk<R>(0, 0);
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < RAD; ++r) v[r] = line[r * S];
+    }
+    dft_small<R, RAD>(v);
+    if constexpr (LAST) {
+      if (j >= p.xw.count) continue;
+      // digits of the position hi RAD: the frequency of output 0
+      int K = 0, rest = hi * RAD;
+      for (int q = 0; q < s; ++q) {
+        const int f = fast_div(rest, p.sp_m[q], p.sp_s[q]);
+        rest -= f * p.span[q];
+        K += f * p.weight[q];
+      }
+      const int q0 = fast_div(K, p.n1_m, p.n1_s), row = (K - q0 * p.n1) * p.n2 + q0;
+#pragma unroll
+      for (int r = 0; r < RAD; ++r)
+        if (in_window(K + r * p.weight[s], p.out, p.n))
+          base[(long long)(row + r * p.last_step) * p.axis_stride + x] = v[r];
+    } else {
+      const int t1 = lo * p.weight[s];  // w_(RAD S)^lo = w_n^t1
+      cplx<R> wp[RAD];
+      wp[1] = tw(t1);
+      if constexpr (RAD > 2) wp[2] = wp[1] * wp[1];
+      if constexpr (RAD > 3) wp[3] = wp[2] * wp[1];
+      if constexpr (RAD > 4) {
+        wp[4] = tw(4 * t1);
+#pragma unroll
+        for (int r = 5; r < RAD && r < 8; ++r) wp[r] = wp[4] * wp[r - 4];
+      }
+      if constexpr (RAD > 8) {
+        wp[8] = tw(8 * t1);
+#pragma unroll
+        for (int r = 9; r < RAD; ++r) wp[r] = wp[8] * wp[r - 8];
+      }
+      line[0] = v[0];
+#pragma unroll
+      for (int r = 1; r < RAD; ++r) line[r * S] = v[r] * wp[r];
+    }
+  }
+}
+
+template <typename R, int NT, bool FIRST, bool LAST>
+__device__ __forceinline__ void axis_radix(const N3AxisParams<R>& p, int s, cplx<R>* lds, const Twid<R>& tw,
+                                           cplx<R>* base, int xt, int tid) {
+  switch (p.r[s]) {
+    case 2: axis_stage<R, NT, 2, FIRST, LAST>(p, s, lds, tw, base, xt, tid); break;
+    case 3: axis_stage<R, NT, 3, FIRST, LAST>(p, s, lds, tw, base, xt, tid); break;
+    case 4: axis_stage<R, NT, 4, FIRST, LAST>(p, s, lds, tw, base, xt, tid); break;
+    case 5: axis_stage<R, NT, 5, FIRST, LAST>(p, s, lds, tw, base, xt, tid); break;
+    case 6: axis_stage<R, NT, 6, FIRST, LAST>(p, s, lds, tw, base, xt, tid); break;
+    case 8: axis_stage<R, NT, 8, FIRST, LAST>(p, s, lds, tw, base, xt, tid); break;
+    case 9: axis_stage<R, NT, 9, FIRST, LAST>(p, s, lds, tw, base, xt, tid); break;
+    case 10: axis_stage<R, NT, 10, FIRST, LAST>(p, s, lds, tw, base, xt, tid); break;
+    case 12: axis_stage<R, NT, 12, FIRST, LAST>(p, s, lds, tw, base, xt, tid); break;
+    case 15: axis_stage<R, NT, 15, FIRST, LAST>(p, s, lds, tw, base, xt, tid); break;
+    default: axis_stage<R, NT, 16, FIRST, LAST>(p, s, lds, tw, base, xt, tid); break;
+  }
+}
+
+template <typename R, int NT>
+__global__ __launch_bounds__(NT) void fft_axis_kernel(N3AxisParams<R> p) {
+  extern __shared__ __align__(16) unsigned char fsh[];
+  cplx<R>* lds = reinterpret_cast<cplx<R>*>(fsh);
+  const int tid = threadIdx.x;
+  const Twid<R> tw = load_twid<R>(p.tw, p.n, lds + ((size_t)p.ld << p.tw_shift), tid, NT);
+  __syncthreads();
+  const int n_xt = (p.xw.count + (1 << p.tw_shift) - 1) >> p.tw_shift;
+  const int n_items = n_xt * p.other.count * p.n_levels;
+  const int at = gridDim.x % 8 == 0 ? (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8 : blockIdx.x;
+  for (int item = at; item < n_items; item += gridDim.x) {
+    const int q1 = fast_div(item, p.xt_m, p.xt_s);
+    const int xt = item - q1 * n_xt;
+    const int lv = fast_div(q1, p.oc_m, p.oc_s);
+    int oo = p.other.start + q1 - lv * p.other.count;
+    oo -= oo >= p.no ? p.no : 0;
+    if (p.operm_n2 > 1) {
+      const int q = fast_div(oo, p.op_m, p.op_s);
+      oo = (oo - q * p.operm_n1) * p.operm_n2 + q;
+    }
+    cplx<R>* base = p.grid + (size_t)lv * p.grid_stride + (size_t)oo * p.outer_stride;
+    axis_radix<R, NT, true, false>(p, 0, lds, tw, base, xt, tid);
+    for (int s = 1; s < p.stages - 1; ++s) {
+      __syncthreads();
+      axis_radix<R, NT, false, false>(p, s, lds, tw, base, xt, tid);
+    }
+    __syncthreads();
+    axis_radix<R, NT, false, true>(p, p.stages - 1, lds, tw, base, xt, tid);
+    __syncthreads();  // lines read before the next tile's first stage
+  }
+}
+
 // --------------------------------------------------------------------------------------
 // Interpolation at the pixels, correction, real part accumulated into the images.
 // --------------------------------------------------------------------------------------
@@ -1955,6 +2079,73 @@ bool fft_rr_factors(int m, int& m1, int& m2) {
 #undef BIPP_RR_FIND
   return found;
 }
+
+// x positions per workgroup of the one-pass form as a power of two, or -1.  Up to 16 where two
+// workgroups of 512 threads fit a CU, down to 2 with one of 1024 (rows of 16 bytes in float, the
+// rest of a line is its neighbours' on the same XCD); two positions are still faster than two
+// passes (the 512-antenna case's axes of 6000 to 6912 points 10.0 to 7.3 ms), 8 positions in half
+// a CU's LDS than in all of it (121 against 126 us at 40 samples of 96 antennas).
+int fft_axis_shift(int n, size_t elem) {
+  for (int k = 4; k >= 1; --k)
+    if (elem * ((size_t)(n + 32) << k) <= (k >= 3 ? 76 : 152) * 1024) return k;
+  return -1;
+}
+
+template <typename R>
+bool launch_fft_axis(const N3AxisParams<R>& p_in, hipStream_t st) {
+  N3AxisParams<R> p = p_in;
+  int f[4];
+  if (p.n2 < 2 || (long long)p.n1 * p.n2 != p.n || !fft_rr_factors(p.n1, f[0], f[1]) ||
+      !fft_rr_factors(p.n2, f[2], f[3]))
+    return false;
+  p.tw_shift = fft_axis_shift(p.n, sizeof(cplx<R>));
+  if (p.tw_shift < 0) return false;
+  if (!window_ok(p.xw, p.nx) || !window_ok(p.other, p.no) || !window_ok(p.in, p.n) ||
+      !window_ok(p.out, p.n))
+    fail(BIPP_INTERNAL_ERROR, "FFT pass windows out of range");
+  p.stages = 0;
+  int done = 1;
+  for (int k = 0; k < 4; ++k) {
+    if (f[k] == 1) continue;
+    const int s = p.stages++;
+    p.r[s] = f[k];
+    p.weight[s] = done;
+    done *= f[k];
+    p.span[s] = p.n / done;
+    n3_div_magic(p.span[s], p.sp_m[s], p.sp_s[s]);
+  }
+  p.last_step = p.weight[p.stages - 1] / p.n1;
+  n3_div_magic(p.n1, p.n1_m, p.n1_s);
+  // line stride 32 / positions modulo 32 elements: a row of positions in different banks
+  const int want = 32 >> p.tw_shift;
+  p.ld = p.n + ((want - p.n) % 32 + 32) % 32;
+  const int TW = 1 << p.tw_shift;
+  const long long items = (long long)((p.xw.count + TW - 1) / TW) * p.other.count * p.n_levels;
+  if (items <= 0) return true;
+  if (items > 0x7fffffffLL) fail(BIPP_INVALID_PARAMETER_ERROR, "NUFFT grid too large for one pass");
+  n3_div_magic((p.xw.count + TW - 1) / TW, p.xt_m, p.xt_s);
+  n3_div_magic(p.other.count, p.oc_m, p.oc_s);
+  n3_div_magic(p.operm_n2 > 1 ? p.operm_n1 : 1, p.op_m, p.op_s);
+  const size_t sh = sizeof(cplx<R>) * (((size_t)p.ld << p.tw_shift) + twid_len(p.n));
+  if (sh > 159 * 1024) fail(BIPP_INTERNAL_ERROR, "FFT pass exceeds LDS");
+  auto go = [&](auto kernel, int nt) {
+    static const hipError_t attr =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, 159 * 1024);
+    hip_check(attr, "hipFuncSetAttribute");
+    // a round is one tile per resident workgroup
+    const long long round = sh <= 39 * 1024 ? 1024 : sh <= 79 * 1024 ? 512 : 256;
+    kernel<<<static_cast<unsigned>(std::min(items, round)), nt, sh, st>>>(p);
+  };
+  if (sh <= 79 * 1024)
+    go(&fft_axis_kernel<R, 512>, 512);
+  else
+    go(&fft_axis_kernel<R, 1024>, 1024);
+  check_launch("fft_axis_kernel");
+  return true;
+}
+template bool launch_fft_axis<float>(const N3AxisParams<float>&, hipStream_t);
+template bool launch_fft_axis<double>(const N3AxisParams<double>&, hipStream_t);
 
 template <typename R>
 void launch_fft_pass(const N3PassParams<R>& p_in, hipStream_t st) {

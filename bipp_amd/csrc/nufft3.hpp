@@ -185,6 +185,30 @@ struct N3PassParams {
   int xt_s, sub_s, oc_s, op_s;
 };
 
+// One-pass transform of a strided axis of n = n1 n2 points (fft_axis_kernel): fields as
+// N3PassParams; frequency k inside `out` is stored at (k mod n1) n2 + k / n1.
+template <typename R>
+struct N3AxisParams {
+  cplx<R>* grid;
+  long long grid_stride;
+  int n_levels;
+  int nx;
+  N3Window xw;
+  int no;
+  N3Window other;
+  int operm_n1, operm_n2;
+  long long outer_stride, axis_stride;
+  int n, n1, n2;
+  N3Window in, out;
+  const cplx<R>* tw;             // exp(+2 pi i t / n), t < n
+  // set by the launcher: stages (radix, span below the digit, weight of the digit in the
+  // frequency), row step of the last stage's outputs, line stride, division constants
+  int stages, tw_shift, ld, last_step;
+  int r[4], span[4], weight[4];
+  unsigned sp_m[4], n1_m, xt_m, oc_m, op_m;
+  int sp_s[4], n1_s, xt_s, oc_s, op_s;
+};
+
 template <typename R>
 struct N3InterpParams {
   int n_pix, n_levels, w1, w2;
@@ -265,6 +289,9 @@ template <typename R>
 void launch_fft_lines(const N3LineParams<R>& p, hipStream_t st);
 template <typename R>
 void launch_fft_pass(const N3PassParams<R>& p, hipStream_t st);
+// false: no form of this length, nothing launched
+template <typename R>
+bool launch_fft_axis(const N3AxisParams<R>& p, hipStream_t st);
 // m = m1 m2 with (m1, m2) a factor pair of the two-stage register pass (m1 >= m2)
 bool fft_rr_factors(int m, int& m1, int& m2);
 template <typename R, typename TI>

@@ -962,6 +962,30 @@ struct N3Runner {
     if (prof) report_spread_profile(sp.prof, nb, pl, st);
   }
 
+  // the axis of a pass in one launch, where its lines fit LDS; tw: roots of its length
+  template <typename R>
+  static bool fft_one_pass(const N3PassParams<R>& fp, int n1, int n2, const cplx<R>* tw, hipStream_t st) {
+    N3AxisParams<R> ap{};
+    ap.grid = fp.grid;
+    ap.grid_stride = fp.grid_stride;
+    ap.n_levels = fp.n_levels;
+    ap.nx = fp.nx;
+    ap.xw = fp.xw;
+    ap.no = fp.no;
+    ap.other = fp.other;
+    ap.operm_n1 = fp.operm_n1;
+    ap.operm_n2 = fp.operm_n2;
+    ap.outer_stride = fp.outer_stride;
+    ap.axis_stride = fp.axis_stride;
+    ap.n = fp.nax;
+    ap.n1 = n1;
+    ap.n2 = n2;
+    ap.in = fp.in;
+    ap.out = fp.out;
+    ap.tw = tw;
+    return launch_fft_axis<R>(ap, st);
+  }
+
   // pruned FFT (sign +) along x, y, z of lg level grids
   void fft_group(const N3Plan& pl, int lg, cplx<TG>* cg, const N3Tuning& cfg, hipStream_t st) {
     const long long G = pl.grid_cells;
@@ -1030,6 +1054,7 @@ struct N3Runner {
         fp.tw = dtw + tw_off[d][0];
         fp.tw2 = nullptr;
         launch_fft_pass<TG>(fp, st);
+      } else if (cfg.pass_rr && fft_one_pass<TG>(fp, n1, n2, dtw + tw_off[d][2], st)) {
       } else {
         // n = n1 n2: transforms of length n1 over stride n2 (inputs pruned), twiddle, then
         // transforms of length n2 over contiguous runs (outputs pruned); frequency k is

@@ -44,3 +44,42 @@ def test_fft_lengths(ctx, length):
     err = O.rel_l2(syn.images()[0], ref[0])
     print(f"grid {syn.nufft_grid()} {compute}: rel L2 {err:.2e}", flush=True)
     assert err <= bound     # the bound of the other mixed NUFFT tests
+
+
+@pytest.mark.parametrize("compute,length", [("mixed", 576), ("mixed", 600), ("mixed", 1152),
+                                            ("mixed", 1200), ("mixed", 4800), ("mixed", 5000),
+                                            ("mixed", 9600), ("mixed", 10000), ("fp64", 240),
+                                            ("fp64", 288), ("fp64", 576), ("fp64", 600),
+                                            ("fp64", 2400), ("fp64", 2500), ("fp64", 4800),
+                                            ("fp64", 5000)])
+def test_fft_axis_lengths(ctx, compute, length):
+    """The y axis in one pass on both sides of the lengths at which its tile halves (16, 8, 4
+    and 2 positions, then two passes), an array stretched along y."""
+    tol = 1e-5 if compute == "mixed" else 1e-9
+    # mixed: the bound of the other tests.  fp64: the points' offsets are held in 32 bits, half a
+    # unit in the last place below 16 cells is 4.8e-7 cells of at most pi / 2 of phase: 7.5e-7
+    bound = 1e-4 if compute == "mixed" else 7.5e-7
+    r = np.random.default_rng(length)
+    n = 9
+    src, flux = synthetic.zenith_cap_sources(r, 5, 5.0)
+    p0 = synthetic.disk_positions(r, n, 1.0) + np.array([0, 0, 0.3]) * r.normal(size=(n, 1))
+    lmn = synthetic.make_lmn_grid(21, math.radians(20))
+    w = math.ceil(math.log10(1 / tol)) + 1
+    a, b = np.tril_indices(n)
+    u = 2 * np.pi * (p0[a, 1] - p0[b, 1])
+    xs = 0.5 * (u.max() - u.min()) * 0.5 * (lmn[:, 1].max() - lmn[:, 1].min())
+    for want in np.arange(length / 2, length / 2 * 0.9 - 12, -length / 400):
+        scale = (want - w - 1) / (4 / math.pi * xs)
+        xyz = p0 * np.array([5.0, scale, 2.0])
+        s = synthetic.visibilities(xyz, 1.0, src, flux, 0.1)
+        syn = bipp_amd.NufftSynthesis(ctx, n, n, [[0.0, 3e38]], lmn, compute=compute,
+                                      imager="nufft", tolerance=tol)
+        syn.collect(1.0, s, xyz)
+        if syn.nufft_grid()[1] == length:
+            break
+    assert syn.nufft_grid()[1] == length
+    ref, _ = O.synthesize([synthetic.Sample(0, 0, 1.0, xyz, s, np.ones(n, bool))],
+                          np.array([[0.0, 3e38]]), lmn)
+    err = O.rel_l2(syn.images()[0], ref[0])
+    print(f"grid {syn.nufft_grid()} {compute}: rel L2 {err:.2e}", flush=True)
+    assert err <= bound
