@@ -92,18 +92,21 @@ struct CiValuTile {
 // krange(i0, j0, klo, khi) bounds the k of a tile; store(i, j, acc) writes a result.
 // B_KFAST: consecutive k of B are contiguous in memory (else consecutive j), which sets how
 // the threads split a tile load.  The arithmetic is the team's tile type (Team::CiTile);
-// the next k chunk is loaded into registers while the current one is used.  Ends with a
-// barrier (the stores are visible to the next product).
+// the next k chunk is loaded into registers while the current one is used.  Only the tiles
+// first, first + step, .. of the sequence are formed (several teams may share a product).  Ends
+// with a barrier (the stores are visible to the team's next product).
 template <typename R, int NT, bool LOWER, bool B_KFAST, class Team, class FA, class FB, class KR,
           class ST>
 BIPP_HD void ci_gemm(Team& tm, int m, int nn, FA fa, FB fb, KR krange, ST store,
-                     CiShared<R>& sh) {
+                     CiShared<R>& sh, int first = 0, int step = 1) {
   constexpr int PER = CI_T * CI_K / NT;
   static_assert(PER * NT == CI_T * CI_K, "tile loads split over NT");
   const int tid = tm.tid;
   const int ntr = (m + CI_T - 1) / CI_T, ntc = (nn + CI_T - 1) / CI_T;
+  int at = 0;
   for (int tj = 0; tj < ntc; ++tj) {
-    for (int ti = LOWER ? tj : 0; ti < ntr; ++ti) {
+    for (int ti = LOWER ? tj : 0; ti < ntr; ++ti, ++at) {
+      if (at < first || (at - first) % step) continue;
       const int i0 = ti * CI_T, j0 = tj * CI_T;
       int klo = 0, khi = 0;
       krange(i0, j0, klo, khi);
@@ -143,6 +146,163 @@ BIPP_HD void ci_gemm(Team& tm, int m, int nn, FA fa, FB fb, KR krange, ST store,
   tm.sync();
 }
 
+// The steps of chol_inverse; `first` and `step` select the tiles of a product (ci_gemm).
+
+// Diagonal block of columns [j0, j0 + CI_CB): factored and inverted in LDS, the inverse W_JJ
+// stored over it.  Returns -1, or the column whose pivot is not positive.
+template <typename R, int NT, class Team>
+BIPP_HD int chol_diagonal(Team& tm, int n, int j0, BIPP_GLOBAL cplx<R>* L, int ld, CiShared<R>& sh) {
+  const int tid = tm.tid;
+  auto at = [=](int i, int j) -> BIPP_GLOBAL cplx<R>& { return L[i + (long long)j * ld]; };
+  const int jb = n - j0 < CI_CB ? n - j0 : CI_CB;
+  for (int e = tid; e < CI_CB * CI_CB; e += NT) {
+    const int i = e % CI_CB, j = e / CI_CB;
+    sh.blk.d[i][j] = (i < jb && i >= j) ? ci_get(at(j0 + i, j0 + j)) : mk<R>(0, 0);
+  }
+  tm.sync();
+  // step k: pivot d_kk (final after step k - 1), trailing columns updated with the
+  // unscaled column k, column k - 1 scaled (nothing reads it in this step)
+  R p_prev = R(1);
+  int fail = -1;
+  for (int k = 0; k < jb; ++k) {
+    const R p = sh.blk.d[k][k].re;
+    if (!(p > R(0) && p == p)) {
+      fail = k;
+      break;
+    }
+    const R ip = R(1) / p;
+    for (int e = tid; e < CI_CB * CI_CB; e += NT) {
+      const int i = e % CI_CB, j = e / CI_CB;
+      if (j > k && i >= j && i < jb)
+        sh.blk.d[i][j] = sh.blk.d[i][j] - sh.blk.d[i][k] * conj(sh.blk.d[j][k]) * ip;
+    }
+    if (k > 0) {
+      const R s = sqrt(p_prev), is = R(1) / s;
+      for (int i = k - 1 + tid; i < jb; i += NT)
+        sh.blk.d[i][k - 1] = i == k - 1 ? mk<R>(s, R(0)) : sh.blk.d[i][k - 1] * is;
+    }
+    p_prev = p;
+    tm.sync();
+  }
+  if (fail >= 0) return j0 + fail;
+  {
+    const int k = jb - 1;
+    const R s = sqrt(p_prev), is = R(1) / s;
+    for (int i = k + tid; i < jb; i += NT)
+      sh.blk.d[i][k] = i == k ? mk<R>(s, R(0)) : sh.blk.d[i][k] * is;
+  }
+  tm.sync();
+  tm.mark(0);
+  // inverse W = L^-1, right-looking over the whole team: a[i][j] = delta_ij - sum_{m < i}
+  // L_im W_mj with W_mj = a[m][j] / L_mm, accumulated one pivot m per step (the elements
+  // of a step spread over the team); then W_ij = a[i][j] / L_ii
+  for (int e = tid; e < CI_CB * CI_CB; e += NT) {
+    const int i = e % CI_CB, j = e / CI_CB;
+    if (i < jb && i >= j) sh.blk.w[i][j] = mk<R>(i == j ? R(1) : R(0), R(0));
+  }
+  tm.sync();
+  for (int m = 0; m + 1 < jb; ++m) {
+    const R im = R(1) / sh.blk.d[m][m].re;
+    for (int e = tid; e < CI_CB * CI_CB; e += NT) {
+      const int i = e % CI_CB, j = e / CI_CB;
+      if (i > m && i < jb && j <= m)
+        sh.blk.w[i][j] = sh.blk.w[i][j] - sh.blk.d[i][m] * (sh.blk.w[m][j] * im);
+    }
+    tm.sync();
+  }
+  for (int e = tid; e < CI_CB * CI_CB; e += NT) {
+    const int i = e % CI_CB, j = e / CI_CB;
+    if (i < jb && i >= j) sh.blk.w[i][j] = sh.blk.w[i][j] * (R(1) / sh.blk.d[i][i].re);
+  }
+  tm.sync();
+  for (int e = tid; e < CI_CB * CI_CB; e += NT) {
+    const int i = e % CI_CB, j = e / CI_CB;
+    if (i < jb && i >= j) ci_put(at(j0 + i, j0 + j), sh.blk.w[i][j]);
+  }
+  tm.sync();
+  return -1;
+}
+
+template <typename R, int NT, class Team>
+BIPP_HD void chol_panel(Team& tm, int n, int j0, BIPP_GLOBAL cplx<R>* L, int ld, CiShared<R>& sh,
+                        int first = 0, int step = 1) {
+  const int jb = CI_CB, r0 = j0 + jb, mp = n - r0;
+  if (mp <= 0) return;
+  // L_{>J,J} = G_{>J,J} W_JJ^H in place (a tile reads its rows' k < jb before it stores)
+  ci_gemm<R, NT, false, false>(
+      tm, mp, jb, [=](int i, int k) { return ci_get(L[(r0 + i) + (long long)(j0 + k) * ld]); },
+      [=](int k, int j) {
+        return k <= j ? conj(ci_get(L[(j0 + j) + (long long)(j0 + k) * ld])) : mk<R>(0, 0);
+      },
+      [=](int, int, int& klo, int& khi) {
+        klo = 0;
+        khi = jb;
+      },
+      [=](int i, int j, cplx<R> v) { ci_put(L[(r0 + i) + (long long)(j0 + j) * ld], v); }, sh, first, step);
+}
+
+template <typename R, int NT, class Team>
+BIPP_HD void chol_trailing(Team& tm, int n, int j0, BIPP_GLOBAL cplx<R>* L, int ld, CiShared<R>& sh,
+                           int first = 0, int step = 1) {
+  const int jb = CI_CB, r0 = j0 + jb, mp = n - r0;
+  if (mp <= 0) return;
+  // G_{>J,>J} -= L_{>J,J} L_{>J,J}^H on and below the diagonal
+  ci_gemm<R, NT, true, false>(
+      tm, mp, mp, [=](int i, int k) { return ci_get(L[(r0 + i) + (long long)(j0 + k) * ld]); },
+      [=](int k, int j) { return conj(ci_get(L[(r0 + j) + (long long)(j0 + k) * ld])); },
+      [=](int, int, int& klo, int& khi) {
+        klo = 0;
+        khi = jb;
+      },
+      [=](int i, int j, cplx<R> v) {
+        if (i >= j) {
+          BIPP_GLOBAL cplx<R>& c = L[(r0 + i) + (long long)(r0 + j) * ld];
+          ci_put(c, ci_get(c) - v);
+        }
+      },
+      sh, first, step);
+}
+
+// T = L21 W11 of the pair of blocks of size s at b0 (b0 + s < n), in columns b0 .. of T
+template <typename R, int NT, class Team>
+BIPP_HD void chol_pair_t(Team& tm, int n, int s, int b0, BIPP_GLOBAL cplx<R>* L, int ld,
+                         BIPP_GLOBAL cplx<R>* T, int ldt, CiShared<R>& sh, int first = 0, int step = 1) {
+  const int b1 = b0 + s, s2 = n - b1 < s ? n - b1 : s;
+  // T = L21 W11 (W11 lower: k >= j)
+  ci_gemm<R, NT, false, true>(
+      tm, s2, s, [=](int i, int k) { return ci_get(L[(b1 + i) + (long long)(b0 + k) * ld]); },
+      [=](int k, int j) {
+        return k >= j ? ci_get(L[(b0 + k) + (long long)(b0 + j) * ld]) : mk<R>(0, 0);
+      },
+      [=](int, int jt, int& klo, int& khi) {
+        klo = jt;
+        khi = s;
+      },
+      [=](int i, int j, cplx<R> v) { ci_put(T[i + (long long)(b0 + j) * ldt], v); }, sh, first, step);
+}
+
+// W21 = -W22 T of that pair, over L21
+template <typename R, int NT, class Team>
+BIPP_HD void chol_pair_w(Team& tm, int n, int s, int b0, BIPP_GLOBAL cplx<R>* L, int ld,
+                         BIPP_GLOBAL cplx<R>* T, int ldt, CiShared<R>& sh, int first = 0, int step = 1) {
+  const int b1 = b0 + s, s2 = n - b1 < s ? n - b1 : s;
+  // W21 = -W22 T (W22 lower: k <= i), over L21
+  ci_gemm<R, NT, false, true>(
+      tm, s2, s,
+      [=](int i, int k) {
+        return k <= i ? ci_get(L[(b1 + i) + (long long)(b1 + k) * ld]) : mk<R>(0, 0);
+      },
+      [=](int k, int j) { return ci_get(T[k + (long long)(b0 + j) * ldt]); },
+      [=](int it, int, int& klo, int& khi) {
+        klo = 0;
+        khi = it + CI_T < s2 ? it + CI_T : s2;
+      },
+      [=](int i, int j, cplx<R> v) {
+        ci_put(L[(b1 + i) + (long long)(b0 + j) * ld], mk<R>(-v.re, -v.im));
+      },
+      sh, first, step);
+}
+
 // G (lower triangle of L, leading dimension ld) -> W = L^-1 in place.  T: scratch of at
 // least ldt x n complex (ldt >= n).  Returns -1, or the 0-based column j whose pivot is
 // not positive (the leading minor of order j + 1 is not positive definite; L is then left
@@ -150,145 +310,20 @@ BIPP_HD void ci_gemm(Team& tm, int m, int nn, FA fa, FB fb, KR krange, ST store,
 template <typename R, int NT, class Team>
 BIPP_HD int chol_inverse(Team& tm, int n, BIPP_GLOBAL cplx<R>* L, int ld, BIPP_GLOBAL cplx<R>* T, int ldt,
                          CiShared<R>& sh) {
-  const int tid = tm.tid;
-  auto at = [=](int i, int j) -> BIPP_GLOBAL cplx<R>& { return L[i + (long long)j * ld]; };
-
-  // ---- 1. blocked right-looking factorisation, diagonal blocks inverted -----------------
   tm.mark(-1);
   for (int j0 = 0; j0 < n; j0 += CI_CB) {
-    const int jb = n - j0 < CI_CB ? n - j0 : CI_CB;
-    for (int e = tid; e < CI_CB * CI_CB; e += NT) {
-      const int i = e % CI_CB, j = e / CI_CB;
-      sh.blk.d[i][j] = (i < jb && i >= j) ? ci_get(at(j0 + i, j0 + j)) : mk<R>(0, 0);
-    }
-    tm.sync();
-    // step k: pivot d_kk (final after step k - 1), trailing columns updated with the
-    // unscaled column k, column k - 1 scaled (nothing reads it in this step)
-    R p_prev = R(1);
-    int fail = -1;
-    for (int k = 0; k < jb; ++k) {
-      const R p = sh.blk.d[k][k].re;
-      if (!(p > R(0) && p == p)) {
-        fail = k;
-        break;
-      }
-      const R ip = R(1) / p;
-      for (int e = tid; e < CI_CB * CI_CB; e += NT) {
-        const int i = e % CI_CB, j = e / CI_CB;
-        if (j > k && i >= j && i < jb)
-          sh.blk.d[i][j] = sh.blk.d[i][j] - sh.blk.d[i][k] * conj(sh.blk.d[j][k]) * ip;
-      }
-      if (k > 0) {
-        const R s = sqrt(p_prev), is = R(1) / s;
-        for (int i = k - 1 + tid; i < jb; i += NT)
-          sh.blk.d[i][k - 1] = i == k - 1 ? mk<R>(s, R(0)) : sh.blk.d[i][k - 1] * is;
-      }
-      p_prev = p;
-      tm.sync();
-    }
-    if (fail >= 0) return j0 + fail;
-    {
-      const int k = jb - 1;
-      const R s = sqrt(p_prev), is = R(1) / s;
-      for (int i = k + tid; i < jb; i += NT)
-        sh.blk.d[i][k] = i == k ? mk<R>(s, R(0)) : sh.blk.d[i][k] * is;
-    }
-    tm.sync();
-    tm.mark(0);
-    // inverse W = L^-1, right-looking over the whole team: a[i][j] = delta_ij - sum_{m < i}
-    // L_im W_mj with W_mj = a[m][j] / L_mm, accumulated one pivot m per step (the elements
-    // of a step spread over the team); then W_ij = a[i][j] / L_ii
-    for (int e = tid; e < CI_CB * CI_CB; e += NT) {
-      const int i = e % CI_CB, j = e / CI_CB;
-      if (i < jb && i >= j) sh.blk.w[i][j] = mk<R>(i == j ? R(1) : R(0), R(0));
-    }
-    tm.sync();
-    for (int m = 0; m + 1 < jb; ++m) {
-      const R im = R(1) / sh.blk.d[m][m].re;
-      for (int e = tid; e < CI_CB * CI_CB; e += NT) {
-        const int i = e % CI_CB, j = e / CI_CB;
-        if (i > m && i < jb && j <= m)
-          sh.blk.w[i][j] = sh.blk.w[i][j] - sh.blk.d[i][m] * (sh.blk.w[m][j] * im);
-      }
-      tm.sync();
-    }
-    for (int e = tid; e < CI_CB * CI_CB; e += NT) {
-      const int i = e % CI_CB, j = e / CI_CB;
-      if (i < jb && i >= j) sh.blk.w[i][j] = sh.blk.w[i][j] * (R(1) / sh.blk.d[i][i].re);
-    }
-    tm.sync();
-    for (int e = tid; e < CI_CB * CI_CB; e += NT) {
-      const int i = e % CI_CB, j = e / CI_CB;
-      if (i < jb && i >= j) ci_put(at(j0 + i, j0 + j), sh.blk.w[i][j]);
-    }
-    tm.sync();
+    const int bad = chol_diagonal<R, NT>(tm, n, j0, L, ld, sh);
+    if (bad >= 0) return bad;
     tm.mark(1);
-    const int mp = n - j0 - jb;
-    if (mp > 0) {
-      const int r0 = j0 + jb;
-      // L_{>J,J} = G_{>J,J} W_JJ^H in place (a tile reads its rows' k < jb before it stores)
-      ci_gemm<R, NT, false, false>(
-          tm, mp, jb, [=](int i, int k) { return ci_get(L[(r0 + i) + (long long)(j0 + k) * ld]); },
-          [=](int k, int j) {
-            return k <= j ? conj(ci_get(L[(j0 + j) + (long long)(j0 + k) * ld])) : mk<R>(0, 0);
-          },
-          [=](int, int, int& klo, int& khi) {
-            klo = 0;
-            khi = jb;
-          },
-          [=](int i, int j, cplx<R> v) { ci_put(L[(r0 + i) + (long long)(j0 + j) * ld], v); }, sh);
-      // G_{>J,>J} -= L_{>J,J} L_{>J,J}^H on and below the diagonal
-      ci_gemm<R, NT, true, false>(
-          tm, mp, mp, [=](int i, int k) { return ci_get(L[(r0 + i) + (long long)(j0 + k) * ld]); },
-          [=](int k, int j) { return conj(ci_get(L[(r0 + j) + (long long)(j0 + k) * ld])); },
-          [=](int, int, int& klo, int& khi) {
-            klo = 0;
-            khi = jb;
-          },
-          [=](int i, int j, cplx<R> v) {
-            if (i >= j) {
-              BIPP_GLOBAL cplx<R>& c = L[(r0 + i) + (long long)(r0 + j) * ld];
-              ci_put(c, ci_get(c) - v);
-            }
-          },
-          sh);
-    }
+    chol_panel<R, NT>(tm, n, j0, L, ld, sh);
+    chol_trailing<R, NT>(tm, n, j0, L, ld, sh);
     tm.mark(2);
   }
-
-  // ---- 2. off-diagonal blocks of W, bottom-up ------------------------------------------
-  for (int s = CI_CB; s < n; s *= 2) {
+  for (int s = CI_CB; s < n; s *= 2)
     for (int b0 = 0; b0 + s < n; b0 += 2 * s) {
-      const int s2 = n - b0 - s < s ? n - b0 - s : s;
-      const int b1 = b0 + s;
-      // T = L21 W11 (W11 lower: k >= j)
-      ci_gemm<R, NT, false, true>(
-          tm, s2, s, [=](int i, int k) { return ci_get(L[(b1 + i) + (long long)(b0 + k) * ld]); },
-          [=](int k, int j) {
-            return k >= j ? ci_get(L[(b0 + k) + (long long)(b0 + j) * ld]) : mk<R>(0, 0);
-          },
-          [=](int, int jt, int& klo, int& khi) {
-            klo = jt;
-            khi = s;
-          },
-          [=](int i, int j, cplx<R> v) { ci_put(T[i + (long long)j * ldt], v); }, sh);
-      // W21 = -W22 T (W22 lower: k <= i), over L21
-      ci_gemm<R, NT, false, true>(
-          tm, s2, s,
-          [=](int i, int k) {
-            return k <= i ? ci_get(L[(b1 + i) + (long long)(b1 + k) * ld]) : mk<R>(0, 0);
-          },
-          [=](int k, int j) { return ci_get(T[k + (long long)j * ldt]); },
-          [=](int it, int, int& klo, int& khi) {
-            klo = 0;
-            khi = it + CI_T < s2 ? it + CI_T : s2;
-          },
-          [=](int i, int j, cplx<R> v) {
-            ci_put(L[(b1 + i) + (long long)(b0 + j) * ld], mk<R>(-v.re, -v.im));
-          },
-          sh);
+      chol_pair_t<R, NT>(tm, n, s, b0, L, ld, T, ldt, sh);
+      chol_pair_w<R, NT>(tm, n, s, b0, L, ld, T, ldt, sh);
     }
-  }
   tm.mark(3);
   return -1;
 }

@@ -6,8 +6,8 @@
 // 400..512-antenna samples, 64 ms for 96 of them (tridiagonalisation 23, back-transform 17,
 // whitening 3.9, un-whitening 3.0, load 1.3 ms per sample).  Here the dense phases run on tiles
 // or column groups of every sample, and the tridiagonalisation, whose column steps depend on
-// each other, takes one launch per column with several workgroups per sample.  The Cholesky
-// inverse and the divide and conquer keep a workgroup per sample (the phases of eig_kernel).
+// each other, takes one launch per column with several workgroups per sample.  The divide and
+// conquer keeps a workgroup per sample (the phase of eig_kernel).
 //
 // Buffers (leading dimension nmax): p.z_out[sample] holds the reduced S, then C, then the
 // reflectors and T factors, and in the end the eigenvectors; p.ws_l[job] G, then W = L^-1;
@@ -73,21 +73,72 @@ __global__ __launch_bounds__(256) void split_load_kernel(EigParams<double> p) {
   }
 }
 
-// W = L^-1 of G = L L^H in place (scratch ws_a); info and, where there is nothing to solve,
-// the eigenvalues.  Workgroup per job.
-template <int NMAX>
-__global__ __launch_bounds__(EigCfg<NMAX>::NT) void split_chol_kernel(EigParams<double> p) {
+// W = L^-1 of G = L L^H in place (scratch ws_a): the steps of chol_inverse, the diagonal blocks
+// on a workgroup per job, the products on one per tile; bound by the chain of diagonal blocks
+// (0.47 ms) and, at many jobs, the trailing matrix's traffic.  96 jobs of 400..512 beams 3.75 to
+// 1.96 ms, 12 jobs 3.4 to 0.99 ms against one workgroup per job for all steps.
+constexpr int SCH_NT = 256, SCH_DIAG_NT = 512;
+
+// diagonal block of column j0; info and, where there is nothing to solve, the eigenvalues
+__global__ __launch_bounds__(SCH_DIAG_NT) void split_chol_diag_kernel(EigParams<double> p, int j0) {
   const int job = blockIdx.x, sid = p.order[job], n = p.n_red[sid], tid = threadIdx.x;
-  int info = 0;
-  if (n > 0) {
-    const int bad = chol_phase<double, NMAX>(n, p.ws_l + (size_t)job * p.ws_stride, p.ws_ld,
-                                             p.ws_a + (size_t)job * p.ws_stride, p.ws_ld, nullptr);
-    // leading minor bad + 1 of G is not positive definite: ?hegv reports info = n + bad + 1
-    if (bad >= 0) info = n + bad + 1;
+  __shared__ CiShared<double> sh;
+  if (j0 == 0 ? n <= 0 : (j0 >= n || p.info[sid])) {  // uniform
+    if (j0 == 0) {
+      for (int j = tid; j < p.nmax; j += SCH_DIAG_NT) p.d_out[(size_t)sid * p.stride_d + j] = 0;
+      if (tid == 0) p.info[sid] = 0;
+    }
+    return;
   }
-  if (n <= 0 || info)
-    for (int j = tid; j < p.nmax; j += EigCfg<NMAX>::NT) p.d_out[(size_t)sid * p.stride_d + j] = 0;
-  if (tid == 0) p.info[sid] = info;
+  WgTeam tm{tid};
+  const int bad = chol_diagonal<double, SCH_DIAG_NT>(tm, n, j0, global_ptr(p.ws_l + (size_t)job * p.ws_stride),
+                                                p.ws_ld, sh);
+  // leading minor bad + 1 of G is not positive definite: ?hegv reports info = n + bad + 1
+  if (bad >= 0)
+    for (int j = tid; j < p.nmax; j += SCH_DIAG_NT) p.d_out[(size_t)sid * p.stride_d + j] = 0;
+  if (tid == 0 && (bad >= 0 || j0 == 0)) p.info[sid] = bad >= 0 ? n + bad + 1 : 0;
+}
+
+// one tile of a product per workgroup: STEP 0 the panel below diagonal block j0, 1 the trailing
+// matrix, 2 and 3 T and W21 of the pairs of blocks of size j0 (unit: pair, tile)
+template <int STEP>
+__global__ __launch_bounds__(SCH_NT) void split_chol_tile_kernel(EigParams<double> p, int j0, int per_job,
+                                                                 int tiles) {
+  const SplitUnit u = split_unit(per_job, p.n_jobs);
+  if (u.job < 0) return;
+  const int sid = p.order[u.job], n = p.n_red[sid];
+  if (n <= 0 || p.info[sid]) return;
+  __shared__ CiShared<double> sh;
+  WgTeam tm{static_cast<int>(threadIdx.x)};
+  BIPP_GLOBAL cplx<double>* L = global_ptr(p.ws_l + (size_t)u.job * p.ws_stride);
+  BIPP_GLOBAL cplx<double>* T = global_ptr(p.ws_a + (size_t)u.job * p.ws_stride);
+  constexpr int ONE = 1 << 30;  // no second tile
+  if (STEP == 0) chol_panel<double, SCH_NT>(tm, n, j0, L, p.ws_ld, sh, u.unit, ONE);
+  if (STEP == 1) chol_trailing<double, SCH_NT>(tm, n, j0, L, p.ws_ld, sh, u.unit, ONE);
+  if (STEP >= 2) {
+    const int b0 = u.unit / tiles * 2 * j0;
+    if (b0 + j0 >= n) return;
+    if (STEP == 2) chol_pair_t<double, SCH_NT>(tm, n, j0, b0, L, p.ws_ld, T, p.ws_ld, sh, u.unit % tiles, ONE);
+    if (STEP == 3) chol_pair_w<double, SCH_NT>(tm, n, j0, b0, L, p.ws_ld, T, p.ws_ld, sh, u.unit % tiles, ONE);
+  }
+}
+
+inline void launch_split_chol(const EigParams<double>& p, int n_max, hipStream_t stream) {
+  const int jobs = p.n_jobs;
+  for (int j0 = 0; j0 < std::max(n_max, 1); j0 += CI_CB) {
+    split_chol_diag_kernel<<<jobs, SCH_DIAG_NT, 0, stream>>>(p, j0);
+    const int rows = n_max - j0 - CI_CB, t = rows > 0 ? ceil_div(rows, CI_T) : 0;
+    if (t == 0) continue;
+    split_chol_tile_kernel<0><<<split_grid(t, jobs), SCH_NT, 0, stream>>>(p, j0, t, t);
+    const int tt = t * (t + 1) / 2;
+    split_chol_tile_kernel<1><<<split_grid(tt, jobs), SCH_NT, 0, stream>>>(p, j0, tt, tt);
+  }
+  for (int s = CI_CB; s < n_max; s *= 2) {
+    const int pairs = ceil_div(n_max - s, 2 * s), side = ceil_div(s, CI_T), tiles = side * side;
+    split_chol_tile_kernel<2><<<split_grid(pairs * tiles, jobs), SCH_NT, 0, stream>>>(p, s, pairs * tiles, tiles);
+    split_chol_tile_kernel<3><<<split_grid(pairs * tiles, jobs), SCH_NT, 0, stream>>>(p, s, pairs * tiles, tiles);
+  }
+  check_launch("split_chol_kernel");
 }
 
 // Dense products on 64 x 64 tiles, a wavefront per 32 x 32 quadrant (2 x 2 blocks of

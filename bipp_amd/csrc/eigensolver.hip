@@ -1547,8 +1547,7 @@ void launch_eig_split(const EigParams<double>& p, const EigSplitBuffers& b, int 
       split_load_kernel<float><<<lg, 256, 0, stream>>>(p);
     check_launch("split_load_kernel");
   }
-  split_chol_kernel<NM><<<jobs, EigCfg<NM>::NT, 0, stream>>>(p);
-  check_launch("split_chol_kernel");
+  launch_split_chol(p, n_max, stream);
   if (n_max <= 0) return;
   const int side = ceil_div(n_max, 64);
   split_gemm_kernel<0><<<split_grid(side * side, jobs), 256, 0, stream>>>(p, side);

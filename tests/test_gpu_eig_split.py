@@ -87,6 +87,20 @@ def test_resident_sizes(ctx, n, live):
         assert rel((v[k] * d[k]) @ v[k].conj().T, (vo * do) @ vo.conj().T) < 1e-10
 
 
+def test_cholesky_tile_sizes(ctx):
+    """The Cholesky inverse on tiles of all samples: sizes on both sides of its diagonal blocks
+    (32), tiles (64) and pairs of blocks, and samples far below the batch's largest."""
+    n, live = 400, [400, 385, 384, 383, 352, 353, 321, 320, 319, 289, 288, 65, 64, 33, 32, 31, 1]
+    samples = make(n, live, 11)
+    print(f"split eigensolve n={n} live={live}", flush=True)
+    d, v, nr = solve(ctx, samples, n)
+    for k, smp in enumerate(samples):
+        vo, do, _, _ = O.eigh_gram(smp.wl, smp.s.astype(np.complex64), None, smp.xyz)
+        assert nr[k] == live[k]
+        assert np.abs(d[k] - do).max() < 1e-10 * np.abs(do).max()
+        assert rel((v[k] * d[k]) @ v[k].conj().T, (vo * do) @ vo.conj().T) < 1e-10
+
+
 def test_handover_sizes(ctx):
     """The tridiagonalisation hands the last 256 columns from the column launches to one workgroup
     per sample: with one and with two updates pending (odd and even counts of columns before
