@@ -1284,19 +1284,32 @@ __global__ __launch_bounds__(FFT_NT) void fft_pass_rr_kernel(N3PassParams<R> p, 
 // Bound by LDS exchanges and the transforms' arithmetic between barriers, behind them HBM (7 GB
 // at configuration 4).  500 samples of 256 antennas, y axis of 3456 points, 4 levels: 3.9 + 3.0
 // ms in two passes, 3.7 ms in one (4.3 ms with 512 threads).
-template <typename R, int NT, int RAD, bool FIRST, bool LAST>
+// NAT: contiguous axis (x lines, a position is a line): consecutive lanes take consecutive
+// elements of one line, and the frequencies are stored in their own order.
+template <typename R, int NT, int RAD, bool FIRST, bool LAST, bool NAT>
 __device__ __forceinline__ void axis_stage(const N3AxisParams<R>& p, int s, cplx<R>* lds, const Twid<R>& tw,
                                            cplx<R>* base, int xt, int tid) {
-  const int tws = p.tw_shift, TW = 1 << tws;
-  const int S = p.span[s], items = (p.n / RAD) << tws;
+  const int tws = p.tw_shift, TW = 1 << tws, per = p.n / RAD;
+  const int S = p.span[s], items = per << tws;
   for (int u = tid; u < items; u += NT) {
-    const int xi = u & (TW - 1), t = u >> tws;
+    const int xi = NAT ? fast_div(u, p.per_m[s], p.per_s[s]) : u & (TW - 1);
+    const int t = NAT ? u - xi * per : u >> tws;
+    int K = 0, rest = t, at = 0;  // LAST: frequency of output 0 and the position it comes from
+    if constexpr (LAST && NAT) {
+      K = t;
+      for (int q = 0; q < s; ++q) {
+        const int f = fast_div(rest, p.rd_m[q], p.rd_s[q]);
+        at += (rest - f * p.r[q]) * p.span[q];
+        rest = f;
+      }
+    }
     const int hi = LAST ? t : FIRST ? 0 : fast_div(t, p.sp_m[s], p.sp_s[s]);
     const int lo = LAST ? 0 : t - hi * S;
-    cplx<R>* line = lds + xi * p.ld + hi * (RAD * S) + lo;
+    cplx<R>* line = lds + xi * p.ld + (LAST && NAT ? at : hi * (RAD * S) + lo);
     const int j = (xt << tws) + xi;
-    int x = p.xw.start + j;
-    x -= x >= p.nx ? p.nx : 0;
+    int xp = p.xw.start + j;
+    xp -= xp >= p.nx ? p.nx : 0;
+    const long long x = NAT ? (long long)xp * p.n : xp;
     cplx<R> v[RAD];
     if constexpr (FIRST) {
 #pragma unroll
@@ -1312,8 +1325,14 @@ __device__ __forceinline__ void axis_stage(const N3AxisParams<R>& p, int s, cplx
     dft_small<R, RAD>(v);
     if constexpr (LAST) {
       if (j >= p.xw.count) continue;
-      // digits of the position hi RAD: the frequency of output 0
-      int K = 0, rest = hi * RAD;
+      if constexpr (NAT) {
+#pragma unroll
+        for (int r = 0; r < RAD; ++r)
+          if (in_window(K + r * p.weight[s], p.out, p.n)) base[x + K + r * p.weight[s]] = v[r];
+        continue;
+      }
+      // digits of the position hi RAD
+      rest = hi * RAD;
       for (int q = 0; q < s; ++q) {
         const int f = fast_div(rest, p.sp_m[q], p.sp_s[q]);
         rest -= f * p.span[q];
@@ -1347,25 +1366,25 @@ __device__ __forceinline__ void axis_stage(const N3AxisParams<R>& p, int s, cplx
   }
 }
 
-template <typename R, int NT, bool FIRST, bool LAST>
+template <typename R, int NT, bool FIRST, bool LAST, bool NAT>
 __device__ __forceinline__ void axis_radix(const N3AxisParams<R>& p, int s, cplx<R>* lds, const Twid<R>& tw,
                                            cplx<R>* base, int xt, int tid) {
   switch (p.r[s]) {
-    case 2: axis_stage<R, NT, 2, FIRST, LAST>(p, s, lds, tw, base, xt, tid); break;
-    case 3: axis_stage<R, NT, 3, FIRST, LAST>(p, s, lds, tw, base, xt, tid); break;
-    case 4: axis_stage<R, NT, 4, FIRST, LAST>(p, s, lds, tw, base, xt, tid); break;
-    case 5: axis_stage<R, NT, 5, FIRST, LAST>(p, s, lds, tw, base, xt, tid); break;
-    case 6: axis_stage<R, NT, 6, FIRST, LAST>(p, s, lds, tw, base, xt, tid); break;
-    case 8: axis_stage<R, NT, 8, FIRST, LAST>(p, s, lds, tw, base, xt, tid); break;
-    case 9: axis_stage<R, NT, 9, FIRST, LAST>(p, s, lds, tw, base, xt, tid); break;
-    case 10: axis_stage<R, NT, 10, FIRST, LAST>(p, s, lds, tw, base, xt, tid); break;
-    case 12: axis_stage<R, NT, 12, FIRST, LAST>(p, s, lds, tw, base, xt, tid); break;
-    case 15: axis_stage<R, NT, 15, FIRST, LAST>(p, s, lds, tw, base, xt, tid); break;
-    default: axis_stage<R, NT, 16, FIRST, LAST>(p, s, lds, tw, base, xt, tid); break;
+    case 2: axis_stage<R, NT, 2, FIRST, LAST, NAT>(p, s, lds, tw, base, xt, tid); break;
+    case 3: axis_stage<R, NT, 3, FIRST, LAST, NAT>(p, s, lds, tw, base, xt, tid); break;
+    case 4: axis_stage<R, NT, 4, FIRST, LAST, NAT>(p, s, lds, tw, base, xt, tid); break;
+    case 5: axis_stage<R, NT, 5, FIRST, LAST, NAT>(p, s, lds, tw, base, xt, tid); break;
+    case 6: axis_stage<R, NT, 6, FIRST, LAST, NAT>(p, s, lds, tw, base, xt, tid); break;
+    case 8: axis_stage<R, NT, 8, FIRST, LAST, NAT>(p, s, lds, tw, base, xt, tid); break;
+    case 9: axis_stage<R, NT, 9, FIRST, LAST, NAT>(p, s, lds, tw, base, xt, tid); break;
+    case 10: axis_stage<R, NT, 10, FIRST, LAST, NAT>(p, s, lds, tw, base, xt, tid); break;
+    case 12: axis_stage<R, NT, 12, FIRST, LAST, NAT>(p, s, lds, tw, base, xt, tid); break;
+    case 15: axis_stage<R, NT, 15, FIRST, LAST, NAT>(p, s, lds, tw, base, xt, tid); break;
+    default: axis_stage<R, NT, 16, FIRST, LAST, NAT>(p, s, lds, tw, base, xt, tid); break;
   }
 }
 
-template <typename R, int NT>
+template <typename R, int NT, bool NAT>
 __global__ __launch_bounds__(NT) void fft_axis_kernel(N3AxisParams<R> p) {
   extern __shared__ __align__(16) unsigned char fsh[];
   cplx<R>* lds = reinterpret_cast<cplx<R>*>(fsh);
@@ -1386,13 +1405,13 @@ __global__ __launch_bounds__(NT) void fft_axis_kernel(N3AxisParams<R> p) {
       oo = (oo - q * p.operm_n1) * p.operm_n2 + q;
     }
     cplx<R>* base = p.grid + (size_t)lv * p.grid_stride + (size_t)oo * p.outer_stride;
-    axis_radix<R, NT, true, false>(p, 0, lds, tw, base, xt, tid);
+    axis_radix<R, NT, true, false, NAT>(p, 0, lds, tw, base, xt, tid);
     for (int s = 1; s < p.stages - 1; ++s) {
       __syncthreads();
-      axis_radix<R, NT, false, false>(p, s, lds, tw, base, xt, tid);
+      axis_radix<R, NT, false, false, NAT>(p, s, lds, tw, base, xt, tid);
     }
     __syncthreads();
-    axis_radix<R, NT, false, true>(p, p.stages - 1, lds, tw, base, xt, tid);
+    axis_radix<R, NT, false, true, NAT>(p, p.stages - 1, lds, tw, base, xt, tid);
     __syncthreads();  // lines read before the next tile's first stage
   }
 }
@@ -1972,9 +1991,13 @@ inline int max_radix(const N3Radix& r) {
 }  // namespace
 
 template <typename R>
+bool launch_fft_xlines(const N3LineParams<R>& q, hipStream_t st);
+
+template <typename R>
 void launch_fft_lines(const N3LineParams<R>& p, hipStream_t st) {
   const long long n_lines = (long long)p.n_levels * p.zw.count * p.yw.count;
   if (n_lines <= 0) return;
+  if (launch_fft_xlines(p, st)) return;
   if (!window_ok(p.yw, p.ny) || !window_ok(p.zw, p.nz) || !window_ok(p.in, p.n) ||
       !window_ok(p.out, p.n))
     fail(BIPP_INTERNAL_ERROR, "FFT line windows out of range");
@@ -2091,15 +2114,32 @@ int fft_axis_shift(int n, size_t elem) {
   return -1;
 }
 
-template <typename R>
-bool launch_fft_axis(const N3AxisParams<R>& p_in, hipStream_t st) {
-  N3AxisParams<R> p = p_in;
-  int f[4];
-  if (p.n2 < 2 || (long long)p.n1 * p.n2 != p.n || !fft_rr_factors(p.n1, f[0], f[1]) ||
-      !fft_rr_factors(p.n2, f[2], f[3]))
-    return false;
-  p.tw_shift = fft_axis_shift(p.n, sizeof(cplx<R>));
-  if (p.tw_shift < 0) return false;
+// radices of a contiguous axis: at most four, the fewest, the most even of those
+bool fft_line_radices(int n, int (&f)[4]) {
+  constexpr int rad[] = {16, 15, 12, 10, 9, 8, 6, 5, 4, 3, 2};
+  int best = 5, best_max = 17, cur[4];
+  auto go = [&](auto&& self, int m, int k, int top) -> void {
+    if (m == 1) {
+      if (k < best || (k == best && cur[0] < best_max)) {
+        best = k;
+        best_max = cur[0];
+        for (int i = 0; i < 4; ++i) f[i] = i < k ? cur[i] : 1;
+      }
+      return;
+    }
+    if (k == 4 || k >= best) return;
+    for (int r : rad)
+      if (r <= top && m % r == 0) {
+        cur[k] = r;
+        self(self, m / r, k + 1, r);
+      }
+  };
+  go(go, n, 0, 16);
+  return best >= 2 && best <= 4;
+}
+
+template <typename R, bool NAT>
+bool go_fft_axis(N3AxisParams<R> p, const int (&f)[4], hipStream_t st) {
   if (!window_ok(p.xw, p.nx) || !window_ok(p.other, p.no) || !window_ok(p.in, p.n) ||
       !window_ok(p.out, p.n))
     fail(BIPP_INTERNAL_ERROR, "FFT pass windows out of range");
@@ -2113,12 +2153,14 @@ bool launch_fft_axis(const N3AxisParams<R>& p_in, hipStream_t st) {
     done *= f[k];
     p.span[s] = p.n / done;
     n3_div_magic(p.span[s], p.sp_m[s], p.sp_s[s]);
+    n3_div_magic(p.n / f[k], p.per_m[s], p.per_s[s]);
+    n3_div_magic(f[k], p.rd_m[s], p.rd_s[s]);
   }
-  p.last_step = p.weight[p.stages - 1] / p.n1;
-  n3_div_magic(p.n1, p.n1_m, p.n1_s);
+  if (!NAT) p.last_step = p.weight[p.stages - 1] / p.n1;
+  n3_div_magic(NAT ? 1 : p.n1, p.n1_m, p.n1_s);
   // line stride 32 / positions modulo 32 elements: a row of positions in different banks
   const int want = 32 >> p.tw_shift;
-  p.ld = p.n + ((want - p.n) % 32 + 32) % 32;
+  p.ld = NAT ? p.n : p.n + ((want - p.n) % 32 + 32) % 32;
   const int TW = 1 << p.tw_shift;
   const long long items = (long long)((p.xw.count + TW - 1) / TW) * p.other.count * p.n_levels;
   if (items <= 0) return true;
@@ -2134,15 +2176,54 @@ bool launch_fft_axis(const N3AxisParams<R>& p_in, hipStream_t st) {
                             hipFuncAttributeMaxDynamicSharedMemorySize, 159 * 1024);
     hip_check(attr, "hipFuncSetAttribute");
     // a round is one tile per resident workgroup
-    const long long round = sh <= 39 * 1024 ? 1024 : sh <= 79 * 1024 ? 512 : 256;
+    const long long round = sh <= 39 * 1024 ? 1024 : sh <= 52 * 1024 ? 768 : sh <= 79 * 1024 ? 512 : 256;
     kernel<<<static_cast<unsigned>(std::min(items, round)), nt, sh, st>>>(p);
   };
   if (sh <= 79 * 1024)
-    go(&fft_axis_kernel<R, 512>, 512);
+    go(&fft_axis_kernel<R, 512, NAT>, 512);
   else
-    go(&fft_axis_kernel<R, 1024>, 1024);
+    go(&fft_axis_kernel<R, 1024, NAT>, 1024);
   check_launch("fft_axis_kernel");
   return true;
+}
+
+template <typename R>
+bool launch_fft_axis(const N3AxisParams<R>& p_in, hipStream_t st) {
+  N3AxisParams<R> p = p_in;
+  int f[4];
+  if (p.n2 < 2 || (long long)p.n1 * p.n2 != p.n || !fft_rr_factors(p.n1, f[0], f[1]) ||
+      !fft_rr_factors(p.n2, f[2], f[3]))
+    return false;
+  p.tw_shift = fft_axis_shift(p.n, sizeof(cplx<R>));
+  return p.tw_shift >= 0 && go_fft_axis<R, false>(p, f, st);
+}
+
+// x lines by the same stages, up to 2048 points: two lines and more per workgroup, one buffer
+// instead of two.  Above, fft_lines_kernel's prefetch and twiddle tables are as good or better
+// (FFT of 64-antenna samples, x and y of 1800 points: 13.7 to 10.6 ms with this form, 768 points
+// 3.1 to 2.1, 240 points 0.49 to 0.39; 2160 points 18.9 and 18.5 in float, 51.9 and 53.4 in
+// double; 3240 points 3.27 against 3.80 for the lines alone, 6000 5.98 against 7.42).
+template <typename R>
+bool launch_fft_xlines(const N3LineParams<R>& q, hipStream_t st) {
+  N3AxisParams<R> p{};
+  int f[4];
+  if (q.n > 2048 || !fft_line_radices(q.n, f)) return false;
+  p.grid = q.grid;
+  p.grid_stride = q.grid_stride;
+  p.n_levels = q.n_levels;
+  p.nx = q.ny;
+  p.xw = q.yw;
+  p.no = q.nz;
+  p.other = q.zw;
+  p.operm_n1 = p.operm_n2 = 1;
+  p.outer_stride = (long long)q.n * q.ny;
+  p.axis_stride = 1;
+  p.n = q.n;
+  p.in = q.in;
+  p.out = q.out;
+  p.tw = q.tw;
+  while (p.tw_shift < 4 && (q.n << (p.tw_shift + 1)) <= 4096) ++p.tw_shift;
+  return go_fft_axis<R, true>(p, f, st);
 }
 template bool launch_fft_axis<float>(const N3AxisParams<float>&, hipStream_t);
 template bool launch_fft_axis<double>(const N3AxisParams<double>&, hipStream_t);

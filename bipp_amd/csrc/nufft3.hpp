@@ -205,8 +205,8 @@ struct N3AxisParams {
   // frequency), row step of the last stage's outputs, line stride, division constants
   int stages, tw_shift, ld, last_step;
   int r[4], span[4], weight[4];
-  unsigned sp_m[4], n1_m, xt_m, oc_m, op_m;
-  int sp_s[4], n1_s, xt_s, oc_s, op_s;
+  unsigned sp_m[4], per_m[4], rd_m[4], n1_m, xt_m, oc_m, op_m;
+  int sp_s[4], per_s[4], rd_s[4], n1_s, xt_s, oc_s, op_s;
 };
 
 template <typename R>

@@ -83,3 +83,37 @@ def test_fft_axis_lengths(ctx, compute, length):
     err = O.rel_l2(syn.images()[0], ref[0])
     print(f"grid {syn.nufft_grid()} {compute}: rel L2 {err:.2e}", flush=True)
     assert err <= bound
+
+
+@pytest.mark.parametrize("compute,length", [(c, n) for c in ("mixed", "fp64")
+                                            for n in (54, 250, 750, 1024, 1250, 2000, 2048, 2160)])
+def test_fft_line_lengths(ctx, compute, length):
+    """The x lines on both sides of the lengths at which their workgroups take 16, 8, 4, 2 lines,
+    and of the longest that they take (2048), an array stretched along x."""
+    tol = 1e-5 if compute == "mixed" else 1e-9
+    bound = 1e-4 if compute == "mixed" else 7.5e-7   # as test_fft_axis_lengths
+    r = np.random.default_rng(length)
+    n = 9
+    src, flux = synthetic.zenith_cap_sources(r, 5, 5.0)
+    p0 = synthetic.disk_positions(r, n, 1.0) + np.array([0, 0, 0.3]) * r.normal(size=(n, 1))
+    lmn = synthetic.make_lmn_grid(21, math.radians(20))
+    w = math.ceil(math.log10(1 / tol)) + 1
+    a, b = np.tril_indices(n)
+    u = 2 * np.pi * (p0[a, 0] - p0[b, 0])
+    xs = 0.5 * (u.max() - u.min()) * 0.5 * (lmn[:, 0].max() - lmn[:, 0].min())
+    for want in np.arange(length / 2, length / 2 * 0.9 - 12, -max(length / 1000, 0.1)):
+        scale = (want - w - 1) / (4 / math.pi * xs)
+        if scale <= 0:
+            break
+        xyz = p0 * np.array([scale, 5.0, 2.0])
+        s = synthetic.visibilities(xyz, 1.0, src, flux, 0.1)
+        syn = bipp_amd.NufftSynthesis(ctx, n, n, [[0.0, 3e38]], lmn, compute=compute,
+                                      imager="nufft", tolerance=tol)
+        syn.collect(1.0, s, xyz)
+        if syn.nufft_grid()[0] <= length:
+            break
+    ref, _ = O.synthesize([synthetic.Sample(0, 0, 1.0, xyz, s, np.ones(n, bool))],
+                          np.array([[0.0, 3e38]]), lmn)
+    err = O.rel_l2(syn.images()[0], ref[0])
+    print(f"grid {syn.nufft_grid()} {compute}: rel L2 {err:.2e}", flush=True)
+    assert err <= bound
