@@ -389,11 +389,15 @@ def main() -> None:
                              "kernel_ms": kern_ms, "fine_grid": list(nf), "spread_grid": nf1,
                              "points": m_pts, "algorithmic_bytes_per_launch": nufft_bytes}
         # measured HBM bytes of the chain: per-dispatch counters times dispatches per step
-        # (one spread launch per 6 levels; strided axes above 128 points take two passes)
+        # (one spread launch per 6 levels; strided axes above 128 points in one pass, x lines up
+        # to 2048 points by the same kernel)
         launches = {"n3_points_kernel": 2,
-                    "n3_spread_kernel": (L + 5) // 6, "fft_lines_kernel": 1,
-                    "fft_pass_rr_kernel": sum(2 if x > 128 else 1 for x in nf[1:]),
+                    "n3_spread_kernel": (L + 5) // 6,
+                    "fft_lines_kernel": 1 if nf[0] > 2048 else 0,
+                    "fft_axis_kernel": sum(x > 128 for x in nf[1:]) + (nf[0] <= 2048),
+                    "fft_pass_rr_kernel": sum(x <= 128 for x in nf[1:]),
                     "n3_interp_kernel": 1}
+        launches = {k: v for k, v in launches.items() if v}
         per_kernel = {}
         for k, cnt in launches.items():
             t = measured_traffic(k, a.config)

@@ -1281,9 +1281,9 @@ __global__ __launch_bounds__(FFT_NT) void fft_pass_rr_kernel(N3PassParams<R> p, 
 // two passes, twice the windows' size each way, stays in the CU.
 // Workgroup i of a round runs on XCD i mod 8 and the tiles of a round are dealt to the XCDs in
 // runs: neighbouring tiles share 128-byte lines (a tile of 4 positions has 32 bytes of each).
-// Bound by LDS exchanges and the transforms' arithmetic between barriers, behind them HBM (7 GB
-// at configuration 4).  500 samples of 256 antennas, y axis of 3456 points, 4 levels: 3.9 + 3.0
-// ms in two passes, 3.7 ms in one (4.3 ms with 512 threads).
+// Bound by LDS exchanges and the transforms' arithmetic between barriers, behind them HBM.  500
+// samples of 256 antennas, y axis of 3456 points, 4 levels: 3.7 ms and 7.9 GB (4.3 ms with 512
+// threads) against 3.9 + 3.0 ms and 23 GB in two passes.
 // NAT: contiguous axis (x lines, a position is a line): consecutive lanes take consecutive
 // elements of one line, and the frequencies are stored in their own order.
 template <typename R, int NT, int RAD, bool FIRST, bool LAST, bool NAT>
