@@ -64,18 +64,19 @@ struct BippImagerImpl {
       staged = std::min(staged, batch);
     }
     if (count < staged) return;
-    staged = std::min(batch, std::max<size_t>(16, 2 * staged));
-    grow(h_uvw, sizeof(float) * 3 * nn());
-    grow(h_v, 8 * (size_t)n_ant * n_beam);
-    grow(h_d, sizeof(float) * (size_t)n_img * n_beam);
-    grow(h_sc, sizeof(float));
-    grow(h_wl, sizeof(float));
+    const size_t room = std::min(batch, std::max<size_t>(16, 2 * staged));
+    grow(h_uvw, sizeof(float) * 3 * nn(), room);
+    grow(h_v, 8 * (size_t)n_ant * n_beam, room);
+    grow(h_d, sizeof(float) * (size_t)n_img * n_beam, room);
+    grow(h_sc, sizeof(float), room);
+    grow(h_wl, sizeof(float), room);
+    staged = room;  // only now: an allocation that failed above leaves the old room
   }
-  // `b` with room for `staged` samples of `bytes` each, the first `count` kept
-  void grow(PinnedBuf& b, size_t bytes) {
-    if (b.cap >= bytes * staged) return;
+  // `b` with room for `room` samples of `bytes` each, the first `count` kept
+  void grow(PinnedBuf& b, size_t bytes, size_t room) {
+    if (b.cap >= bytes * room) return;
     PinnedBuf n;
-    n.get(bytes * staged);
+    n.get(bytes * room);
     if (count) std::memcpy(n.p, b.p, bytes * count);
     n.swap(b);
   }
