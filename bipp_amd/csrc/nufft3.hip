@@ -24,6 +24,7 @@
 #include "nufft3.hpp"
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <type_traits>
 
@@ -2138,6 +2139,21 @@ bool fft_line_radices(int n, int (&f)[4]) {
   return best >= 2 && best <= 4;
 }
 
+// The LDS limit is a property of the kernel, so its flag belongs to the instantiation (the kernels
+// of the two workgroup sizes have one function type), and is set once the runtime took the limit.
+template <typename R, int NT, bool NAT>
+void start_fft_axis(const N3AxisParams<R>& p, long long items, size_t sh, hipStream_t st) {
+  static std::atomic<bool> attr{false};
+  if (!attr) {
+    BIPP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&fft_axis_kernel<R, NT, NAT>),
+                                 hipFuncAttributeMaxDynamicSharedMemorySize, 159 * 1024));
+    attr = true;
+  }
+  // a round is one tile per resident workgroup
+  const long long round = sh <= 39 * 1024 ? 1024 : sh <= 52 * 1024 ? 768 : sh <= 79 * 1024 ? 512 : 256;
+  fft_axis_kernel<R, NT, NAT><<<static_cast<unsigned>(std::min(items, round)), NT, sh, st>>>(p);
+}
+
 template <typename R, bool NAT>
 bool go_fft_axis(N3AxisParams<R> p, const int (&f)[4], hipStream_t st) {
   if (!window_ok(p.xw, p.nx) || !window_ok(p.other, p.no) || !window_ok(p.in, p.n) ||
@@ -2169,20 +2185,12 @@ bool go_fft_axis(N3AxisParams<R> p, const int (&f)[4], hipStream_t st) {
   n3_div_magic(p.other.count, p.oc_m, p.oc_s);
   n3_div_magic(p.operm_n2 > 1 ? p.operm_n1 : 1, p.op_m, p.op_s);
   const size_t sh = sizeof(cplx<R>) * (((size_t)p.ld << p.tw_shift) + twid_len(p.n));
-  if (sh > 159 * 1024) fail(BIPP_INTERNAL_ERROR, "FFT pass exceeds LDS");
-  auto go = [&](auto kernel, int nt) {
-    static const hipError_t attr =
-        hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, 159 * 1024);
-    hip_check(attr, "hipFuncSetAttribute");
-    // a round is one tile per resident workgroup
-    const long long round = sh <= 39 * 1024 ? 1024 : sh <= 52 * 1024 ? 768 : sh <= 79 * 1024 ? 512 : 256;
-    kernel<<<static_cast<unsigned>(std::min(items, round)), nt, sh, st>>>(p);
-  };
-  if (sh <= 79 * 1024)
-    go(&fft_axis_kernel<R, 512, NAT>, 512);
-  else
-    go(&fft_axis_kernel<R, 1024, NAT>, 1024);
+  // x lines (at most 4096 elements per tile) stay below 79 KiB
+  if (sh > (NAT ? 79 : 159) * 1024) fail(BIPP_INTERNAL_ERROR, "FFT pass exceeds LDS");
+  if (NAT || sh <= 79 * 1024)
+    start_fft_axis<R, 512, NAT>(p, items, sh, st);
+  else if constexpr (!NAT)
+    start_fft_axis<R, 1024, false>(p, items, sh, st);
   check_launch("fft_axis_kernel");
   return true;
 }

@@ -92,3 +92,48 @@ hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
 hipError_t hipEventQuery(hipEvent_t) { return ++stub::stream_waits, hipSuccess; }
 hipError_t hipEventElapsedTime(float* t, hipEvent_t, hipEvent_t) { return *t = 0, hipSuccess; }
 }
+
+// Kernel launches: nothing runs; the dynamic LDS of each launch is held against the limit that
+// was set for its kernel before (64 KiB without one).
+namespace stub {
+struct Launch {
+  const void* kernel;
+  unsigned threads;
+  size_t lds, limit;
+};
+inline std::map<const void*, size_t> lds_limit;
+inline Launch last{};
+inline int launches = 0, attribute_failures = 0;  // attribute calls to fail
+inline dim3 cfg_grid, cfg_block;
+inline size_t cfg_lds = 0;
+}  // namespace stub
+
+extern "C" {
+hipError_t hipFuncSetAttribute(const void* f, hipFuncAttribute, int v) {
+  if (stub::attribute_failures > 0) return --stub::attribute_failures, hipErrorUnknown;
+  return stub::lds_limit[f] = static_cast<size_t>(v), hipSuccess;
+}
+hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t lds, hipStream_t) {
+  stub::cfg_grid = g;
+  stub::cfg_block = b;
+  stub::cfg_lds = lds;
+  return hipSuccess;
+}
+hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* lds, hipStream_t* s) {
+  *g = stub::cfg_grid;
+  *b = stub::cfg_block;
+  *lds = stub::cfg_lds;
+  *s = nullptr;
+  return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void* f, dim3, dim3 b, void**, size_t lds, hipStream_t) {
+  const auto it = stub::lds_limit.find(f);
+  stub::last = {f, b.x, lds, it == stub::lds_limit.end() ? size_t(64) << 10 : it->second};
+  ++stub::launches;
+  return hipSuccess;
+}
+void** __hipRegisterFatBinary(const void*) { return nullptr; }
+void __hipRegisterFunction(void**, const void*, char*, const char*, unsigned, void*, void*, void*, void*, int*) {}
+void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
+void __hipUnregisterFatBinary(void**) {}
+}
