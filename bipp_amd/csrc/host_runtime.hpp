@@ -61,19 +61,34 @@ inline void require(bool cond, BippError code, const std::string& msg) {
 // Memory blocks given back by short-lived buffers of a context (the imager of one
 // image_synthesis call, the arrays of one host eigensolve), for the next ones: allocating,
 // pinning and freeing them took 5.5 ms of a 15 ms call.  At most DEV_BOUND bytes of device and
-// PIN_BOUND of pinned host memory are held; above that the blocks longest unused, and
-// everything when the context goes or a device allocation fails, go back to the runtime (a
-// pool that kept its first blocks instead was full of one call's sizes, and the next kind of
-// call allocated everything anew: 2.2 ms became 9 to 17 ms).  Device blocks are handed on in stream
+// PIN_BOUND of pinned host memory are held per context; above that the blocks longest unused go
+// back to the runtime (a pool that kept its first blocks instead was full of one call's sizes,
+// and the next kind of call allocated everything anew: 2.2 ms became 9 to 17 ms).  Everything goes
+// back when the context goes, and the blocks of every pool when an allocation of the library fails,
+// in a pool's scope or not, before it is tried again.  Device blocks are handed on in stream
 // order: all users of a context's pool work on its one stream.  Pinned blocks are given back
 // only after the stream has been waited for.
 struct BufferPool {
   static constexpr size_t DEV_BOUND = size_t(2) << 30, PIN_BOUND = size_t(256) << 20;
   enum Kind { DEV = 0, PIN = 1 };
 
-  BufferPool() = default;
+  BufferPool() {
+    std::lock_guard<std::mutex> lock(all().mu);
+    all().pools.push_back(this);
+  }
   BufferPool(const BufferPool&) = delete;
-  ~BufferPool() { trim(); }
+  ~BufferPool() {
+    {
+      std::lock_guard<std::mutex> lock(all().mu);
+      all().pools.erase(std::find(all().pools.begin(), all().pools.end(), this));
+    }
+    trim();
+  }
+  // the held blocks of every pool back to the runtime
+  static void trim_all() {
+    std::lock_guard<std::mutex> lock(all().mu);
+    for (BufferPool* p : all().pools) p->trim();
+  }
   // a held block of at least `bytes` (and not much more), or nullptr
   void* take(Kind k, size_t bytes, size_t& cap) {
     std::lock_guard<std::mutex> lock(mu_);
@@ -126,6 +141,14 @@ struct BufferPool {
     void* p;
     unsigned long long since;  // of clock_
   };
+  struct Registry {
+    std::mutex mu;
+    std::vector<BufferPool*> pools;
+  };
+  static Registry& all() {
+    static Registry* r = new Registry;  // outlives every pool
+    return *r;
+  }
   std::mutex mu_;
   std::multimap<size_t, Block> free_[2];
   unsigned long long clock_ = 0;
@@ -173,9 +196,9 @@ struct PooledBuf {
       if (pool) p = pool->take(K, bytes, cap);
       if (!p) {
         hipError_t e = allocate(bytes);
-        if (e != hipSuccess && pool) {
+        if (e != hipSuccess) {
           (void)hipGetLastError();
-          pool->trim();
+          BufferPool::trim_all();
           e = allocate(bytes);
         }
         if (e != hipSuccess) p = nullptr;

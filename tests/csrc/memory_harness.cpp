@@ -58,12 +58,72 @@ void staging_growth_fails() {
   }
 }
 
+// Blocks that a context's pool holds go back when an allocation fails for want of them: in a
+// buffer outside any scope (as those of synthesis handles and batched eigensolves are), in
+// another context's scope, and for pinned memory.
+void pool_gives_way() {
+  BippContextImpl *a = context(), *b = context();
+  {
+    PoolScope scope(a->impl->pool);
+    DevBuf d;
+    d.get(40 << 20);
+    PinnedBuf p;
+    p.get(20 << 20);
+  }
+  EXPECT(stub::dev.used == 40 << 20 && stub::pin.used == 20 << 20);  // held, not in use
+  stub::dev.limit = 64 << 20;
+  stub::pin.limit = 32 << 20;
+  {
+    DevBuf d;
+    EXPECT(d.get(50 << 20));
+    EXPECT(stub::dev.used == 50 << 20);
+  }
+  EXPECT(stub::dev.used == 0);
+  {
+    PoolScope scope(a->impl->pool);
+    DevBuf d;
+    d.get(40 << 20);
+    PinnedBuf p;
+    p.get(20 << 20);
+  }
+  {
+    PoolScope scope(b->impl->pool);
+    DevBuf d;
+    EXPECT(d.get(60 << 20));
+    PinnedBuf p;
+    EXPECT(p.get(30 << 20));
+  }
+  // with nothing left to give back the failure is reported, and the next call succeeds
+  DevBuf d;
+  bool threw = false;
+  try {
+    d.get(65 << 20);
+  } catch (const BippException&) {
+    threw = true;
+  }
+  EXPECT(threw && d.p == nullptr && d.cap == 0);
+  EXPECT(d.get(64 << 20));
+  d.drop();
+  // a context that is gone is no longer asked
+  b->release();
+  stub::dev.fail_after = 0;
+  threw = false;
+  try {
+    d.get(1);
+  } catch (const BippException&) {
+    threw = true;
+  }
+  EXPECT(threw);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::string name = argc > 1 ? argv[1] : "";
   if (name == "staging_growth_fails")
     staging_growth_fails();
+  else if (name == "pool_gives_way")
+    pool_gives_way();
   else
     return 2;
   return 0;
