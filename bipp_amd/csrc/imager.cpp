@@ -105,8 +105,19 @@ struct BippImagerImpl {
     if (!count) return;
     const int nS = static_cast<int>(count);
     count = 0;  // a failure below drops the staged samples
-    ContextImpl& c = *ctx->impl;
-    hipStream_t st = c.stream;
+    try {
+      process(nS);
+    } catch (...) {
+      // the staging buffers may still be read by an upload
+      (void)hipStreamSynchronize(ctx->impl->stream);
+      throw;
+    }
+    ctx->impl->sync();  // the staging buffers are refilled by the next add
+  }
+
+  // uploads the staged samples and adds them to the images, on the stream
+  void process(int nS) {
+    hipStream_t st = ctx->impl->stream;
     float* du = d_uvw.as<float>(3 * nn() * nS);
     BIPP_HIP(hipMemcpyAsync(du, h_uvw.p, sizeof(float) * 3 * nn() * nS, hipMemcpyHostToDevice, st));
     void* dv = d_v.get(8 * (size_t)n_ant * n_beam * nS);
@@ -124,7 +135,6 @@ struct BippImagerImpl {
       run<double, double>(nS, du, dv, dd, ds, dw, hwl, n3d);
     else
       run<double, float>(nS, du, dv, dd, ds, dw, hwl, n3f);
-    c.sync();  // the staging buffers are refilled by the next add
   }
 
   // R: virtual-visibility precision; TG: NUFFT grid and image precision

@@ -58,6 +58,18 @@ void staging_growth_fails() {
   }
 }
 
+// A batch that fails after its first upload was enqueued: the stream is waited for before the call
+// returns, since the staging buffers are written or handed on next.
+void failed_flush_waits() {
+  Imager im(context());
+  for (int k = 0; k < 3; ++k) EXPECT(im.add() == BIPP_SUCCESS);
+  float out[Imager::NP];
+  stub::dev.fail_after = 1;
+  const int before = stub::stream_waits;
+  EXPECT(bipp_imager_get(im.h, 0, out) != BIPP_SUCCESS);
+  EXPECT(stub::dev.fail_after == 0 && stub::stream_waits > before);
+}
+
 // Blocks that a context's pool holds go back when an allocation fails for want of them: in a
 // buffer outside any scope (as those of synthesis handles and batched eigensolves are), in
 // another context's scope, and for pinned memory.
@@ -122,6 +134,8 @@ int main(int argc, char** argv) {
   const std::string name = argc > 1 ? argv[1] : "";
   if (name == "staging_growth_fails")
     staging_growth_fails();
+  else if (name == "failed_flush_waits")
+    failed_flush_waits();
   else if (name == "pool_gives_way")
     pool_gives_way();
   else

@@ -32,7 +32,8 @@ def harness(tmp_path_factory):
                         "memory_harness.cpp")
 
 
-@pytest.mark.parametrize("scenario", ["staging_growth_fails", "pool_gives_way"])
+@pytest.mark.parametrize("scenario", ["staging_growth_fails", "pool_gives_way",
+                                      "failed_flush_waits"])
 def test_memory(harness, scenario):
     r = subprocess.run([harness, scenario], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, f"exit {r.returncode}: {r.stderr[-2000:]}"
