@@ -190,32 +190,36 @@ std::vector<double> es_ft_weights(double beta, const std::vector<double>& x,
   for (size_t i = 0; i < x.size(); ++i) ew[i] = w[i] * std::exp(beta * (std::sqrt(1 - x[i] * x[i]) - 1));
   return ew;
 }
-// phi(xi0 + j dxi) for j < n.  The cosines of a node step by a rotation, started afresh from
-// cos and sin every 16 entries (rounding of a few 1e-15): a tolerance's tables took 3 ms with
-// a cosine per node and entry.
+// phi(xi0 + j dxi) for j < n.  An entry's cosines are one rotation away from those of every 32nd
+// entry, cos(a + b) = cos a cos b - sin a sin b, and are summed in eight parts: worst error 3.2e-16
+// of phi(0) over all widths, against 1.3e-15 for a cosine per node and entry added one after another
+// and 1.4e-15 for cosines stepped from entry to entry.  All widths' tables on the CPU: 4.5 ms
+// against 21.7 and 6.7 ms.
 std::vector<double> es_ft_table(double xi0, double dxi, int n, const std::vector<double>& x,
                                 const std::vector<double>& ew) {
+  constexpr int NEAR = 32, PARTS = 8;
   const size_t m = x.size();
-  std::vector<double> out(n), c(m), s(m), cd(m), sd(m);
-  for (size_t i = 0; i < m; ++i) {
-    cd[i] = std::cos(dxi * x[i]);
-    sd[i] = std::sin(dxi * x[i]);
-  }
+  std::vector<double> out(n), c(m), s(m), cn(NEAR * m), sn(NEAR * m);
+  for (int k = 0; k < std::min(n, NEAR); ++k)
+    for (size_t i = 0; i < m; ++i) {
+      cn[k * m + i] = std::cos(k * dxi * x[i]);
+      sn[k * m + i] = std::sin(k * dxi * x[i]);
+    }
   for (int j = 0; j < n; ++j) {
-    if (j % 16 == 0)
+    const int k = j % NEAR;
+    if (k == 0)
       for (size_t i = 0; i < m; ++i) {
         const double a = (xi0 + j * dxi) * x[i];
-        c[i] = std::cos(a);
-        s[i] = std::sin(a);
+        c[i] = ew[i] * std::cos(a);
+        s[i] = ew[i] * std::sin(a);
       }
-    double sum = 0;
-    for (size_t i = 0; i < m; ++i) {
-      sum += ew[i] * c[i];
-      const double t = c[i] * cd[i] - s[i] * sd[i];
-      s[i] = s[i] * cd[i] + c[i] * sd[i];
-      c[i] = t;
-    }
-    out[j] = 2 * sum;
+    const double *ck = &cn[k * m], *sk = &sn[k * m];
+    double p[PARTS] = {};
+    size_t i = 0;
+    for (; i + PARTS <= m; i += PARTS)
+      for (int q = 0; q < PARTS; ++q) p[q] += c[i + q] * ck[i + q] - s[i + q] * sk[i + q];
+    for (; i < m; ++i) p[0] += c[i] * ck[i] - s[i] * sk[i];
+    out[j] = 2 * (((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7])));
   }
   return out;
 }
