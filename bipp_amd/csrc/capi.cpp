@@ -302,7 +302,8 @@ struct BippSynthesisImpl {
   }
 
   // ---- per-timestep chain captured in a HIP graph (steering imager, identity beamforming) ----
-  // flag -> eigensolve (samples in index order) -> level weights and operands -> steering
+  // flag -> eigensolve (samples in index order, in the form of eager collects) -> level weights and
+  // operands -> steering
   // image into a scratch image -> added to the images unless a solve failed.  No host
   // round trip inside the chain, so it is captured once per argument set and replayed.
   struct GraphState {
@@ -315,8 +316,9 @@ struct BippSynthesisImpl {
     long long lds = 0, stride_s = 0;
     const double* xyz = nullptr;
     long long ldxyz = 0, stride_xyz = 0;
-    DevBuf n_red, idx, n_vis, info, counter, d, z, ws_a, ws_l, ws_z, n_eig, n_ant_used, pos,
+    DevBuf n_red, idx, n_vis, info, counter, order, d, z, ws_a, ws_l, ws_z, n_eig, n_ant_used, pos,
         afrag, wts, img_tmp, flag;
+    EigSplit split;
     long long captures = 0, launches = 0;
     void drop() {
       if (exec) (void)hipGraphExecDestroy(exec);
@@ -371,11 +373,21 @@ struct BippSynthesisImpl {
     ep.ldz = nmax;
     ep.ws_ld = nmax;
     ep.ws_stride = nn;
-    ep.ws_a = static_cast<cplx<R>*>(gs.ws_a.p);
-    ep.ws_l = static_cast<cplx<R>*>(gs.ws_l.p);
-    ep.ws_z = static_cast<R*>(gs.ws_z.p);
     ep.info = static_cast<int*>(gs.info.p);
-    launch_eig<R>(ep, n_slots, s_double, st);
+    bool phases = false;
+    if constexpr (sizeof(R) == 8) {
+      phases = nmax > EigSplit::ABOVE;
+      if (phases) {
+        ep.order = static_cast<const int*>(gs.order.p);
+        gs.split.launch(ep, [nmax](int) { return nmax; }, ctx->impl->n_cu, s_double, st);
+      }
+    }
+    if (!phases) {
+      ep.ws_a = static_cast<cplx<R>*>(gs.ws_a.p);
+      ep.ws_l = static_cast<cplx<R>*>(gs.ws_l.p);
+      ep.ws_z = static_cast<R*>(gs.ws_z.p);
+      launch_eig<R>(ep, n_slots, s_double, st);
+    }
     const int mode = steer_mode();
     const int apad = ((n_ant + 15) / 16) * 16;
     const int kchunks = apad / 16;
@@ -471,9 +483,18 @@ struct BippSynthesisImpl {
       gs.counter.as<unsigned>(1);
       gs.d.as<R>((size_t)nS * nmax);
       gs.z.as<cplx<R>>((size_t)nS * nn);
-      gs.ws_a.as<cplx<R>>((size_t)n_slots * nn);
-      gs.ws_l.as<cplx<R>>((size_t)n_slots * nn);
-      gs.ws_z.as<R>((size_t)n_slots * nn);
+      if (sizeof(R) == 8 && nmax > EigSplit::ABOVE) {
+        gs.split.reserve(nS, nmax);
+        std::vector<int> order(nS);
+        std::iota(order.begin(), order.end(), 0);
+        BIPP_HIP(hipMemcpyAsync(gs.order.as<int>(nS), order.data(), sizeof(int) * nS,
+                                hipMemcpyHostToDevice, st));
+        BIPP_HIP(hipStreamSynchronize(st));
+      } else {
+        gs.ws_a.as<cplx<R>>((size_t)n_slots * nn);
+        gs.ws_l.as<cplx<R>>((size_t)n_slots * nn);
+        gs.ws_z.as<R>((size_t)n_slots * nn);
+      }
       gs.n_eig.as<int>(nS);
       gs.n_ant_used.as<int>(nS);
       gs.pos.as<double>((size_t)nS * 3 * apad);

@@ -7,6 +7,47 @@
 
 namespace bippamd {
 
+// Above ABOVE beams a float64 batch is solved phase by phase over all samples (eig_split.hpp), at
+// most JOBS of them at a time (10 MB of scratch per sample at 512 beams, as many as the
+// persistent form's slots).  Milliseconds per batch against the persistent form's, a workgroup per
+// sample, with all beams live: 257 beams 4.5 against 15.9 (1 sample), 6.0 / 18.2 (96), 9.2 / 19.7
+// (256), 18.0 / 39.0 (500); 400 beams 8.1 / 35.2, 14.9 / 41.1, 28.6 / 51.1, 56.5 / 100.7; 512
+// beams 11.5 / 55.1, 27.8 / 68.4, 60.3 / 86.9, 118.5 / 171.6; 40 of 300 beams live 0.5 / 0.9 (1),
+// 1.3 / 2.0 (500).  It is the faster one at every number of samples, so the rule is by size alone.
+struct EigSplit {
+  static constexpr int ABOVE = 256, JOBS = 256;
+  DevBuf a, l, z, c, r, i;
+  int per = 0;  // jobs of a chunk
+  EigSplitBuffers bufs{};
+
+  // every buffer for batches of nS samples of nmax beams
+  void reserve(int nS, int nmax) {
+    per = ceil_div(nS, ceil_div(nS, JOBS));
+    const size_t nn = (size_t)nmax * nmax;
+    a.as<cplx<double>>(per * nn);
+    l.as<cplx<double>>(per * nn);
+    z.as<double>(per * nn);
+    const EigSplitSizes n = eig_split_sizes(per, nmax);
+    bufs = {c.as<cplx<double>>(n.cplx_elems), r.as<double>(n.real_elems), i.as<int>(n.int_elems)};
+  }
+  // n_max(k): largest reduced size, or a bound on it, of the chunk that begins at job k.  Every
+  // chunk's launches are shaped for `per` jobs, so a sample's result does not depend on its place
+  // in the order (a captured batch, in index order, gives the bits of an eager one).
+  template <class F>
+  void launch(EigParams<double> ep, F n_max, int n_cu, bool s_double, hipStream_t st) const {
+    const int nS = ep.n_jobs;
+    const int* order = ep.order;
+    ep.ws_a = static_cast<cplx<double>*>(a.p);
+    ep.ws_l = static_cast<cplx<double>*>(l.p);
+    ep.ws_z = static_cast<double*>(z.p);
+    for (int k = 0; k < nS; k += per) {
+      ep.order = order + k;
+      ep.n_jobs = std::min(per, nS - k);
+      launch_eig_split(ep, bufs, n_max(k), per, n_cu, s_double, st);
+    }
+  }
+};
+
 // ---------------------------------------------------------------------------------------
 // Stage A on a batch: flag -> [Gram/W congruence] -> generalized eigensolve.
 // Results stay on the device: d (R, stride nmax), z (reduced eigenvectors, ld nmax) and,
@@ -16,7 +57,7 @@ template <typename R>
 struct EigRunner {
   DevBuf n_red, idx, n_vis, info, counter, order, d, z, ws_a, ws_l, ws_z, prof_buf;
   DevBuf sig, w_i, tmp, g, v_full;
-  DevBuf split_c, split_r, split_i;
+  EigSplit split;
   int n_samples = 0, n_ant = 0, nmax = 0;
   bool general_w = false;
   std::vector<int> h_info;
@@ -156,7 +197,7 @@ struct EigRunner {
     ep.ws_stride = nn;
     ep.info = info.as<int>(nS);
     if constexpr (sizeof(R) == 8) {
-      if (nmax > SPLIT_ABOVE && !standard) {
+      if (nmax > EigSplit::ABOVE && !standard) {
         run_split(ctx, ep, h_nred, h_order, s_double);
         unbeam_general(nS, nAnt, st);
         return;
@@ -241,31 +282,11 @@ struct EigRunner {
     launch_gemm_batch<R>(g3, nAnt, nmax, st);
   }
 
-  // Above this many beams the batch is solved phase by phase over all samples, at most
-  // SPLIT_JOBS of them at a time (10 MB of scratch per sample at 512 beams, as many as the
-  // persistent form's slots): a sample's single-CU time there is 55 ms (400..512 beams), a
-  // phase-split batch of 12 takes 15.7 ms, one of 96 30.9 ms (64 before).  Up to 256 beams the persistent form keeps one workgroup
-  // per sample.
-  static constexpr int SPLIT_ABOVE = 256;
-  static constexpr int SPLIT_JOBS = 256;
-
-  void run_split(ContextImpl& ctx, EigParams<double> ep, const std::vector<int>& h_nred,
+  void run_split(ContextImpl& ctx, const EigParams<double>& ep, const std::vector<int>& h_nred,
                  const std::vector<int>& h_order, bool s_double) {
-    const int nS = ep.n_jobs, n_chunks = ceil_div(nS, SPLIT_JOBS), per = ceil_div(nS, n_chunks);
-    const size_t nn = (size_t)ep.ws_stride;
-    ep.ws_a = ws_a.as<cplx<double>>(per * nn);
-    ep.ws_l = ws_l.as<cplx<double>>(per * nn);
-    ep.ws_z = ws_z.as<double>(per * nn);
-    const EigSplitSizes z = eig_split_sizes(per, ep.nmax);
-    const EigSplitBuffers b{split_c.as<cplx<double>>(z.cplx_elems), split_r.as<double>(z.real_elems),
-                            split_i.as<int>(z.int_elems)};
-    const int* order0 = ep.order;
-    for (int k = 0; k < nS; k += per) {
-      ep.order = order0 + k;
-      ep.n_jobs = std::min(per, nS - k);
-      // largest first: the chunk's first sample has its largest reduced size
-      launch_eig_split(ep, b, h_nred[h_order[k]], ctx.n_cu, s_double, ctx.stream);
-    }
+    split.reserve(ep.n_jobs, ep.nmax);
+    // largest first: the chunk's first sample has its largest reduced size
+    split.launch(ep, [&](int k) { return h_nred[h_order[k]]; }, ctx.n_cu, s_double, ctx.stream);
   }
 
   // Throws EigensolverError if any solve failed (LAPACK info != 0 analogue).

@@ -1522,10 +1522,10 @@ EigSplitSizes eig_split_sizes(int n_jobs, int nmax) {
   return z;
 }
 
-void launch_eig_split(const EigParams<double>& p, const EigSplitBuffers& b, int n_max, int n_cu,
-                      bool in_double, hipStream_t stream) {
+void launch_eig_split(const EigParams<double>& p, const EigSplitBuffers& b, int n_max, int n_shape,
+                      int n_cu, bool in_double, hipStream_t stream) {
   if (p.n_jobs <= 0) return;
-  if (eig_nmax_bucket<double>(p.nmax) != 512 || p.n_jobs > 65535 || n_max > p.nmax || !p.order ||
+  if (eig_nmax_bucket<double>(p.nmax) != 512 || p.n_jobs > 65535 || n_max > p.nmax || n_shape < 1 || !p.order ||
       p.standard || p.ldz != p.ws_ld || p.stride_z != p.ws_stride)
     fail(BIPP_INTERNAL_ERROR, "phase-split eigensolve arguments");
   const int jobs = p.n_jobs;
@@ -1559,8 +1559,8 @@ void launch_eig_split(const EigParams<double>& p, const EigSplitBuffers& b, int 
   // vectors per sample), else two 256-thread ones per CU, whose prologues and passes overlap.
   // Whole batch of 400..512 beams: 12 samples 15.7 ms (17.0 with 256 threads), 32 samples 20.0
   // (20.8), 96 samples 32.5 against 30.9 with 256 threads.
-  const bool wide = n_cu / jobs >= 4;
-  const int G = std::max(1, std::min(TRI_GMAX, (wide ? n_cu : 2 * n_cu) / jobs));
+  const bool wide = n_cu / n_shape >= 4;
+  const int G = std::max(1, std::min(TRI_GMAX, (wide ? n_cu : 2 * n_cu) / n_shape));
   auto column = [&](auto pending, int c) {
     constexpr int P = decltype(pending)::value;
     if (wide)

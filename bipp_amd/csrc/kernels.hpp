@@ -75,8 +75,9 @@ void launch_flag(const FlagParams& p, int n_samples, bool in_double, hipStream_t
 template <typename R>
 void launch_eig(const EigParams<R>& p, int n_slots, bool in_double, hipStream_t stream);
 // Phase-split float64 form (eig_split.hpp): p.ws_a, p.ws_l and p.ws_z hold one matrix per job
-// (p.order is required, ldz == ws_ld, stride_z == ws_stride, p.counter unused); n_max: the
-// largest reduced size of the jobs.
+// (p.order is required, ldz == ws_ld, stride_z == ws_stride, p.counter unused); n_max: at least the
+// largest reduced size of the jobs (no result depends on it); n_shape: the number of jobs that the
+// column launches are shaped for, on which the order of their sums depends.
 struct EigSplitSizes {
   size_t cplx_elems, real_elems, int_elems;
 };
@@ -86,8 +87,8 @@ struct EigSplitBuffers {
   int* int_buf;
 };
 EigSplitSizes eig_split_sizes(int n_jobs, int nmax);
-void launch_eig_split(const EigParams<double>& p, const EigSplitBuffers& b, int n_max, int n_cu,
-                      bool in_double, hipStream_t stream);
+void launch_eig_split(const EigParams<double>& p, const EigSplitBuffers& b, int n_max, int n_shape,
+                      int n_cu, bool in_double, hipStream_t stream);
 template <typename R>
 void launch_unbeam_identity(const UnbeamParams<R>& p, int n_samples, int n_beam, bool out_double,
                             hipStream_t stream);
