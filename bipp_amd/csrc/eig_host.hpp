@@ -20,9 +20,13 @@ struct EigSplit {
   int per = 0;  // jobs of a chunk
   EigSplitBuffers bufs{};
 
-  // every buffer for batches of nS samples of nmax beams
+  // every buffer for batches of nS samples of nmax beams; BIPP_EIG_MAX_SLOTS caps the jobs of a
+  // chunk, as it caps the persistent form's slots
   void reserve(int nS, int nmax) {
-    per = ceil_div(nS, ceil_div(nS, JOBS));
+    int most = JOBS;
+    if (const char* e = std::getenv("BIPP_EIG_MAX_SLOTS"))
+      if (std::atoi(e) > 0) most = std::min(most, std::atoi(e));
+    per = ceil_div(nS, ceil_div(nS, most));
     const size_t nn = (size_t)nmax * nmax;
     a.as<cplx<double>>(per * nn);
     l.as<cplx<double>>(per * nn);
@@ -34,7 +38,8 @@ struct EigSplit {
   // chunk's launches are shaped for `per` jobs, so a sample's result does not depend on its place
   // in the order (a captured batch, in index order, gives the bits of an eager one).
   template <class F>
-  void launch(EigParams<double> ep, F n_max, int n_cu, bool s_double, hipStream_t st) const {
+  void launch(EigParams<double> ep, F n_max, int n_cu, bool s_double, hipStream_t st,
+              EigSplitMarks* marks = nullptr) const {
     const int nS = ep.n_jobs;
     const int* order = ep.order;
     ep.ws_a = static_cast<cplx<double>*>(a.p);
@@ -43,9 +48,41 @@ struct EigSplit {
     for (int k = 0; k < nS; k += per) {
       ep.order = order + k;
       ep.n_jobs = std::min(per, nS - k);
-      launch_eig_split(ep, bufs, n_max(k), per, n_cu, s_double, st);
+      launch_eig_split(ep, bufs, n_max(k), per, n_cu, s_double, st, marks);
     }
   }
+};
+
+// Time of each phase of a phase-split batch, from events between its launches.
+struct EigSplitProfile final : EigSplitMarks {
+  EigSplitProfile() = default;
+  EigSplitProfile(const EigSplitProfile&) = delete;
+  ~EigSplitProfile() {
+    for (auto& m : marks) (void)hipEventDestroy(m.second);
+  }
+  void mark(const char* phase, hipStream_t st) override {
+    hipEvent_t e = nullptr;
+    BIPP_HIP(hipEventCreate(&e));
+    marks.emplace_back(phase, e);
+    BIPP_HIP(hipEventRecord(e, st));
+  }
+  // after the stream has been waited for; chunks of the same phase are added up
+  void report(int n_samples, int per) const {
+    std::vector<std::pair<std::string, double>> sum;
+    for (size_t k = 1; k < marks.size(); ++k) {
+      float t = 0;
+      BIPP_HIP(hipEventElapsedTime(&t, marks[k - 1].second, marks[k].second));
+      auto it = std::find_if(sum.begin(), sum.end(), [&](auto& s) { return s.first == marks[k].first; });
+      if (it == sum.end()) it = sum.insert(sum.end(), {marks[k].first, 0.0});
+      it->second += t;
+    }
+    std::fprintf(stderr, "[bipp eig profile] %d samples phase by phase, %d at a time, ms/batch:", n_samples, per);
+    for (const auto& s : sum) std::fprintf(stderr, " %s %.3f", s.first.c_str(), s.second);
+    std::fprintf(stderr, "\n");
+  }
+
+ private:
+  std::vector<std::pair<const char*, hipEvent_t>> marks;
 };
 
 // ---------------------------------------------------------------------------------------
@@ -285,8 +322,18 @@ struct EigRunner {
   void run_split(ContextImpl& ctx, const EigParams<double>& ep, const std::vector<int>& h_nred,
                  const std::vector<int>& h_order, bool s_double) {
     split.reserve(ep.n_jobs, ep.nmax);
+    // BIPP_EIG_PROFILE=1: per-phase times of this batch on stderr
+    std::unique_ptr<EigSplitProfile> prof;
+    if (std::getenv("BIPP_EIG_PROFILE")) {
+      prof = std::make_unique<EigSplitProfile>();
+      prof->mark("", ctx.stream);
+    }
     // largest first: the chunk's first sample has its largest reduced size
-    split.launch(ep, [&](int k) { return h_nred[h_order[k]]; }, ctx.n_cu, s_double, ctx.stream);
+    split.launch(ep, [&](int k) { return h_nred[h_order[k]]; }, ctx.n_cu, s_double, ctx.stream, prof.get());
+    if (prof) {
+      BIPP_HIP(hipStreamSynchronize(ctx.stream));
+      prof->report(ep.n_jobs, split.per);
+    }
   }
 
   // Throws EigensolverError if any solve failed (LAPACK info != 0 analogue).

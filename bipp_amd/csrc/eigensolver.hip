@@ -1523,8 +1523,11 @@ EigSplitSizes eig_split_sizes(int n_jobs, int nmax) {
 }
 
 void launch_eig_split(const EigParams<double>& p, const EigSplitBuffers& b, int n_max, int n_shape,
-                      int n_cu, bool in_double, hipStream_t stream) {
+                      int n_cu, bool in_double, hipStream_t stream, EigSplitMarks* marks) {
   if (p.n_jobs <= 0) return;
+  auto mark = [&](const char* phase) {
+    if (marks) marks->mark(phase, stream);
+  };
   if (eig_nmax_bucket<double>(p.nmax) != 512 || p.n_jobs > 65535 || n_max > p.nmax || n_shape < 1 || !p.order ||
       p.standard || p.ldz != p.ws_ld || p.stride_z != p.ws_stride)
     fail(BIPP_INTERNAL_ERROR, "phase-split eigensolve arguments");
@@ -1547,13 +1550,16 @@ void launch_eig_split(const EigParams<double>& p, const EigSplitBuffers& b, int 
       split_load_kernel<float><<<lg, 256, 0, stream>>>(p);
     check_launch("split_load_kernel");
   }
+  mark("load");
   launch_split_chol(p, n_max, stream);
+  mark("cholesky");
   if (n_max <= 0) return;
   const int side = ceil_div(n_max, 64);
   split_gemm_kernel<0><<<split_grid(side * side, jobs), 256, 0, stream>>>(p, side);
   check_launch("split_gemm_kernel");
   split_gemm_kernel<1><<<split_grid(side * (side + 1) / 2, jobs), 256, 0, stream>>>(p, side);
   check_launch("split_gemm_kernel");
+  mark("whiten");
   // Column launches: one 512-thread workgroup per CU over all samples while that gives a sample
   // at least four (at most eight: every workgroup reads the row sums of all of them, G^2
   // vectors per sample), else two 256-thread ones per CU, whose prologues and passes overlap.
@@ -1578,10 +1584,13 @@ void launch_eig_split(const EigParams<double>& p, const EigSplitBuffers& b, int 
   }
   static_assert(TRI_LAG == 2, "one launch for each count of pending updates");
   check_launch("tri_column_kernel");
+  mark("tridiag columns");
   split_tail_kernel<<<jobs, EigCfg<TRI_TAIL>::NT, 0, stream>>>(p, tw);
   check_launch("split_tail_kernel");
+  mark("tridiag tail");
   split_dc_kernel<NM><<<jobs, EigCfg<NM>::NT, 0, stream>>>(p, tw);
   check_launch("split_dc_kernel");
+  mark("tridiag_eig");
   if (n_max > 1) {
     split_tfac_kernel<<<dim3((n_max + 14) / 16, jobs), 256, 0, stream>>>(p);
     check_launch("split_tfac_kernel");
@@ -1589,8 +1598,10 @@ void launch_eig_split(const EigParams<double>& p, const EigSplitBuffers& b, int 
   const int groups = ceil_div(n_max, 16);
   split_bt_kernel<NM><<<split_grid(groups, jobs), 256, 0, stream>>>(p, tw, groups);
   check_launch("split_bt_kernel");
+  mark("backtransform");
   split_gemm_kernel<2><<<split_grid(side * side, jobs), 256, 0, stream>>>(p, side);
   check_launch("split_gemm_kernel");
+  mark("unwhiten");
 }
 
 template <typename R>

@@ -86,9 +86,16 @@ struct EigSplitBuffers {
   double* real_buf;
   int* int_buf;
 };
+// marks the end of a phase of launch_eig_split (for a profile), on its stream
+struct EigSplitMarks {
+  virtual void mark(const char* phase, hipStream_t stream) = 0;
+
+ protected:
+  ~EigSplitMarks() = default;
+};
 EigSplitSizes eig_split_sizes(int n_jobs, int nmax);
 void launch_eig_split(const EigParams<double>& p, const EigSplitBuffers& b, int n_max, int n_shape,
-                      int n_cu, bool in_double, hipStream_t stream);
+                      int n_cu, bool in_double, hipStream_t stream, EigSplitMarks* marks = nullptr);
 template <typename R>
 void launch_unbeam_identity(const UnbeamParams<R>& p, int n_samples, int n_beam, bool out_double,
                             hipStream_t stream);
