@@ -455,7 +455,7 @@ def main() -> None:
         "plain_fp32": plain,
         "speedup_vs_plain": (value / plain["samples_per_s"]) if (plain and value) else None,
         "stages_ms_per_step": stages,
-        "nufft_tuning": ({"shape": tuning[0], "candidates_timed": len(tuning[1]),
+        "nufft_tuning": ({"shape": tuning[0], "candidates_timed": len({r[1] for r in tuning[1]}),
                           "fastest_ms": min((r[1] for r in tuning[1]), default=None),
                           "slowest_ms": max((r[1] for r in tuning[1]), default=None)}
                          if tuning else None),

@@ -2195,13 +2195,19 @@ bool go_fft_axis(N3AxisParams<R> p, const int (&f)[4], hipStream_t st) {
   return true;
 }
 
+bool fft_axis_radices(int n, int n1, int n2, int (&f)[4]) {
+  return n2 >= 2 && (long long)n1 * n2 == n && fft_rr_factors(n1, f[0], f[1]) && fft_rr_factors(n2, f[2], f[3]);
+}
+bool fft_axis_form(int n, int n1, int n2, size_t elem) {
+  int f[4];
+  return fft_axis_radices(n, n1, n2, f) && fft_axis_shift(n, elem) >= 0;
+}
+
 template <typename R>
 bool launch_fft_axis(const N3AxisParams<R>& p_in, hipStream_t st) {
   N3AxisParams<R> p = p_in;
   int f[4];
-  if (p.n2 < 2 || (long long)p.n1 * p.n2 != p.n || !fft_rr_factors(p.n1, f[0], f[1]) ||
-      !fft_rr_factors(p.n2, f[2], f[3]))
-    return false;
+  if (!fft_axis_radices(p.n, p.n1, p.n2, f)) return false;
   p.tw_shift = fft_axis_shift(p.n, sizeof(cplx<R>));
   return p.tw_shift >= 0 && go_fft_axis<R, false>(p, f, st);
 }
@@ -2211,11 +2217,17 @@ bool launch_fft_axis(const N3AxisParams<R>& p_in, hipStream_t st) {
 // (FFT of 64-antenna samples, x and y of 1800 points: 13.7 to 10.6 ms with this form, 768 points
 // 3.1 to 2.1, 240 points 0.49 to 0.39; 2160 points 18.9 and 18.5 in float, 51.9 and 53.4 in
 // double; 3240 points 3.27 against 3.80 for the lines alone, 6000 5.98 against 7.42).
+constexpr int FFT_XLINES_MAX = 2048;
+bool fft_xlines_form(int n) {
+  int f[4];
+  return n <= FFT_XLINES_MAX && fft_line_radices(n, f);
+}
+
 template <typename R>
 bool launch_fft_xlines(const N3LineParams<R>& q, hipStream_t st) {
   N3AxisParams<R> p{};
   int f[4];
-  if (q.n > 2048 || !fft_line_radices(q.n, f)) return false;
+  if (q.n > FFT_XLINES_MAX || !fft_line_radices(q.n, f)) return false;
   p.grid = q.grid;
   p.grid_stride = q.grid_stride;
   p.n_levels = q.n_levels;

@@ -289,6 +289,10 @@ template <typename R>
 void launch_fft_lines(const N3LineParams<R>& p, hipStream_t st);
 template <typename R>
 void launch_fft_pass(const N3PassParams<R>& p, hipStream_t st);
+// whether an axis of n = n1 n2 points (elements of `elem` bytes) has the one-pass form, and
+// whether x lines of n points run in the same kernel
+bool fft_axis_form(int n, int n1, int n2, size_t elem);
+bool fft_xlines_form(int n);
 // false: no form of this length, nothing launched
 template <typename R>
 bool launch_fft_axis(const N3AxisParams<R>& p, hipStream_t st);
