@@ -167,7 +167,6 @@ struct BippSynthesisImpl {
       sp.w_stride = pp.w_stride;
       sp.epad = epad;
       sp.lmn = static_cast<const double*>(lmn64.p);
-      sp.phase_fp32 = compute == BIPP_COMPUTE_FP32 ? 1 : 0;
       sp.img = img.p;
       sp.img_ld = n_pix;
       launch_steer(sp, mode, st);
@@ -447,7 +446,6 @@ struct BippSynthesisImpl {
     sp.w_stride = pp.w_stride;
     sp.epad = epad;
     sp.lmn = static_cast<const double*>(lmn64.p);
-    sp.phase_fp32 = compute == BIPP_COMPUTE_FP32 ? 1 : 0;
     sp.img = gs.img_tmp.p;
     sp.img_ld = n_pix;
     launch_steer(sp, mode, st);

@@ -199,7 +199,6 @@ struct SteerParams {
   long long w_stride;
   int epad;
   const double* lmn;  // [3][n_pix]
-  int phase_fp32;     // plain form: phases formed in float32
   void* img;          // [n_levels][img_ld] float (double for FP64 mode), accumulated
   long long img_ld;
 };
