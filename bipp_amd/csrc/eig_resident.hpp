@@ -155,7 +155,7 @@ __device__ __forceinline__ void tri_sweep(int g0, int off, const BufMat<double>&
 // d and e into sh.de, the reflectors below the subdiagonal of A with tau in the diagonal slots
 // (0 for the last column), as tridiag_phase leaves them; n >= 2.  Out of line: its registers
 // are allocated apart from the other phases.
-template <int NMAX>
+template <int NMAX, int USE = 0>
 __device__ __noinline__ void tridiag_resident(int n, cplx<double>* __restrict__ A, int ld,
                                               unsigned long long* prof) {
   using T = TriRes<NMAX>;
@@ -163,7 +163,7 @@ __device__ __noinline__ void tridiag_resident(int n, cplx<double>* __restrict__ 
   ld = uniform(ld);
   A = uniform(A);
   prof = uniform(prof);
-  EigShared<double, NMAX>& sh = eig_sh<double, NMAX>;
+  EigShared<double, NMAX>& sh = eig_sh<double, NMAX, USE>;
   static_assert(EigCfg<NMAX>::NT >= NMAX, "one row per thread");
   const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lc = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);

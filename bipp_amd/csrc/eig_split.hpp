@@ -571,13 +571,13 @@ __global__ __launch_bounds__(NT) void tri_column_kernel(EigParams<double> p, Tri
 
 // The trailing matrix from column n - TRI_TAIL on (all of a smaller one).  Workgroup per job.
 __global__ __launch_bounds__(EigCfg<TRI_TAIL>::NT) void split_tail_kernel(EigParams<double> p, TriWork tw) {
-  EigShared<double, TRI_TAIL>& sh = eig_sh<double, TRI_TAIL>;
+  EigShared<double, TRI_TAIL>& sh = eig_sh<double, TRI_TAIL, 1>;
   const int job = blockIdx.x, sid = p.order[job], n = p.n_red[sid], ld = p.ldz;
   if (n <= 0 || p.info[sid] != 0) return;
   const int c0 = max(0, n - TRI_TAIL), m = n - c0;
   cplx<double>* A = p.z_out + (size_t)sid * p.stride_z + c0 + (size_t)c0 * ld;
   if (m > 1) {
-    tridiag_resident<TRI_TAIL>(m, A, ld, nullptr);
+    tridiag_resident<TRI_TAIL, 1>(m, A, ld, nullptr);
   } else {
     if (threadIdx.x == 0) {
       sh.de[0].x = A[0].re;
@@ -596,7 +596,7 @@ __global__ __launch_bounds__(EigCfg<TRI_TAIL>::NT) void split_tail_kernel(EigPar
 // d_out, the column order to perm.  Workgroup per job.
 template <int NMAX>
 __global__ __launch_bounds__(EigCfg<NMAX>::NT) void split_dc_kernel(EigParams<double> p, TriWork tw) {
-  EigShared<double, NMAX>& sh = eig_sh<double, NMAX>;
+  EigShared<double, NMAX>& sh = eig_sh<double, NMAX, 1>;
   constexpr int NT_ = EigCfg<NMAX>::NT;
   const int job = blockIdx.x, sid = p.order[job], n = p.n_red[sid], tid = threadIdx.x;
   if (n <= 0 || p.info[sid] != 0) return;
@@ -605,7 +605,7 @@ __global__ __launch_bounds__(EigCfg<NMAX>::NT) void split_dc_kernel(EigParams<do
     sh.de[i].y = tw.de[((size_t)job * p.nmax + i) * 2 + 1];
   }
   __syncthreads();
-  dc_phase<double, NMAX>(n, p.ws_z + (size_t)job * p.ws_stride, p.ws_ld,
+  dc_phase<double, NMAX, 1>(n, p.ws_z + (size_t)job * p.ws_stride, p.ws_ld,
                          reinterpret_cast<double*>(p.ws_a + (size_t)job * p.ws_stride), nullptr);
   rank_order<double, NMAX>(n, sh);
   for (int j = tid; j < p.nmax; j += NT_) {

@@ -168,8 +168,12 @@ static_assert(DcCfg<256>::TILE_ELEMS <= 8 * 256 && DcCfg<64>::TILE_ELEMS <= 8 * 
 
 // The eigensolver's LDS, at namespace scope: the phases kept out of line (own register
 // allocation) name it directly, so that their accesses compile to LDS instructions rather
-// than generic (flat) ones through a reference parameter.
-template <typename R, int NMAX>
+// than generic (flat) ones through a reference parameter.  USE: 0 in eig_kernel, 1 in the
+// phase-split kernels.  The compiler gives out-of-line functions a block's address directly where one
+// kernel reaches it, and for the one block that most kernels reach; the others are looked up in
+// a table.  With the phase-split kernels on eig_kernel's blocks the 512-beam one took that
+// place from the float32 64-beam one (one sample of 24 beams 228 to 244 us, 64 beams 720 to 769).
+template <typename R, int NMAX, int USE = 0>
 __shared__ EigShared<R, NMAX> eig_sh;
 
 // --------------------------------------------------------------------------------------
@@ -804,9 +808,9 @@ __device__ __noinline__ int chol_phase(int n, cplx<R>* L, int ld, cplx<R>* T, in
 
 // eigenpairs of the tridiagonal in sh.de by divide and conquer (tridiag_dc.hpp), eigenvectors
 // into Z; work: 2 n^2 reals of scratch; out of line
-template <typename R, int NMAX>
+template <typename R, int NMAX, int USE = 0>
 __device__ __noinline__ void dc_phase(int n, R* Z, int ld, R* work, unsigned long long* prof) {
-  EigShared<R, NMAX>& sh = eig_sh<R, NMAX>;
+  EigShared<R, NMAX>& sh = eig_sh<R, NMAX, USE>;
   n = uniform(n);
   WgTeam tm{static_cast<int>(threadIdx.x), uniform(prof)};
   BIPP_GLOBAL R* w = global_ptr(work);
