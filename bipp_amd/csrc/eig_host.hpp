@@ -1,4 +1,5 @@
-// Host side of the batched generalized eigensolve (flag -> Gram -> eig_kernel -> un-beam)
+// Host side of the batched generalized eigensolve (flag -> Gram -> eig_kernel, or the phases of
+// eig_split.hpp -> un-beam)
 // and the library context object that owns its workspaces.
 #pragma once
 

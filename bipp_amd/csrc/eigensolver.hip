@@ -1567,8 +1567,8 @@ void launch_eig_split(const EigParams<double>& p, const EigSplitBuffers& b, int 
   // Column launches: one 512-thread workgroup per CU over all samples while that gives a sample
   // at least four (at most eight: every workgroup reads the row sums of all of them, G^2
   // vectors per sample), else two 256-thread ones per CU, whose prologues and passes overlap.
-  // Whole batch of 400..512 beams: 12 samples 15.7 ms (17.0 with 256 threads), 32 samples 20.0
-  // (20.8), 96 samples 32.5 against 30.9 with 256 threads.
+  // Whole batch of 400..512 beams, 512 and 256 threads: 12 samples 12.0 and 13.1 ms, 32 samples
+  // 14.6 and 15.4, 64 samples 18.3 and 18.8, 96 samples 23.7 and 23.1, 160 samples 36.4 and 32.6.
   const bool wide = n_cu / n_shape >= 4;
   const int G = std::max(1, std::min(TRI_GMAX, (wide ? n_cu : 2 * n_cu) / n_shape));
   auto column = [&](auto pending, int c) {

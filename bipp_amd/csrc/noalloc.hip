@@ -1,6 +1,8 @@
 // Batched generalized eigensolve without device allocation.
 //
-// The same kernels as bipp_eigh_gram_batched (flag, eig_kernel, export), with every scratch
+// The persistent form of bipp_eigh_gram_batched (flag, eig_kernel, export; that entry solves
+// float64 batches above 256 beams phase by phase instead, so results agree to rounding there,
+// not bit for bit), with every scratch
 // buffer -- per-sample kept-beam lists, counts, eigenvalues and reduced eigenvectors, the
 // per-workgroup matrix slots of the persistent eigensolver and its job counter -- carved from
 // one file-scope device array of a fixed size instead of hipMalloc'd workspaces.  The

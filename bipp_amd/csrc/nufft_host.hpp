@@ -40,9 +40,9 @@ int radix_cap(const char* name, int dflt) {
   return x >= 16 ? 16 : (x >= 9 ? 9 : (x >= 8 ? 8 : (x >= 6 ? 6 : 4)));
 }
 // contiguous-axis lines (BIPP_FFT_RADIX_MAX, default 9) and strided passes
-// (BIPP_FFT_PASS_RADIX_MAX, default 4); the defaults were the fastest at configuration 4
-// (x lines of 3456 as radices 6, 8, 8, 9: 20.9 ms for the FFT against 22.4 ms with radices
-// up to 4; composite radices in the strided passes cost occupancy and were slower)
+// (BIPP_FFT_PASS_RADIX_MAX, default 4), where a length is transformed by Stockham stages at
+// all: x lines above 2048 points, strided passes of a length with a factor of 125 (figures
+// at N3Tuning)
 int fft_radix_max() {
   static const int v = radix_cap("BIPP_FFT_RADIX_MAX", 9);
   return v;
