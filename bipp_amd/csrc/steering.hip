@@ -475,7 +475,7 @@ __device__ __forceinline__ float sum_columns(const float* v) {
 // (RTW <= 2) two workgroups fit a CU.  The fragments of a step are loaded one step ahead.  Every
 // wavefront adds its sums into an image of its own in LDS: LDS float atomics took 2.4 cycles
 // per lane (2.5 ms of 31 ms at 96 samples, 512^2 pixels).
-// Measured, 512^2 pixels, 4 levels: 96 samples of 180..256 antennas 41.4 to 28.2 ms (a
+// Measured, 512^2 pixels, 4 levels: 96 samples of 180..256 antennas 41.4 to 28.7 ms (a
 // full-rate loop of these MFMAs alone runs at 1.5 PFLOP/s here, about 19 ms); 256^2 pixels,
 // 32 samples of 96 antennas 1.47 to 0.56 ms.
 // (the accumulators live in registers only if every lambda is inlined)
